@@ -237,10 +237,10 @@ __device__ __forceinline__ void reconstruct(const StageParams &p, int phim, int6
     } else {
         // eight correctly rounded quotients over one shared reciprocal of det
         const Recip<FT> rd = recip(det);
-        gx.d = rdiv(Dx.d * DyDy - Dy.d * DxDy, rd); gx.vx = rdiv(Dx.vx * DyDy - Dy.vx * DxDy, rd);
-        gx.vy = rdiv(Dx.vy * DyDy - Dy.vy * DxDy, rd); gx.p = rdiv(Dx.p * DyDy - Dy.p * DxDy, rd);
-        gy.d = rdiv(Dy.d * DxDx - Dx.d * DxDy, rd); gy.vx = rdiv(Dy.vx * DxDx - Dx.vx * DxDy, rd);
-        gy.vy = rdiv(Dy.vy * DxDx - Dx.vy * DxDy, rd); gy.p = rdiv(Dy.p * DxDx - Dx.p * DxDy, rd);
+        gx.d = rdivf(Dx.d * DyDy - Dy.d * DxDy, rd); gx.vx = rdivf(Dx.vx * DyDy - Dy.vx * DxDy, rd);
+        gx.vy = rdivf(Dx.vy * DyDy - Dy.vy * DxDy, rd); gx.p = rdivf(Dx.p * DyDy - Dy.p * DxDy, rd);
+        gy.d = rdivf(Dy.d * DxDx - Dx.d * DxDy, rd); gy.vx = rdivf(Dy.vx * DxDx - Dx.vx * DxDy, rd);
+        gy.vy = rdivf(Dy.vy * DxDx - Dx.vy * DxDy, rd); gy.p = rdivf(Dy.p * DxDx - Dx.p * DxDy, rd);
     }
     if (phim == PHI_LOAD) {
         ph.d = (FT)p.phi[c]; ph.vx = (FT)p.phi[ncp + c]; ph.vy = (FT)p.phi[2 * ncp + c]; ph.p = (FT)p.phi[3 * ncp + c];
@@ -872,17 +872,17 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
                 double d = dU[v];
                 if (res) {
                     // (Flux*l)/A of dUdt_Residual_Evaluation, Euler2DQuad.cc:1001-1006
-                    d += rdiv(FW * lW, rA);
-                    d -= rdiv(FE * lE, rA);
+                    d += rdivf(FW * lW, rA);
+                    d -= rdivf(FE * lE, rA);
                     if (axi) d += Sx[v];
-                    d += rdiv(FS * lS, rA);
-                    d -= rdiv(FN * lN, rA);
+                    d += rdivf(FS * lS, rA);
+                    d -= rdivf(FN * lN, rA);
                 } else {
-                    d += rdiv(cdt * FW * lW, rA);
-                    d -= rdiv(cdt * FE * lE, rA);
+                    d += rdivf(cdt * FW * lW, rA);
+                    d -= rdivf(cdt * FE * lE, rA);
                     if (axi) d += cdt * Sx[v];
-                    d += rdiv(cdt * FS * lS, rA);
-                    d -= rdiv(cdt * FN * lN, rA);
+                    d += rdivf(cdt * FS * lS, rA);
+                    d -= rdivf(cdt * FN * lN, rA);
                 }
                 dU[v] = d;
             }

@@ -80,45 +80,72 @@ template <typename T> struct Fast { static constexpr bool on = false; };
 template <> struct Fast<float> { static constexpr bool on = true; };
 
 // Correctly rounded FP64 division with the divisor's reciprocal shared by
-// every quotient over the same divisor.  The device steps are gfx950's own
-// IEEE a / b: r = v_rcp_f64(b) refined by two Newton steps
-// r += r(1 - b r), then q = a r, the exact FMA remainder a - b q, the
-// corrected quotient q + (a - b q) r and v_div_fixup_f64, which gives zeros,
-// infinities and NaNs their IEEE results.  Only the operand scaling
-// (v_div_scale_f64 and the scale applied by v_div_fmas_f64) is left out: it
-// acts when a/b or 1/b would be subnormal, |a/b| >= 2^767 or a nonzero
-// |a| < 2^-969, so for every other operand pair the result is a / b bit for
-// bit.  The Newton steps depend on b alone, which is what makes the
-// reciprocal shareable.  float: plain division (callers choose their own
-// approximations on the mixed path).
+// every quotient over the same divisor.  r = v_rcp_f64(b) (about 23 good
+// bits) refined by one cubic step, r += r(e + e^2) with e = 1 - b r, which
+// leaves about 2^-69 before its rounding; then q = a r, the FMA remainder
+// a - b q and the corrected quotient q + (a - b q) r.  The remainder is below
+// two units of q's last place, so r's own last-place error enters at 2^-104 of
+// q: the result is a / b correctly rounded, as the compiler's sequence (two
+// Newton steps, one instruction more) gives it.  v_div_fixup_f64 gives zeros,
+// infinities and NaNs their IEEE results (rdiv); rdivf leaves it out, for
+// finite operands and a nonzero finite divisor, where it only restores the sign
+// of a -0 dividend's quotient.  The operand scaling of the compiler's
+// division (v_div_scale_f64 and the scale applied by v_div_fmas_f64) is left
+// out of both: it acts when a/b or 1/b would be subnormal, |a/b| >= 2^767 or a
+// nonzero |a| < 2^-969, so for every other operand pair the result is a / b bit
+// for bit.  The refinement depends on b alone, which is what makes the
+// reciprocal shareable; recip_near starts it from a value already close to
+// 1/b (a reciprocal of a related divisor), without the quarter-rate v_rcp_f64.
+// float: plain division (callers choose their own approximations on the mixed
+// path).
 template <typename T> struct Recip { T b, r; };
 template <typename T> CFFC_HD Recip<T> recip(T b) {
 #if defined(__HIP_DEVICE_COMPILE__)
     if constexpr (!Fast<T>::on) {
-        double r = __builtin_amdgcn_rcp(b);
-        double e = fma(-b, r, 1.0);
-        r = fma(r, e, r);
-        e = fma(-b, r, 1.0);
-        r = fma(r, e, r);
-        return {b, r};
+        const double r = __builtin_amdgcn_rcp(b);
+        const double e = fma(-b, r, 1.0);
+        return {b, fma(r, fma(e, e, e), r)};
     }
 #endif
     return {b, T(0)};
 }
-template <typename T> CFFC_HD T rdiv(T a, const Recip<T> &d) {
+// 1/b from r0 = 1/b (1 + d), |d| < 2^-40 or so: one Newton step leaves d^2,
+// below the step's own rounding
+template <typename T> CFFC_HD Recip<T> recip_near(T b, T r0) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (!Fast<T>::on) return {b, fma(r0, fma(-b, r0, 1.0), r0)};
+#endif
+    return {b, T(0)};
+}
+template <typename T> CFFC_HD T rdivf(T a, const Recip<T> &d) {
 #if defined(__HIP_DEVICE_COMPILE__)
     if constexpr (!Fast<T>::on) {
-        double q = a * d.r;
-        const double rem = fma(-d.b, q, a);
-        q = fma(rem, d.r, q);
-        return __builtin_amdgcn_div_fixup(q, d.b, a);
+        const double q = a * d.r;
+        return fma(fma(-d.b, q, a), d.r, q);
     }
+#endif
+    return a / d.b;
+}
+template <typename T> CFFC_HD T rdiv(T a, const Recip<T> &d) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (!Fast<T>::on) return __builtin_amdgcn_div_fixup(rdivf(a, d), d.b, a);
 #endif
     return a / d.b;
 }
 template <typename T> CFFC_HD T qdiv(T a, T b) {
     if constexpr (Fast<T>::on) return a * __builtin_amdgcn_rcpf(b);
     else return rdiv(a, recip(b));
+}
+// the same without the special operands' fix-up (rdivf)
+template <typename T> CFFC_HD T qdivf(T a, T b) {
+    if constexpr (Fast<T>::on) return a * __builtin_amdgcn_rcpf(b);
+    else return rdivf(a, recip(b));
+}
+// a + s*x for s = +-2^k: s*x is exact, so the fused result is the separately
+// rounded one (FP64 path; the mixed path contracts by itself)
+template <typename T> CFFC_HD T add2k(T a, T s, T x) {
+    if constexpr (Fast<T>::on) return a + s * x;
+    else return fma(s, x, a);
 }
 // Correctly rounded FP64 square root: gfx950's own IEEE sqrt(x) (v_rsq_f64,
 // then Goldschmidt's coupled iteration for g ~ sqrt(x) and h ~ 1/(2 sqrt(x))
@@ -146,6 +173,27 @@ template <typename T> CFFC_HD T qsqrt(T a) {
     }
 }
 
+// qsqrt of an FP64 value, with h = 1/(2 sqrt(a)) to about 2^-44 from the same
+// iteration (a starting value for recip_near)
+CFFC_HD double qsqrt_h(double a, double &h) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double y = __builtin_amdgcn_rsq(a);
+    double g = a * y;
+    h = y * 0.5;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    double d = fma(-g, g, a);
+    h = fma(h, r, h);
+    g = fma(d, h, g);
+    d = fma(-g, g, a);
+    g = fma(d, h, g);
+    return __builtin_amdgcn_class(a, 0x260) ? a : g;
+#else
+    h = 0.5 / sqrt(a);
+    return sqrt(a);
+#endif
+}
+
 template <typename T> struct PS { T d, vx, vy, p; };   // Euler2D_pState
 template <typename T> struct CS { T d, mx, my, E; };   // Euler2D_cState
 
@@ -159,7 +207,7 @@ template <typename T> CFFC_HD PS<T> W_of_U(const CS<T> &U) {
     W.d = U.d;
     W.vx = rdiv(U.mx, rd);
     W.vy = rdiv(U.my, rd);
-    W.p = gm1<T>() * (U.E - rdiv(Consts<T>::HALF * (U.mx * U.mx + U.my * U.my), rd));
+    W.p = gm1<T>() * (U.E - rdivf(Consts<T>::HALF * (U.mx * U.mx + U.my * U.my), rd));
     return W;
 }
 template <typename T> CFFC_HD CS<T> U_of_W(const PS<T> &W) {
@@ -213,7 +261,7 @@ template <typename T> CFFC_HD T harten_delta(T la, T ll, T lr) {
         return (tabs(la) > delta || delta < K::TOLER) ? K::ZERO : fixd;
     } else {
         if (tabs(la) > delta || delta < K::TOLER) return K::ZERO;
-        return K::HALF * (qdiv(sqr(la), delta) + delta) - tabs(la);
+        return add2k(-tabs(la), K::HALF, qdivf(sqr(la), delta) + delta);
     }
 }
 template <typename T> CFFC_HD T harten_pos(T la, T ll, T lr) {
@@ -246,6 +294,21 @@ template <typename T> CFFC_HD PS<T> roe_average(const PS<T> &Wl, const PS<T> &Wr
         Wa.p = qdiv(Wa.d * aa2, gam<T>());
     }
     return Wa;
+}
+
+// waves 2 and 3 of FluxRoe_x (FP64), which share the eigenvalue u: lp2 =
+// (1,0,0,-1/a2), rc2 = (1,u,v,|v|^2/2); lp3 = (0,0,1,0), rc3 = (0,0,d,d*v)
+template <typename T> CFFC_HD CS<T> roe_shear(CS<T> F, const PS<T> &Wl, const PS<T> &Wr, const PS<T> &Wa, T w2, T dp,
+                                              const Recip<T> &ra2, T v2) {
+    const T a = w2 * ((Wr.d - Wl.d) + rdivf(T(-1), ra2) * dp);
+    F.d += a;
+    F.mx += a * Wa.vx;
+    F.my += a * Wa.vy;
+    F.E += a * (T(0.5) * v2);
+    const T b = w2 * (Wr.vy - Wl.vy);
+    F.my += b * Wa.d;
+    F.E += b * (Wa.d * Wa.vy);
+    return F;
 }
 
 // FluxRoe_x, Euler2DState.cc:2311-2353.  The wave loop is unrolled; the
@@ -289,66 +352,74 @@ template <typename T> CFFC_HD CS<T> flux_roe_x(const PS<T> &Wl, const PS<T> &Wr)
         F.E += a1 * (ha - uc) + a2 * (K::HALF * (Wa.vx * Wa.vx + Wa.vy * Wa.vy)) + a3 * (Wa.d * Wa.vy) +
                a4 * (ha + uc);
         return F;
+    } else {
+        // FP64: the reference's values in its order of rounding.  Reciprocals of
+        // related divisors start from one another (recip_near): d and gm1*d on
+        // each side and of the average, c, c^2 and the a2() of the average.
+        // Products with the zero entries of lp/rc and the sums that only add them
+        // are left out: they could change a value only in the sign of a zero
+        // flux, and the residual, which starts from +0, adds such a flux away.
+        const T g1i = T(1.0 / (1.40 - 1.0));
+        // h() and a() of both sides and RoeAverage, Euler2DState.cc:654-683
+        const Recip<T> rdl = recip(Wl.d), rdr = recip(Wr.d);
+        const T gpl = gam<T>() * Wl.p, gpr = gam<T>() * Wr.p;
+        const T hl = add2k(rdivf(gpl, recip_near(gm1<T>() * Wl.d, rdl.r * g1i)), K::HALF, sqr(Wl.vx) + sqr(Wl.vy));
+        const T hr = add2k(rdivf(gpr, recip_near(gm1<T>() * Wr.d, rdr.r * g1i)), K::HALF, sqr(Wr.vx) + sqr(Wr.vy));
+        const T cl = qsqrt(rdivf(gpl, rdl)), cr = qsqrt(rdivf(gpr, rdr));
+        const T sdl = qsqrt(Wl.d), sdr = qsqrt(Wr.d);
+        const Recip<T> rs = recip(sdl + sdr);
+        PS<T> Wa;
+        Wa.d = sdl * sdr;
+        Wa.vx = rdivf(sdl * Wl.vx + sdr * Wr.vx, rs);
+        Wa.vy = rdivf(sdl * Wl.vy + sdr * Wr.vy, rs);
+        const T v2 = sqr(Wa.vx) + sqr(Wa.vy);
+        const T aa2 = gm1<T>() * add2k(rdivf(sdl * hl + sdr * hr, rs), -K::HALF, v2);
+        const Recip<T> rgam = {gam<T>(), T(1.0 / 1.40)};
+        Wa.p = rdivf(Wa.d * aa2, rgam);
+        // a2(), a() and h() of the average
+        const T gpa = gam<T>() * Wa.p;
+        const Recip<T> rda = recip(Wa.d);
+        const T a2a = rdivf(gpa, rda);
+        T hc;
+        const T ca = qsqrt_h(a2a, hc);
+        const T ha = add2k(rdivf(gpa, recip_near(gm1<T>() * Wa.d, rda.r * g1i)), K::HALF, v2);
+        const T la1 = Wa.vx - ca, la4 = Wa.vx + ca;
+        const bool left = (Wa.vx >= K::ZERO);
+        const T d1 = harten_delta(la1, Wl.vx - cl, Wr.vx - cr);
+        const T d4 = harten_delta(la4, Wl.vx + cl, Wr.vx + cr);
+        // Flux += the negative parts HALF*(la - |la| - delta) on the left side,
+        // Flux -= the positive parts HALF*(la + |la| + delta) on the right: with
+        // la' = la or -la both are added as HALF*(la' - |la| - delta)
+        const T w1 = K::HALF * ((left ? la1 : -la1) - tabs(la1) - d1);
+        const T w2 = K::HALF * ((left ? Wa.vx : -Wa.vx) - tabs(Wa.vx));
+        const T w4 = K::HALF * ((left ? la4 : -la4) - tabs(la4) - d4);
+        const PS<T> Wu = left ? Wl : Wr;
+        CS<T> F = W_Fx(Wu);
+        const T du = Wr.vx - Wl.vx, dp = Wr.p - Wl.p;
+        const Recip<T> rc = recip_near(ca, K::TWO * hc);
+        const Recip<T> rc2 = recip_near(sqr(ca), sqr(rc.r));
+        // waves 1 and 4: lp = (0, -+HALF*d/c, 0, HALF/c^2), rc = (1, u-+c, v,
+        // h-+u*c); (-HALF*d)/c is -(HALF*d/c) bit for bit
+        if (w1 != K::ZERO || w4 != K::ZERO) {
+            const T lu = rdivf(K::HALF * Wa.d, rc) * du, lp = rdivf(K::HALF, rc2) * dp;
+            const T uc = Wa.vx * ca;
+            const T a = w1 * (lp - lu);
+            F.d += a;
+            F.mx += a * la1;
+            F.my += a * Wa.vy;
+            F.E += a * (ha - uc);
+            // F changes by the waves one after the other: 1, then 2 and 3, then 4
+            if (w2 != K::ZERO) F = roe_shear(F, Wl, Wr, Wa, w2, dp, recip_near(a2a, rc2.r), v2);
+            const T b = w4 * (lu + lp);
+            F.d += b;
+            F.mx += b * la4;
+            F.my += b * Wa.vy;
+            F.E += b * (ha + uc);
+        } else if (w2 != K::ZERO) {
+            F = roe_shear(F, Wl, Wr, Wa, w2, dp, recip_near(a2a, rc2.r), v2);
+        }
+        return F;
     }
-    const PS<T> Wa = roe_average(Wl, Wr);
-    const PS<T> dW = {Wr.d - Wl.d, Wr.vx - Wl.vx, Wr.vy - Wl.vy, Wr.p - Wl.p};
-    // a() = sqrt(g*p/d) and a2() = g*p/d share the quotient; h() is needed by
-    // rc_x for waves 1 and 4, computed once
-    const T a2a = W_a2(Wa);
-    const T cl = W_a(Wl), cr = W_a(Wr), ca = qsqrt(a2a);
-    const T ha = W_h(Wa);
-    const T la1 = Wa.vx - ca, la4 = Wa.vx + ca;
-    const bool left = (Wa.vx >= K::ZERO);
-    const T d1 = harten_delta(la1, Wl.vx - cl, Wr.vx - cr);
-    const T d4 = harten_delta(la4, Wl.vx + cl, Wr.vx + cr);
-    const T w1 = left ? K::HALF * (la1 - tabs(la1) - d1) : K::HALF * (la1 + tabs(la1) + d1);
-    const T w2 = left ? K::HALF * (Wa.vx - tabs(Wa.vx)) : K::HALF * (Wa.vx + tabs(Wa.vx));
-    const T w4 = left ? K::HALF * (la4 - tabs(la4) - d4) : K::HALF * (la4 + tabs(la4) + d4);
-    const PS<T> Wu = left ? Wl : Wr;
-    CS<T> F = W_Fx(Wu);
-    const T sg = left ? T(1) : T(-1);   // Flux += (left) / Flux -= (right): exact sign flip
-    // waves 1 and 4 share lp4 = HALF/c^2 and, up to sign, lp2 = -+HALF*d/c:
-    // (-HALF*d)/c is -(HALF*d/c) bit for bit (a negated product, then a
-    // negated quotient), so each is divided once
-    T lp2w4 = K::ZERO, lp4w14 = K::ZERO;
-    if (w1 != K::ZERO || w4 != K::ZERO) {
-        lp2w4 = qdiv(K::HALF * Wa.d, ca);
-        lp4w14 = qdiv(K::HALF, sqr(ca));
-    }
-    // wave 1: lp = (0, -HALF*d/c, 0, HALF/c^2), rc = (1, u-c, v, h-u*c)
-    if (Fast<T>::on || w1 != K::ZERO) {
-        const T lp2 = -lp2w4, lp4 = lp4w14;
-        const T a = sg * (w1 * (K::ZERO * dW.d + (lp2 * dW.vx + K::ZERO * dW.vy) + lp4 * dW.p));
-        F.d += a * K::ONE;
-        F.mx += a * (Wa.vx - ca);
-        F.my += a * Wa.vy;
-        F.E += a * (ha - Wa.vx * ca);
-    }
-    // waves 2 and 3 share the eigenvalue u; lp2 = (1,0,0,-1/a2), rc2 =
-    // (1,u,v,|v|^2/2); lp3 = (0,0,1,0), rc3 = (0,0,d,d*v)
-    if (Fast<T>::on || w2 != K::ZERO) {
-        const T lp4 = qdiv(-K::ONE, a2a);
-        const T a = sg * (w2 * (K::ONE * dW.d + (K::ZERO * dW.vx + K::ZERO * dW.vy) + lp4 * dW.p));
-        F.d += a * K::ONE;
-        F.mx += a * Wa.vx;
-        F.my += a * Wa.vy;
-        F.E += a * (K::HALF * (Wa.vx * Wa.vx + Wa.vy * Wa.vy));
-        const T b = sg * (w2 * (K::ZERO * dW.d + (K::ZERO * dW.vx + K::ONE * dW.vy) + K::ZERO * dW.p));
-        F.d += b * K::ZERO;
-        F.mx += b * K::ZERO;
-        F.my += b * Wa.d;
-        F.E += b * (Wa.d * Wa.vy);
-    }
-    // wave 4: lp = (0, HALF*d/c, 0, HALF/c^2), rc = (1, u+c, v, h+u*c)
-    if (Fast<T>::on || w4 != K::ZERO) {
-        const T lp2 = lp2w4, lp4 = lp4w14;
-        const T a = sg * (w4 * (K::ZERO * dW.d + (lp2 * dW.vx + K::ZERO * dW.vy) + lp4 * dW.p));
-        F.d += a * K::ONE;
-        F.mx += a * (Wa.vx + ca);
-        F.my += a * Wa.vy;
-        F.E += a * (ha + Wa.vx * ca);
-    }
-    return F;
 }
 
 // FluxRoe_n, Euler2DState.cc:2446-2489
@@ -436,8 +507,8 @@ template <typename T> CFFC_HD PS<T> bc_characteristic_pressure(const PS<T> &Wi, 
 // caller folds phi = min(phi, f) over the four face midpoints.  For y >= 2
 // the rational term f(y) = (y^2+2y)/(y^2+y+2) is >= 1 and cannot lower
 // phi <= 1.  When a multiply-only test proves y >= 2.001 (a margin far above
-// rounding) and y is nowhere near overflow, both divisions are skipped: the
-// result is bit-identical to evaluating the reference's expression.
+// rounding), both divisions are skipped: the result is bit-identical to
+// evaluating the reference's expression.
 template <typename T> CFFC_HD T venkat_fold(T phi, T uq, T u0, T u0Min, T u0Max) {
     typedef Consts<T> K;
     const T du = uq - u0;
@@ -451,21 +522,17 @@ template <typename T> CFFC_HD T venkat_fold(T phi, T uq, T u0, T u0Min, T u0Max)
         const T f = (y * y + K::TWO * y) * __builtin_amdgcn_rcpf(y * y + y + K::TWO);
         return fminf(phi, fabsf(du) > K::TOLER ? f : K::ONE);
     }
-    T num;
-    if (du > K::TOLER) {
-        num = u0Max - u0;  // y = num/du, both >= 0
-        if (num >= T(2.002) * du && num <= T(1.0e12) * du) return phi;
-    } else if (du < -K::TOLER) {
-        num = u0Min - u0;  // y = num/du, both <= 0
-        if (num <= T(2.002) * du && num >= T(1.0e12) * du) return phi;
-    } else {
-        return vmin64(phi, K::ONE);
+    // y = num/du >= 0, both of one sign; f(y >= 2) >= 1 after its roundings,
+    // so such a quotient and the dead band leave phi <= 1 as it is
+    const T num = du > T(0) ? u0Max - u0 : u0Min - u0;
+    if (tabs(du) > K::TOLER && tabs(num) < T(2.002) * tabs(du)) {
+        // f is never -0 or NaN, so the one-instruction minimum equals the
+        // reference's compare-and-select
+        const T y = qdivf(num, du);
+        const T y2 = sqr(y);
+        phi = vmin64(phi, qdivf(add2k(y2, K::TWO, y), y2 + y + K::TWO));
     }
-    // phi and f(y) are never -0 or NaN (phi starts at 1, f(+-0) = +0; y is
-    // finite since |du| > TOLER and |num| << 1e147), so the one-instruction
-    // minimum equals the reference's compare-and-select
-    const T y = qdiv(num, du);
-    return vmin64(phi, qdiv(sqr(y) + K::TWO * y, sqr(y) + y + K::TWO));
+    return phi;
 }
 
 }  // namespace cffc
