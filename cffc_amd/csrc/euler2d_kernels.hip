@@ -869,10 +869,17 @@ hipError_t cffc_launch_finish(const FinishParams *p, double *chunk_part, int nch
 }
 
 hipError_t cffc_launch_stage_fp64(const StageParams *p, int ti, int tj, int fused, hipStream_t st) {
+    int kind = stage_kind(*p, fused);
 #define L(TI, TJ)                                                                                          \
     if (ti == TI && tj == TJ) {                                                                            \
-        if (fused) hipLaunchKernelGGL((stage_kernel<double, TI, TJ, true>), dim3(p->ntiles), dim3((TileThreads<TI, TJ>::value)), 0, st, *p); \
-        else hipLaunchKernelGGL((stage_kernel<double, TI, TJ, false>), dim3(p->ntiles), dim3((TileThreads<TI, TJ>::value)), 0, st, *p); \
+        switch (kind) {                                                                                    \
+        case SK_PLAIN: launch_stage_kernel<double, TI, TJ, SK_PLAIN>(p, st); break;                            \
+        case SK_LEVELS: launch_stage_kernel<double, TI, TJ, SK_LEVELS>(p, st); break;                          \
+        case SK_MG: launch_stage_kernel<double, TI, TJ, SK_MG>(p, st); break;                              \
+        case SK_MG_FIRST: launch_stage_kernel<double, TI, TJ, SK_MG_FIRST>(p, st); break;                  \
+        case SK_FUSED: launch_stage_kernel<double, TI, TJ, SK_FUSED>(p, st); break;                            \
+        default: launch_stage_kernel<double, TI, TJ, SK_GRANULAR>(p, st); break;                               \
+        }                                                                                                  \
         return hipGetLastError();                                                                          \
     }
     CFFC_TILE_LIST(L)

@@ -10,10 +10,16 @@
 using namespace cffc;
 
 extern "C" hipError_t cffc_launch_stage_mixed(const StageParams *p, int ti, int tj, int fused, hipStream_t st) {
+    int kind = stage_kind(*p, fused);
+    if (kind == SK_MG || kind == SK_MG_FIRST) kind = SK_GRANULAR;   // FP64 only
 #define L(TI, TJ)                                                                                          \
     if (ti == TI && tj == TJ) {                                                                            \
-        if (fused) hipLaunchKernelGGL((stage_kernel<float, TI, TJ, true>), dim3(p->ntiles), dim3((TileThreads<TI, TJ>::value)), 0, st, *p); \
-        else hipLaunchKernelGGL((stage_kernel<float, TI, TJ, false>), dim3(p->ntiles), dim3((TileThreads<TI, TJ>::value)), 0, st, *p); \
+        switch (kind) {                                                                                    \
+        case SK_PLAIN: launch_stage_kernel<float, TI, TJ, SK_PLAIN>(p, st); break;                            \
+        case SK_LEVELS: launch_stage_kernel<float, TI, TJ, SK_LEVELS>(p, st); break;                          \
+        case SK_FUSED: launch_stage_kernel<float, TI, TJ, SK_FUSED>(p, st); break;                            \
+        default: launch_stage_kernel<float, TI, TJ, SK_GRANULAR>(p, st); break;                               \
+        }                                                                                                  \
         return hipGetLastError();                                                                          \
     }
     CFFC_TILE_LIST(L)

@@ -182,13 +182,83 @@ __device__ __forceinline__ typename CoordT<FT>::type rdgeo(const StageParams &p,
     else return p.geom[gd * p.ncp + i];
 }
 
+// Element access by a 32-bit byte offset from a base that is the same for the
+// whole workgroup (plane + row j0 of the block, the tile's first window row):
+// one scalar register pair per plane and one vector register per cell,
+// instead of a 64-bit vector address per access.  A window of TJ + 4 rows
+// stays far below 4 GiB whatever the block's size.
+template <typename T> __device__ __forceinline__ T at(const T *base, uint32_t off) {
+    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + off);
+}
+template <typename T> __device__ __forceinline__ T &at(T *base, uint32_t off) {
+    return *reinterpret_cast<T *>(reinterpret_cast<char *>(base) + off);
+}
+// geometry planes from padded cell `org` on: element offsets in bytes of XT
+template <typename FT> struct BlockGeo {
+    typedef typename CoordT<FT>::type XT;
+    const XT *g;    // plane 0 at the origin
+    int64_t ncp;
+    uint32_t row;   // bytes per row
+    __device__ __forceinline__ BlockGeo(const StageParams &p, const BlockMeta &m, int64_t org) : ncp(p.ncp) {
+        if constexpr (Fast<FT>::on) g = p.geomf + org;
+        else g = p.geom + org;
+        row = (uint32_t)m.pitch * (uint32_t)sizeof(XT);
+    }
+    __device__ __forceinline__ XT rd(int gd, int gf, uint32_t off) const {
+        return at(g + (Fast<FT>::on ? gf : gd) * ncp, off);
+    }
+    // the same plane one cell to the west, one row to the south
+    __device__ __forceinline__ XT rdw(int gd, int gf, uint32_t off) const {
+        return at(g + (Fast<FT>::on ? gf : gd) * ncp - 1, off);
+    }
+    __device__ __forceinline__ XT rds(int gd, int gf, uint32_t off) const {
+        return at(g + (Fast<FT>::on ? gf : gd) * ncp - row / (uint32_t)sizeof(XT), off);
+    }
+};
+
+// What a stage kernel is built to do.  The general kernels carry every option
+// as a run-time switch; their scalar registers spill into vector lanes and
+// more than a third of their vector instructions do no arithmetic.  The others
+// drop at compile time what a launch does not use; stage_kind picks by the
+// parameters.  The limiter's load/evaluate switch stays in all of them: without
+// its branch the compiler moves the limiter's geometry loads up into the
+// gradient, which takes 128 VGPRs and spills (FP64 32 x 16: 0.50 ms per stage
+// at 4.2 M cells against 0.39 ms).
+enum StageKind {
+    SK_GRANULAR = 0,   // dUdt_Multistage_Explicit on its own, every option
+    SK_FUSED = 1,      // residual + update, every option
+    SK_PLAIN = 2,      // fused: one level, planar, Venkatakrishnan
+    SK_LEVELS = 3,     // the same with resolution changes
+    SK_MG = 4,         // granular: one level, planar, Venkatakrishnan, Roe
+    SK_MG_FIRST = 5    // granular multigrid stage of a first-order level: zero limiter, so no reconstruction
+};
+template <int K> struct StageOpt {
+    static constexpr bool fused = K == SK_FUSED || K == SK_PLAIN || K == SK_LEVELS;
+    static constexpr bool general = K == SK_GRANULAR || K == SK_FUSED;   // axisymmetric, any limiter
+    static constexpr bool amr = general || K == SK_LEVELS;
+    static constexpr bool first = K == SK_MG_FIRST;
+};
+// the leanest kernel that has every option of the launch
+inline int stage_kind(const StageParams &p, int fused) {
+    const bool venkat = p.limiter == 9;
+    if (fused) {
+        if (p.axisym || !venkat || p.defer_update) return SK_FUSED;
+        return p.eflux || p.tile_defer || p.Ustage ? SK_LEVELS : SK_PLAIN;
+    }
+    if (p.axisym || p.eflux || p.mode == GINIT_RK4) return SK_GRANULAR;
+    if (p.hlle) return p.limiter == 0 && p.phi_mode != PHI_LOAD ? SK_MG_FIRST : SK_GRANULAR;
+    return venkat ? SK_MG : SK_GRANULAR;
+}
+
 // Least-squares gradient and Venkatakrishnan limiter of one cell
 // (Linear_Reconstruction_LeastSquares, SingleBlock.cc:3678-4087).  FULL: the
 // 8-point stencil, straight-line; otherwise the reduced stencil in mask.
 // The window arrays are indexed [row][col] with the cell at (jl, il).
-template <typename FT, bool FULL, int LJ, int LI, typename XT>
-__device__ __forceinline__ void reconstruct(const StageParams &p, int phim, int64_t c, int64_t ncp, int pitch, int il,
-                                            int jl, unsigned mask, const FT (&sW)[4][LJ][LI], const XT (&sX)[LJ][LI],
+// off: the cell's byte offset in a geometry plane; o8: in an FP64 plane.
+template <typename FT, typename O, bool FULL, int LJ, int LI, typename XT>
+__device__ __forceinline__ void reconstruct(const StageParams &p, const BlockGeo<FT> &geo, const double *phi, int phim,
+                                            uint32_t off, uint32_t o8, int il, int jl, unsigned mask,
+                                            const FT (&sW)[4][LJ][LI], const XT (&sX)[LJ][LI],
                                             const XT (&sY)[LJ][LI], PS<FT> &gx, PS<FT> &gy, PS<FT> &ph) {
     const PS<FT> W0 = {sW[0][jl][il], sW[1][jl][il], sW[2][jl][il], sW[3][jl][il]};
     gx = {FT(0), FT(0), FT(0), FT(0)};
@@ -243,18 +313,21 @@ __device__ __forceinline__ void reconstruct(const StageParams &p, int phim, int6
         gy.vy = rdivf(Dy.vy * DxDx - Dx.vy * DxDy, rd); gy.p = rdivf(Dy.p * DxDx - Dx.p * DxDy, rd);
     }
     if (phim == PHI_LOAD) {
-        ph.d = (FT)p.phi[c]; ph.vx = (FT)p.phi[ncp + c]; ph.vy = (FT)p.phi[2 * ncp + c]; ph.p = (FT)p.phi[3 * ncp + c];
+        ph.d = (FT)at(phi, o8); ph.vx = (FT)at(phi + geo.ncp, o8);
+        ph.vy = (FT)at(phi + 2 * geo.ncp, o8); ph.p = (FT)at(phi + 3 * geo.ncp, o8);
         return;
     }
-    if (p.limiter == -1) { ph.d = ph.vx = ph.vy = ph.p = FT(1); return; }
-    if (p.limiter == 0) { ph.d = ph.vx = ph.vy = ph.p = FT(0); return; }
+    if constexpr (O::general) {
+        if (p.limiter == -1) { ph.d = ph.vx = ph.vy = ph.p = FT(1); return; }
+        if (p.limiter == 0) { ph.d = ph.vx = ph.vy = ph.p = FT(0); return; }
+    }
+    // the eight midpoint loads stay here (see StageKind)
+    if constexpr (Fast<FT>::on) __builtin_amdgcn_sched_barrier(0);
     // face-midpoint offsets: E, W (= E of i-1), N, S (= N of j-1)
-    const FT dxE = (FT)(rdgeo<FT>(p, GEO_XFE, GF_XFE, c) - xc0), dyE = (FT)(rdgeo<FT>(p, GEO_YFE, GF_YFE, c) - yc0);
-    const FT dxW = (FT)(rdgeo<FT>(p, GEO_XFE, GF_XFE, c - 1) - xc0);
-    const FT dyW = (FT)(rdgeo<FT>(p, GEO_YFE, GF_YFE, c - 1) - yc0);
-    const FT dxN = (FT)(rdgeo<FT>(p, GEO_XFN, GF_XFN, c) - xc0), dyN = (FT)(rdgeo<FT>(p, GEO_YFN, GF_YFN, c) - yc0);
-    const FT dxS = (FT)(rdgeo<FT>(p, GEO_XFN, GF_XFN, c - pitch) - xc0);
-    const FT dyS = (FT)(rdgeo<FT>(p, GEO_YFN, GF_YFN, c - pitch) - yc0);
+    const FT dxE = (FT)(geo.rd(GEO_XFE, GF_XFE, off) - xc0), dyE = (FT)(geo.rd(GEO_YFE, GF_YFE, off) - yc0);
+    const FT dxW = (FT)(geo.rdw(GEO_XFE, GF_XFE, off) - xc0), dyW = (FT)(geo.rdw(GEO_YFE, GF_YFE, off) - yc0);
+    const FT dxN = (FT)(geo.rd(GEO_XFN, GF_XFN, off) - xc0), dyN = (FT)(geo.rd(GEO_YFN, GF_YFN, off) - yc0);
+    const FT dxS = (FT)(geo.rds(GEO_XFN, GF_XFN, off) - xc0), dyS = (FT)(geo.rds(GEO_YFN, GF_YFN, off) - yc0);
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
         const FT u0 = n == 0 ? W0.d : n == 1 ? W0.vx : n == 2 ? W0.vy : W0.p;
@@ -325,13 +398,16 @@ template <typename FT> __device__ __forceinline__ bool positivity_fails(const CS
 // planes in the FP64 path, FP32 planes in the mixed path); U0: U^n of the
 // cell; Sacc: the FP64 accumulator's value as the caller loaded it, if
 // have_Sacc.
-template <typename FT>
-__device__ __forceinline__ void fused_update(const StageParams &p, const BlockMeta &m, const TileDesc &t, int64_t c,
-                                             int ip, int jp, double A, double dtc, double lW, double lE, double lS,
+template <typename FT, typename O>
+__device__ __forceinline__ void fused_update(const StageParams &p, const BlockGeo<FT> &geo, const BlockMeta &m,
+                                             const TileDesc &t, int64_t org, uint32_t o8, int ip, int jp, double A, double dtc, double lW, double lE, double lS,
                                              double lN, const double (&U0)[4], bool have_Sacc,
                                              const double (&Sacc)[4], double (&dU)[4], double &l1, double &l2,
                                              double &mx, double &dtn) {
     const double om = p.omega;
+    const int64_t ncp = p.ncp;
+    const uint32_t o4 = o8 / 2, og = Fast<FT>::on ? o4 : o8;
+    double *dtb = p.dt + org;
     CS<double> Un;
     Un.d = U0[0] + om * dU[0]; Un.mx = U0[1] + om * dU[1];
     Un.my = U0[2] + om * dU[2]; Un.E = U0[3] + om * dU[3];
@@ -348,7 +424,7 @@ __device__ __forceinline__ void fused_update(const StageParams &p, const BlockMe
             Un.my = U0[2] + om * dU[2]; Un.E = U0[3] + om * dU[3];
             if (!positivity_fails<FT>(Un)) break;
         }
-        p.dt[c] = dtl;
+        at(dtb, o8) = dtl;
         bad = positivity_fails<FT>(Un);
     }
     if (bad) {
@@ -367,17 +443,24 @@ __device__ __forceinline__ void fused_update(const StageParams &p, const BlockMe
         Wn = W_of_U(Un);
     }
     if constexpr (Fast<FT>::on) {
-        p.Woutf[c] = (float)Wn.d; p.Woutf[p.ncp + c] = (float)Wn.vx;
-        p.Woutf[2 * p.ncp + c] = (float)Wn.vy; p.Woutf[3 * p.ncp + c] = (float)Wn.p;
+        float *Wb = p.Woutf + org;
+        at(Wb, o4) = (float)Wn.d; at(Wb + ncp, o4) = (float)Wn.vx;
+        at(Wb + 2 * ncp, o4) = (float)Wn.vy; at(Wb + 3 * ncp, o4) = (float)Wn.p;
         if (p.push) push_ghosts(p, p.Woutf, m, t.b, ip, jp, Wn);
     } else {
-        p.Wout[c] = Wn.d; p.Wout[p.ncp + c] = Wn.vx; p.Wout[2 * p.ncp + c] = Wn.vy; p.Wout[3 * p.ncp + c] = Wn.p;
+        double *Wb = p.Wout + org;
+        at(Wb, o8) = Wn.d; at(Wb + ncp, o8) = Wn.vx; at(Wb + 2 * ncp, o8) = Wn.vy; at(Wb + 3 * ncp, o8) = Wn.p;
         if (p.push) push_ghosts(p, p.Wout, m, t.b, ip, jp, Wn);
     }
-    if ((m.amr & AMR_USTORE) && p.Ustage && p.ustore[c]) {
-        // a coarser neighbour restricts U^(s+1) of this cell into its ghosts
-        p.Ustage[c] = Un.d; p.Ustage[p.ncp + c] = Un.mx; p.Ustage[2 * p.ncp + c] = Un.my; p.Ustage[3 * p.ncp + c] = Un.E;
+    if constexpr (O::amr) {
+        if ((m.amr & AMR_USTORE) && p.Ustage && p.ustore[org + o8 / 8]) {
+            // a coarser neighbour restricts U^(s+1) of this cell into its ghosts
+            double *Us = p.Ustage + org;
+            at(Us, o8) = Un.d; at(Us + ncp, o8) = Un.mx; at(Us + 2 * ncp, o8) = Un.my; at(Us + 3 * ncp, o8) = Un.E;
+        }
     }
+    float *Sfb = Fast<FT>::on && p.Sf ? p.Sf + org : nullptr;
+    double *Sb = p.S + org;
     if (p.skip_S) {
         // the next stage starts from zero and the last stage stores dUdt[0]
     } else if (Fast<FT>::on && p.Sf) {
@@ -385,39 +468,38 @@ __device__ __forceinline__ void fused_update(const StageParams &p, const BlockMe
         // is kept in FP32 (half the bytes); the stage's own dU stays FP64
         if (p.mode == MODE_ZERO_ACC2) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) p.Sf[v * p.ncp + c] = (float)((double)p.Sf[v * p.ncp + c] + 2.0 * dU[v]);
+            for (int v = 0; v < 4; ++v) at(Sfb + v * ncp, o4) = (float)((double)at(Sfb + v * ncp, o4) + 2.0 * dU[v]);
         } else {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) p.Sf[v * p.ncp + c] = (float)dU[v];
+            for (int v = 0; v < 4; ++v) at(Sfb + v * ncp, o4) = (float)dU[v];
         }
     } else if (p.mode == MODE_ZERO_ACC2) {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) p.S[v * p.ncp + c] = (have_Sacc ? Sacc[v] : p.S[v * p.ncp + c]) + 2.0 * dU[v];
+        for (int v = 0; v < 4; ++v) at(Sb + v * ncp, o8) = add2k(have_Sacc ? Sacc[v] : at(Sb + v * ncp, o8), 2.0, dU[v]);
     } else {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) p.S[v * p.ncp + c] = dU[v];
+        for (int v = 0; v < 4; ++v) at(Sb + v * ncp, o8) = dU[v];
     }
     if (p.last_stage) {
-        p.U[c] = Un.d; p.U[p.ncp + c] = Un.mx; p.U[2 * p.ncp + c] = Un.my; p.U[3 * p.ncp + c] = Un.E;
+        double *Ub = p.U + org;
+        at(Ub, o8) = Un.d; at(Ub + ncp, o8) = Un.mx; at(Ub + 2 * ncp, o8) = Un.my; at(Ub + 3 * ncp, o8) = Un.E;
         l1 = fabs(dU[0]);
         l2 = dU[0] * dU[0];
         mx = l1;
         // CFL of the next step, SingleBlock.cc:3036-3053, in FP64 from the
         // geometry planes the stage reads (the mixed path's FP32 normals and
         // lengths are still in cache from its flux phase)
-        const double d_i = 2.0 * qdiv(A, lE + lW);
-        const double d_j = 2.0 * qdiv(A, lN + lS);
-        const double nEx = rdgeo<FT>(p, GEO_NEX, GF_NEX, c), nEy = rdgeo<FT>(p, GEO_NEY, GF_NEY, c);
-        const double nNx = rdgeo<FT>(p, GEO_NNX, GF_NNX, c), nNy = rdgeo<FT>(p, GEO_NNY, GF_NNY, c);
-        const double nWx = -(double)rdgeo<FT>(p, GEO_NEX, GF_NEX, c - 1);
-        const double nWy = -(double)rdgeo<FT>(p, GEO_NEY, GF_NEY, c - 1);
-        const double nSx = -(double)rdgeo<FT>(p, GEO_NNX, GF_NNX, c - m.pitch);
-        const double nSy = -(double)rdgeo<FT>(p, GEO_NNY, GF_NNY, c - m.pitch);
+        const double d_i = 2.0 * qdivf(A, lE + lW);
+        const double d_j = 2.0 * qdivf(A, lN + lS);
+        const double nEx = geo.rd(GEO_NEX, GF_NEX, og), nEy = geo.rd(GEO_NEY, GF_NEY, og);
+        const double nNx = geo.rd(GEO_NNX, GF_NNX, og), nNy = geo.rd(GEO_NNY, GF_NNY, og);
+        const double nWx = -(double)geo.rdw(GEO_NEX, GF_NEX, og), nWy = -(double)geo.rdw(GEO_NEY, GF_NEY, og);
+        const double nSx = -(double)geo.rds(GEO_NNX, GF_NNX, og), nSy = -(double)geo.rds(GEO_NNY, GF_NNY, og);
         const double v_i = 0.5 * (Wn.vx * (nEx - nWx) + Wn.vy * (nEy - nWy));
         const double v_j = 0.5 * (Wn.vx * (nNx - nSx) + Wn.vy * (nNy - nSy));
         const double a = W_a(Wn);
         dtn = dmin(qdiv(d_i, a + fabs(v_i)), qdiv(d_j, a + fabs(v_j)));
-        if (p.lts) p.dt[c] = dtn;
+        if (p.lts) at(dtb, o8) = dtn;
     }
 }
 
@@ -437,12 +519,14 @@ template <int TI, int TJ> struct TileThreads {
 // tiles fit six in 80 VGPRs without spilling (0.5% faster at 32 x 8 than the
 // five that 82 VGPRs allow); the FP64 kernels are left to the compiler.
 template <typename FT, int TI, int TJ> struct StageWaves {
-    static constexpr int value = (Fast<FT>::on && TileThreads<TI, TJ>::ring_pass) ? 6 : 1;
+    static constexpr int value = Fast<FT>::on ? (TileThreads<TI, TJ>::ring_pass ? 6 : 1) : 4;
 };
 
-template <typename FT, int TI, int TJ, bool FUSED>
+template <typename FT, int TI, int TJ, int KIND>
 __global__ __launch_bounds__((TileThreads<TI, TJ>::value))
 __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_kernel(StageParams p) {
+    typedef StageOpt<KIND> O;
+    constexpr bool FUSED = O::fused;
     constexpr int NT = TileThreads<TI, TJ>::value;
     constexpr int NTILE = TI * TJ;
     constexpr int LI = TI + 4, LJ = TJ + 4;
@@ -473,6 +557,9 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
     if (!FUSED && m.skip) return;   // a converged case of a multigrid batch
     const int tid = threadIdx.x;
     const int64_t ncp = p.ncp;
+    // origin of the tile's 32-bit offsets: cell (0, j0) of the padded block
+    const int64_t org = m.coff + (int64_t)t.j0 * m.pitch;
+    const BlockGeo<FT> geo(p, m, org);
     int phim = p.phi_mode;
     if (FUSED && p.part_state) {
         // batched steady run: a converged part is left alone, a frozen part
@@ -503,12 +590,11 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
         phim = ps == PART_FROZEN ? PHI_LOAD : p.last_stage ? PHI_COMPUTE_STORE : PHI_COMPUTE;
     }
     if (!FUSED && p.part_frozen) phim = p.part_frozen[p.part_of_block[t.b]] ? PHI_LOAD : PHI_COMPUTE_STORE;
-    const double *G = p.geom;
     const int ICu = m.ni + 1, JCu = m.nj + 1;
     const int pi0 = t.i0, pj0 = t.j0;   // padded index of the LDS window origin
     // the update waits (in update_tile_kernel) for residual smoothing, or
     // for the flux correction of a tile next to a finer neighbour
-    const bool defer = FUSED && (p.defer_update || (p.tile_defer && p.tile_defer[tix]));
+    const bool defer = FUSED && O::amr && (p.defer_update || (p.tile_defer && p.tile_defer[tix]));
     const int32_t *bcW = p.bc + m.bcoff, *bcE = bcW + m.ncj, *bcS = bcE + m.ncj, *bcN = bcS + m.nci;
     // role of this thread: a tile cell (tc, tr), or a ring cell of side
     // 0 = W (column -1), 1 = E (column TI), 2 = S (row -1), 3 = N (row TJ)
@@ -524,6 +610,9 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
     }
 
     // ---- phase 1: W and centroids of the window ---------------------------
+    const double *Win = p.Win + org;
+    const float *Winf = FUSED && Fast<FT>::on ? p.Winf + org : nullptr;
+    constexpr uint32_t XS = sizeof(XT);
     if constexpr (!RP) {
         // tiles with ring threads: every thread issues the loads of all its
         // window cells before its first LDS store, without branches.  A
@@ -542,14 +631,14 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
             slot[k] = qq;
             const int ip = pi0 + qq % LI, jp = pj0 + qq / LI;
             const int ipc = ip < m.nci ? ip : m.nci - 1, jpc = jp < m.ncj ? jp : m.ncj - 1;
-            const int64_t c = m.coff + (int64_t)jpc * m.pitch + ipc;
+            const uint32_t e = (uint32_t)((jpc - pj0) * m.pitch + ipc);
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                if constexpr (FUSED && Fast<FT>::on) wv[k][v] = p.Winf[v * ncp + c];
-                else wv[k][v] = (FT)p.Win[v * ncp + c];
+                if constexpr (FUSED && Fast<FT>::on) wv[k][v] = at(Winf + v * ncp, e * 4u);
+                else wv[k][v] = (FT)at(Win + v * ncp, e * 8u);
             }
-            xw[k] = rdgeo<FT>(p, GEO_XC, GF_XC, c);
-            yw[k] = rdgeo<FT>(p, GEO_YC, GF_YC, c);
+            xw[k] = geo.rd(GEO_XC, GF_XC, e * XS);
+            yw[k] = geo.rd(GEO_YC, GF_YC, e * XS);
         }
 #pragma unroll
         for (int k = 0; k < NIT; ++k) {
@@ -564,14 +653,14 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
             const int il = q % LI, jl = q / LI;
             const int ip = pi0 + il, jp = pj0 + jl;
             if (ip < m.nci && jp < m.ncj) {
-                const int64_t c = m.coff + (int64_t)jp * m.pitch + ip;
+                const uint32_t e = (uint32_t)((jp - pj0) * m.pitch + ip);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    if constexpr (FUSED && Fast<FT>::on) sW[v][jl][il] = p.Winf[v * ncp + c];
-                    else sW[v][jl][il] = (FT)p.Win[v * ncp + c];
+                    if constexpr (FUSED && Fast<FT>::on) sW[v][jl][il] = at(Winf + v * ncp, e * 4u);
+                    else sW[v][jl][il] = (FT)at(Win + v * ncp, e * 8u);
                 }
-                sX[jl][il] = rdgeo<FT>(p, GEO_XC, GF_XC, c);
-                sY[jl][il] = rdgeo<FT>(p, GEO_YC, GF_YC, c);
+                sX[jl][il] = geo.rd(GEO_XC, GF_XC, e * XS);
+                sY[jl][il] = geo.rd(GEO_YC, GF_YC, e * XS);
             }
         }
     }
@@ -583,7 +672,9 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
     // boundaries, and cells away from the ring next to a physical boundary,
     // use the full 8-point stencil; only the ring cells of boundary blocks
     // read the BC arrays (reduced stencils).
-    for (int role = tid; role < (RP ? NTILE + 2 * (TI + TJ) : tid + 1); role += NT) {
+    // A first-order level only records its zero limiters.
+    for (int role = tid; role < (RP ? NTILE + 2 * (TI + TJ) : tid + 1) && !(O::first && phim != PHI_COMPUTE_STORE);
+         role += NT) {
         // role: a tile cell, then the W, E, S, N ring cells
         int ir = -1, jr = -1;
         if (RP) {
@@ -601,22 +692,27 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
         const int il = ir + 1, jl = jr + 1;
         const int ip = pi0 + il, jp = pj0 + jl;
         if (ir >= 0 && ip <= m.nci - 2 && jp <= m.ncj - 2) {
-            const int64_t c = m.coff + (int64_t)jp * m.pitch + ip;
+            const uint32_t e = (uint32_t)((jp - pj0) * m.pitch + ip);
+            double *phib = p.phi + org;
             unsigned mask = 0xFFu;
-            if (m.has_bc && (ip <= 1 || ip >= ICu + 1 || jp <= 1 || jp >= JCu + 1))
+            if (!O::first && m.has_bc && (ip <= 1 || ip >= ICu + 1 || jp <= 1 || jp >= JCu + 1))
                 mask = stencil_mask(ip, jp, ICu, JCu, bcW[jp], bcE[jp], bcS[ip], bcN[ip]);
             PS<FT> gx, gy, ph;
-            if (mask == 0xFFu) reconstruct<FT, true>(p, phim, c, ncp, m.pitch, il, jl, 0xFFu, sW, sX, sY, gx, gy, ph);
-            else reconstruct<FT, false>(p, phim, c, ncp, m.pitch, il, jl, mask, sW, sX, sY, gx, gy, ph);
+            if constexpr (O::first) ph = {FT(0), FT(0), FT(0), FT(0)};
+            else if (mask == 0xFFu)
+                reconstruct<FT, O, true>(p, geo, phib, phim, e * XS, e * 8u, il, jl, 0xFFu, sW, sX, sY, gx, gy, ph);
+            else reconstruct<FT, O, false>(p, geo, phib, phim, e * XS, e * 8u, il, jl, mask, sW, sX, sY, gx, gy, ph);
             if (phim == PHI_COMPUTE_STORE) {
                 // each stored cell is owned by exactly one tile: its own
                 // cells, plus the block's outer ring on the block edge
                 const bool own_i = (ip >= pi0 + 2 && ip < pi0 + 2 + TI) || ip == 1 || ip == m.nci - 2;
                 const bool own_j = (jp >= pj0 + 2 && jp < pj0 + 2 + TJ) || jp == 1 || jp == m.ncj - 2;
                 if (own_i && own_j) {
-                    p.phi[c] = ph.d; p.phi[ncp + c] = ph.vx; p.phi[2 * ncp + c] = ph.vy; p.phi[3 * ncp + c] = ph.p;
+                    at(phib, e * 8u) = ph.d; at(phib + ncp, e * 8u) = ph.vx;
+                    at(phib + 2 * ncp, e * 8u) = ph.vy; at(phib + 3 * ncp, e * 8u) = ph.p;
                 }
             }
+            if constexpr (O::first) continue;
             // phi^dWdx, phi^dWdy (zero stencil: both products are 0*0)
             sPx[0][jr][ir] = ph.d * gx.d; sPx[1][jr][ir] = ph.vx * gx.vx;
             sPx[2][jr][ir] = ph.vy * gx.vy; sPx[3][jr][ir] = ph.p * gx.p;
@@ -632,24 +728,27 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
     // of row k = tid or the S ring face of column k = tid - TJ.
     // A face's normal and midpoint are read from the cell on its low side.
     struct FaceGeo { XT nx, ny, xf, yf; };
-    auto face_cell = [&](bool idir, int f, int g, int64_t &cL) -> bool {
+    auto face_cell = [&](bool idir, int f, int g, uint32_t &eL) -> bool {
         const int ipL = idir ? pi0 + 1 + f : pi0 + 2 + g;
         const int jpL = idir ? pj0 + 2 + g : pj0 + 1 + f;
-        cL = m.coff + (int64_t)jpL * m.pitch + ipL;
+        eL = (uint32_t)((jpL - pj0) * m.pitch + ipL) * XS;
         return jpL <= JCu && ipL <= ICu;
     };
-    auto face_geo = [&](bool idir, int64_t cL) -> FaceGeo {
+    // idir the same for the workgroup: each plane's base stays scalar
+    auto face_geo = [&](bool idir, uint32_t eL) -> FaceGeo {
         FaceGeo q;
-        q.nx = idir ? rdgeo<FT>(p, GEO_NEX, GF_NEX, cL) : rdgeo<FT>(p, GEO_NNX, GF_NNX, cL);
-        q.ny = idir ? rdgeo<FT>(p, GEO_NEY, GF_NEY, cL) : rdgeo<FT>(p, GEO_NNY, GF_NNY, cL);
-        q.xf = idir ? rdgeo<FT>(p, GEO_XFE, GF_XFE, cL) : rdgeo<FT>(p, GEO_XFN, GF_XFN, cL);
-        q.yf = idir ? rdgeo<FT>(p, GEO_YFE, GF_YFE, cL) : rdgeo<FT>(p, GEO_YFN, GF_YFN, cL);
+        q.nx = idir ? geo.rd(GEO_NEX, GF_NEX, eL) : geo.rd(GEO_NNX, GF_NNX, eL);
+        q.ny = idir ? geo.rd(GEO_NEY, GF_NEY, eL) : geo.rd(GEO_NNY, GF_NNY, eL);
+        if (!O::first) {
+            q.xf = idir ? geo.rd(GEO_XFE, GF_XFE, eL) : geo.rd(GEO_XFN, GF_XFN, eL);
+            q.yf = idir ? geo.rd(GEO_YFE, GF_YFE, eL) : geo.rd(GEO_YFN, GF_YFN, eL);
+        }
         return q;
     };
     const bool ring_face = RP && tid < TI + TJ;
     const bool ring_w = tid < TJ;
     const int ring_fk = ring_w ? tid : tid - TJ;
-    int64_t cF1 = 0, cF2 = 0, cFR = 0;
+    uint32_t cF1 = 0, cF2 = 0, cFR = 0;
     bool v1 = false, v2 = false, vR = false;
     if (is_tile) {
         v1 = face_cell(true, tc + 1, tr, cF1);
@@ -665,7 +764,10 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
     FaceGeo g1{}, g2{}, gR{};
     if (v1) g1 = face_geo(true, cF1);
     if (v2) g2 = face_geo(false, cF2);
-    if (vR) gR = face_geo(ring_w, cFR);
+    if (vR) {
+        if (ring_w) gR = face_geo(true, cFR);
+        else gR = face_geo(false, cFR);
+    }
     __syncthreads();
 
     // ---- phase 3: Roe fluxes ------------------------------------------------
@@ -685,6 +787,7 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
         auto load_state = [&](int ri, int rj, PS<FT> &W) {
             const int il = ri + 1, jl = rj + 1;
             W.d = sW[0][jl][il]; W.vx = sW[1][jl][il]; W.vy = sW[2][jl][il]; W.p = sW[3][jl][il];
+            if constexpr (O::first) return;   // zero limiter: the cell's own state
             const PS<FT> px = {sPx[0][rj][ri], sPx[1][rj][ri], sPx[2][rj][ri], sPx[3][rj][ri]};
             const PS<FT> py = {sPy[0][rj][ri], sPy[1][rj][ri], sPy[2][rj][ri], sPy[3][rj][ri]};
             W = face_state(W, px, py, (FT)(xf - sX[jl][il]), (FT)(yf - sY[jl][il]));
@@ -728,7 +831,9 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
             load_state(rl_i, rl_j, Wl);
             load_state(rr_i, rr_j, Wr);
         }
-        if constexpr (!FUSED && !Fast<FT>::on) {
+        if constexpr (O::first) {
+            Fout = flux_hlle_n(Wl, Wr, nx, ny);
+        } else if constexpr (KIND == SK_GRANULAR && !Fast<FT>::on) {
             Fout = p.hlle ? flux_hlle_n(Wl, Wr, nx, ny) : flux_roe_n(Wl, Wr, nx, ny);
         } else {
             Fout = flux_roe_n(Wl, Wr, nx, ny);
@@ -755,26 +860,26 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
     // thread writes U, S and dt of its cell in this launch.
     const int ip = pi0 + 2 + tc, jp = pj0 + 2 + tr;
     const bool valid = is_tile && (ip <= ICu) && (jp <= JCu);
-    const int64_t c4 = m.coff + (int64_t)jp * m.pitch + ip;
+    const uint32_t e4 = (uint32_t)((jp - pj0) * m.pitch + ip), o8 = e4 * 8u, og = e4 * XS;
     double A4 = 0.0, lW4 = 0.0, lE4 = 0.0, lS4 = 0.0, lN4 = 0.0, dt4 = 0.0;
     double U4[4] = {0.0, 0.0, 0.0, 0.0}, S4[4] = {0.0, 0.0, 0.0, 0.0};
     const bool fastS = Fast<FT>::on && p.Sf;
     const bool readS = FUSED && !fastS &&
                        (p.mode == MODE_FROM_S || (p.mode == MODE_ZERO_ACC2 && !defer && !p.skip_S));
     auto load4 = [&]() {
-        A4 = G[GEO_A * ncp + c4];
-        lW4 = rdgeo<FT>(p, GEO_LE, GF_LE, c4 - 1);
-        lE4 = rdgeo<FT>(p, GEO_LE, GF_LE, c4);
-        lS4 = rdgeo<FT>(p, GEO_LN, GF_LN, c4 - m.pitch);
-        lN4 = rdgeo<FT>(p, GEO_LN, GF_LN, c4);
-        dt4 = p.lts ? p.dt[c4] : bitsd(*p.dtmin_in);
+        A4 = at(p.geom + GEO_A * ncp + org, o8);
+        lW4 = geo.rdw(GEO_LE, GF_LE, og);
+        lE4 = geo.rd(GEO_LE, GF_LE, og);
+        lS4 = geo.rds(GEO_LN, GF_LN, og);
+        lN4 = geo.rd(GEO_LN, GF_LN, og);
+        dt4 = p.lts ? at(p.dt + org, o8) : bitsd(*p.dtmin_in);
         if (FUSED && !defer) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) U4[v] = p.U[v * ncp + c4];
+            for (int v = 0; v < 4; ++v) U4[v] = at(p.U + v * ncp + org, o8);
         }
         if (readS) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) S4[v] = p.S[v * ncp + c4];
+            for (int v = 0; v < 4; ++v) S4[v] = at(p.S + v * ncp + org, o8);
         }
     };
     // issued before the two barriers of the flux exchange, which they overlap
@@ -793,14 +898,13 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
     // ---- phase 4: accumulate (+W -E +S -N) and update -------------------------
     double l1 = 0.0, l2 = 0.0, mx = 0.0, dtn = MILLION;
     if (valid) {
-        const int64_t c = c4;
         const double A = A4, lW = lW4, lE = lE4, lS = lS4, lN = lN4, dtc = dt4;
         const double cdt = p.cfl * dtc;
         double dU[4];
         if (FUSED) {
             if (p.mode == MODE_FROM_S && fastS) {
 #pragma unroll
-                for (int v = 0; v < 4; ++v) dU[v] = (double)p.Sf[v * ncp + c];
+                for (int v = 0; v < 4; ++v) dU[v] = (double)at(p.Sf + v * ncp + org, e4 * 4u);
             } else if (p.mode == MODE_FROM_S) {
 #pragma unroll
                 for (int v = 0; v < 4; ++v) dU[v] = S4[v];
@@ -811,11 +915,12 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
         } else {
             if (p.mode == GINIT_KEEP) {
 #pragma unroll
-                for (int v = 0; v < 4; ++v) dU[v] = p.S[v * ncp + c];
-            } else if (p.mode == GINIT_RK4) {
+                for (int v = 0; v < 4; ++v) dU[v] = at(p.S + v * ncp + org, o8);
+            } else if (KIND == SK_GRANULAR && p.mode == GINIT_RK4) {
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    dU[v] = p.S[v * ncp + c] + 2.0 * p.S1[v * ncp + c] + 2.0 * p.S2[v * ncp + c];
+                    dU[v] = at(p.S + v * ncp + org, o8) + 2.0 * at(p.S1 + v * ncp + org, o8) +
+                            2.0 * at(p.S2 + v * ncp + org, o8);
             } else {
 #pragma unroll
                 for (int v = 0; v < 4; ++v) dU[v] = 0.0;
@@ -834,8 +939,9 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
         // axisymmetric source terms (Euler2DQuad.cc:1511-1516, 1016-1020):
         // S(W, Xc) of the cell's W^(s) and centroid radius
         double Sx[4] = {0.0, 0.0, 0.0, 0.0};
-        const bool axi = p.axisym != 0;
+        const bool axi = O::general && p.axisym != 0;
         if (axi) {
+            const int64_t c = org + e4;
             // the stage's W as the tile loaded it (the fused mixed path
             // keeps W^(s) in FP32 only)
             PS<double> Wc;
@@ -845,7 +951,7 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
             } else {
                 Wc = {p.Win[c], p.Win[ncp + c], p.Win[2 * ncp + c], p.Win[3 * ncp + c]};
             }
-            const CS<double> s = axisym_source(Wc, G[GEO_YC * ncp + c]);
+            const CS<double> s = axisym_source(Wc, p.geom[GEO_YC * ncp + c]);
             Sx[0] = s.d; Sx[1] = s.mx; Sx[2] = s.my; Sx[3] = s.E;
         }
         if constexpr (Fast<FT>::on) {
@@ -890,11 +996,14 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
                 // FAS forcing term (FASMultigrid2D.h:2736-2739, 2840-2847)
                 if (p.P) {
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) dU[v] += res ? p.P[v * ncp + c] : cdt * p.P[v * ncp + c];
+                    for (int v = 0; v < 4; ++v) {
+                        const double P = at(p.P + v * ncp + org, o8);
+                        dU[v] += res ? P : cdt * P;
+                    }
                 }
             }
         }
-        if (m.amr & AMR_FLUX_ANY) {
+        if (O::amr && (m.amr & AMR_FLUX_ANY)) {
             // block-edge fluxes FluxN/S/E/W = (+/-) Flux*lface (Euler2DQuad.cc:
             // 1518-1523, 1709-1715) for the resolution-change corrections
             double *eb = p.eflux + 4 * m.eoff;
@@ -923,9 +1032,9 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
             // granular residual, or a correction / smoothing follows: store dUdt
             double *Sx = FUSED ? p.Sd : p.S;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) Sx[v * ncp + c] = dU[v];
+            for (int v = 0; v < 4; ++v) at(Sx + v * ncp + org, o8) = dU[v];
         } else {
-            fused_update<FT>(p, m, t, c, ip, jp, A, dtc, lW, lE, lS, lN, U4, readS, S4, dU, l1, l2, mx, dtn);
+            fused_update<FT, O>(p, geo, m, t, org, o8, ip, jp, A, dtc, lW, lE, lS, lN, U4, readS, S4, dU, l1, l2, mx, dtn);
         }
     }
     if (!(FUSED) || !p.last_stage || defer) return;
@@ -954,6 +1063,11 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
         p.norm_part[2 * p.ntiles + tix] = cmx;
         p.norm_part[3 * p.ntiles + tix] = dmn;
     }
+}
+
+template <typename FT, int TI, int TJ, int KIND>
+inline void launch_stage_kernel(const StageParams *p, hipStream_t st) {
+    hipLaunchKernelGGL((stage_kernel<FT, TI, TJ, KIND>), dim3(p->ntiles), dim3((TileThreads<TI, TJ>::value)), 0, st, *p);
 }
 
 // Update of a tile from a stored residual: the second half of a fused stage
@@ -1001,10 +1115,13 @@ __global__ __launch_bounds__(UPD_NT) void update_tile_kernel(StageParams p, int 
         const double dtc = p.lts ? p.dt[c] : bitsd(*p.dtmin_in);
         double dU[4] = {p.Sd[c], p.Sd[ncp + c], p.Sd[2 * ncp + c], p.Sd[3 * ncp + c]};
         double a1 = 0.0, a2 = 0.0, a3 = 0.0, a4 = MILLION;
-        const double lW = rdgeo<FT>(p, GEO_LE, GF_LE, c - 1), lE = rdgeo<FT>(p, GEO_LE, GF_LE, c);
-        const double lS = rdgeo<FT>(p, GEO_LN, GF_LN, c - m.pitch), lN = rdgeo<FT>(p, GEO_LN, GF_LN, c);
+        const int64_t org = m.coff + (int64_t)t.j0 * m.pitch;
+        const BlockGeo<FT> geo(p, m, org);
+        const uint32_t e = (uint32_t)((jp - t.j0) * m.pitch + ip), og = e * (uint32_t)sizeof(typename CoordT<FT>::type);
+        const double lW = geo.rdw(GEO_LE, GF_LE, og), lE = geo.rd(GEO_LE, GF_LE, og);
+        const double lS = geo.rds(GEO_LN, GF_LN, og), lN = geo.rd(GEO_LN, GF_LN, og);
         const double U0[4] = {p.U[c], p.U[ncp + c], p.U[2 * ncp + c], p.U[3 * ncp + c]};
-        fused_update<FT>(p, m, t, c, ip, jp, A, dtc, lW, lE, lS, lN, U0, false, U0, dU, a1, a2, a3, a4);
+        fused_update<FT, StageOpt<SK_LEVELS>>(p, geo, m, t, org, e * 8u, ip, jp, A, dtc, lW, lE, lS, lN, U0, false, U0, dU, a1, a2, a3, a4);
         l1 += a1; l2 += a2; mx = dmax(mx, a3); dtn = dmin(dtn, a4);
     }
     if (!p.last_stage) return;
