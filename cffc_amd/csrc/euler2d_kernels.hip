@@ -874,6 +874,7 @@ hipError_t cffc_launch_stage_fp64(const StageParams *p, int ti, int tj, int fuse
     if (ti == TI && tj == TJ) {                                                                            \
         switch (kind) {                                                                                    \
         case SK_PLAIN: launch_stage_kernel<double, TI, TJ, SK_PLAIN>(p, st); break;                            \
+        case SK_WINDOW: launch_stage_kernel<double, TI, TJ, SK_WINDOW>(p, st); break;                          \
         case SK_LEVELS: launch_stage_kernel<double, TI, TJ, SK_LEVELS>(p, st); break;                          \
         case SK_MG: launch_stage_kernel<double, TI, TJ, SK_MG>(p, st); break;                              \
         case SK_MG_FIRST: launch_stage_kernel<double, TI, TJ, SK_MG_FIRST>(p, st); break;                  \

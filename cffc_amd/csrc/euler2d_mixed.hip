@@ -16,6 +16,7 @@ extern "C" hipError_t cffc_launch_stage_mixed(const StageParams *p, int ti, int 
     if (ti == TI && tj == TJ) {                                                                            \
         switch (kind) {                                                                                    \
         case SK_PLAIN: launch_stage_kernel<float, TI, TJ, SK_PLAIN>(p, st); break;                            \
+        case SK_WINDOW: launch_stage_kernel<float, TI, TJ, SK_WINDOW>(p, st); break;                          \
         case SK_LEVELS: launch_stage_kernel<float, TI, TJ, SK_LEVELS>(p, st); break;                          \
         case SK_FUSED: launch_stage_kernel<float, TI, TJ, SK_FUSED>(p, st); break;                            \
         default: launch_stage_kernel<float, TI, TJ, SK_GRANULAR>(p, st); break;                               \

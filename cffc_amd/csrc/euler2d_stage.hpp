@@ -56,6 +56,7 @@ struct StageParams {
     int32_t done_copy;      // parts that are done copy W forward (odd stage count)
     const int32_t *nbr;     // 8 same-level neighbours per block (push exchange)
     int32_t push;           // fused: also write W^(s+1) into the neighbours' ghost cells
+    int32_t window_bcs;     // fused: the tile forms the physical ghost states of its window itself
     int32_t defer_update;   // fused: store the residual only; update_tile_kernel follows
     int32_t skip_S;         // fused: no stage after this one reads S (multistage smoothing), so it is not stored
     // resolution changes
@@ -89,7 +90,7 @@ __device__ __forceinline__ void push_ghosts(const StageParams &p, ST *Wo, const 
                                             const PS<double> &Wn) {
     const int ICu = m.ni + 1, JCu = m.nj + 1;
     const bool nW = ip <= 3, nE = ip >= ICu - 1, nS = jp <= 3, nN = jp >= JCu - 1;
-    if (!(nW || nE || nS || nN)) return;
+    if (__builtin_expect(!(nW || nE || nS || nN), 1)) return;
     const int32_t *nb8 = p.nbr + 8 * b;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
@@ -228,14 +229,16 @@ enum StageKind {
     SK_GRANULAR = 0,   // dUdt_Multistage_Explicit on its own, every option
     SK_FUSED = 1,      // residual + update, every option
     SK_PLAIN = 2,      // fused: one level, planar, Venkatakrishnan
-    SK_LEVELS = 3,     // the same with resolution changes
-    SK_MG = 4,         // granular: one level, planar, Venkatakrishnan, Roe
-    SK_MG_FIRST = 5    // granular multigrid stage of a first-order level: zero limiter, so no reconstruction
+    SK_WINDOW = 3,     // the same, physical ghosts formed in the tile's window
+    SK_LEVELS = 4,     // SK_PLAIN with resolution changes
+    SK_MG = 5,         // granular: one level, planar, Venkatakrishnan, Roe
+    SK_MG_FIRST = 6    // granular multigrid stage of a first-order level: zero limiter, so no reconstruction
 };
 template <int K> struct StageOpt {
-    static constexpr bool fused = K == SK_FUSED || K == SK_PLAIN || K == SK_LEVELS;
+    static constexpr bool fused = K == SK_FUSED || K == SK_PLAIN || K == SK_WINDOW || K == SK_LEVELS;
     static constexpr bool general = K == SK_GRANULAR || K == SK_FUSED;   // axisymmetric, any limiter
     static constexpr bool amr = general || K == SK_LEVELS;
+    static constexpr bool window = K == SK_FUSED || K == SK_WINDOW;
     static constexpr bool first = K == SK_MG_FIRST;
 };
 // the leanest kernel that has every option of the launch
@@ -243,7 +246,7 @@ inline int stage_kind(const StageParams &p, int fused) {
     const bool venkat = p.limiter == 9;
     if (fused) {
         if (p.axisym || !venkat || p.defer_update) return SK_FUSED;
-        return p.eflux || p.tile_defer || p.Ustage ? SK_LEVELS : SK_PLAIN;
+        return p.eflux || p.tile_defer || p.Ustage ? SK_LEVELS : p.window_bcs ? SK_WINDOW : SK_PLAIN;
     }
     if (p.axisym || p.eflux || p.mode == GINIT_RK4) return SK_GRANULAR;
     if (p.hlle) return p.limiter == 0 && p.phi_mode != PHI_LOAD ? SK_MG_FIRST : SK_GRANULAR;
@@ -412,7 +415,7 @@ __device__ __forceinline__ void fused_update(const StageParams &p, const BlockGe
     Un.d = U0[0] + om * dU[0]; Un.mx = U0[1] + om * dU[1];
     Un.my = U0[2] + om * dU[2]; Un.E = U0[3] + om * dU[3];
     bool bad = positivity_fails<FT>(Un);
-    if (bad && p.lts) {
+    if (__builtin_expect(bad && p.lts, 0)) {
         // scalar local time stepping: halve dt and dUdt up to 10 times
         double f = 1.0, dtl = dtc;
         for (int n = 1; n <= 10; ++n) {
@@ -427,7 +430,7 @@ __device__ __forceinline__ void fused_update(const StageParams &p, const BlockGe
         at(dtb, o8) = dtl;
         bad = positivity_fails<FT>(Un);
     }
-    if (bad) {
+    if (__builtin_expect(bad, 0)) {
         const unsigned long long key =
             ((unsigned long long)t.b << 32) | ((unsigned long long)jp << 16) | (unsigned long long)ip;
         atomicMin(p.err, key);
@@ -503,6 +506,88 @@ __device__ __forceinline__ void fused_update(const StageParams &p, const BlockGe
     }
 }
 
+// Physical ghost states of a tile's window (BCs, Euler2DQuadSingleBlock.cc:
+// 2354-3010), formed in LDS from the window's own cells: both ghost layers
+// copy, mirror or replace the two cells next to the boundary, which a window
+// that holds them always contains (not so for periodic boundaries: the host
+// keeps the exchange kernel for those).  In the exchange kernel's order: the
+// west and east columns (corner rows only where the south or north boundary
+// of the ghost column is none), a barrier, then the south and north rows over
+// all columns.  States are formed in FP64 and stored as FT, as the exchange
+// kernel stores them.  This saves the launch that filled the same ghosts in
+// HBM before every stage (4.7 us of a 23 us stage at 65 k cells).
+// il, jl: window coordinates; cell (ip, jp) = (pi0 + il, pj0 + jl).
+template <typename FT, int LJ, int LI>
+__device__ __forceinline__ void window_ghosts(const StageParams &p, const BlockMeta &m, int pi0, int pj0, int tid,
+                                              int nt, FT (&sW)[4][LJ][LI]) {
+    const int ICu = m.ni + 1, JCu = m.nj + 1;
+    const bool tw = pi0 == 0, te = pi0 + LI > ICu + 1, ts = pj0 == 0, tn = pj0 + LJ > JCu + 1;
+    if (__builtin_expect(!(tw || te || ts || tn), 1)) return;   // uniform over the workgroup
+    const int32_t *bcW = p.bc + m.bcoff, *bcE = bcW + m.ncj, *bcS = bcE + m.ncj, *bcN = bcS + m.nci;
+    const double *woW = p.wo + 4 * (int64_t)m.bcoff;
+    auto ld = [&](int jl, int il) -> PS<double> {
+        return {(double)sW[0][jl][il], (double)sW[1][jl][il], (double)sW[2][jl][il], (double)sW[3][jl][il]};
+    };
+    auto st = [&](int jl, int il, const PS<double> &w) {
+        if (il < 0 || il >= LI || jl < 0 || jl >= LJ) return;
+        sW[0][jl][il] = (FT)w.d; sW[1][jl][il] = (FT)w.vx; sW[2][jl][il] = (FT)w.vy; sW[3][jl][il] = (FT)w.p;
+    };
+    // ghosts (jl, il) + (dj, di) and + 2 (dj, di) of the boundary cell (jl, il);
+    // cf: the cell whose E (or N) face is the boundary, sgn its outward sign
+    auto fill = [&](int bcv, int slot, int64_t cf, int gx, int gy, double sgn, int jl, int il, int dj, int di) {
+        if (bcv == 11000 || bcv == 8001) {
+            const double *a = woW + 4 * slot;
+            const PS<double> w0 = {a[0], a[1], a[2], a[3]};
+            if (bcv == 11000) {
+                st(jl + dj, il + di, w0);
+                st(jl + 2 * dj, il + 2 * di, w0);
+                return;
+            }
+            const double nx = sgn * p.geom[gx * p.ncp + cf], ny = sgn * p.geom[gy * p.ncp + cf];
+            const PS<double> g = bc_characteristic_pressure(ld(jl, il), w0, nx, ny);
+            st(jl + dj, il + di, g);
+            st(jl + 2 * dj, il + 2 * di, g);
+        } else if (bcv == 7001) {
+            const double nx = sgn * p.geom[gx * p.ncp + cf], ny = sgn * p.geom[gy * p.ncp + cf];
+            const PS<double> w1 = ld(jl, il), w2 = ld(jl - dj, il - di);
+            st(jl + dj, il + di, reflect(w1, nx, ny));
+            st(jl + 2 * dj, il + 2 * di, reflect(w2, nx, ny));
+        } else {   // constant extrapolation (and the reference's default)
+            const PS<double> w1 = ld(jl, il);
+            st(jl + dj, il + di, w1);
+            st(jl + 2 * dj, il + 2 * di, w1);
+        }
+    };
+    __syncthreads();
+    if (tw || te) {
+        for (int q = tid; q < 2 * LJ; q += nt) {
+            const int jl = q >> 1, j = pj0 + jl;
+            const bool west = (q & 1) == 0;
+            if (j >= m.ncj || !(west ? tw : te)) continue;
+            const int bcv = west ? bcW[j] : bcE[j];
+            if (bcv == 0) continue;
+            const int in = west ? 2 : ICu, icol = west ? 1 : ICu + 1;
+            if ((j < 2 && bcS[icol] != 0) || (j > JCu && bcN[icol] != 0)) continue;
+            const int64_t cf = m.coff + (int64_t)j * m.pitch + (west ? 1 : ICu);
+            fill(bcv, west ? j : m.ncj + j, cf, GEO_NEX, GEO_NEY, west ? -1.0 : 1.0, jl, in - pi0, 0, west ? -1 : 1);
+        }
+        __syncthreads();
+    }
+    if (ts || tn) {
+        for (int q = tid; q < 2 * LI; q += nt) {
+            const int il = q >> 1, i = pi0 + il;
+            const bool south = (q & 1) == 0;
+            if (i >= m.nci || !(south ? ts : tn)) continue;
+            const int bcv = south ? bcS[i] : bcN[i];
+            if (bcv == 0) continue;
+            const int in = south ? 2 : JCu;
+            const int64_t cf = m.coff + (int64_t)(south ? 1 : JCu) * m.pitch + i;
+            fill(bcv, 2 * m.ncj + (south ? i : m.nci + i), cf, GEO_NNX, GEO_NNY, south ? -1.0 : 1.0, in - pj0, il,
+                 south ? -1 : 1, 0);
+        }
+    }
+}
+
 // Threads per workgroup for a TI x TJ tile: one per tile cell plus one per
 // halo ("ring") cell whose reconstruction the tile's boundary faces need,
 // rounded up to whole wavefronts.  For 16 x 16: 256 + 64 = 320 (5 waves),
@@ -565,7 +650,7 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
         // batched steady run: a converged part is left alone, a frozen part
         // loads its limiters, a running part stores them at its last stage
         const int ps = p.part_state[t.part];
-        if (ps == PART_DONE) {
+        if (__builtin_expect(ps == PART_DONE, 0)) {
             if (p.done_copy) {
                 for (int q = tid; q < TI * TJ; q += NT) {
                     const int ip = t.i0 + 2 + q % TI, jp = t.j0 + 2 + q / TI;
@@ -664,6 +749,7 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
             }
         }
     }
+    if (O::window && p.window_bcs && m.has_bc) window_ghosts<FT, LJ, LI>(p, m, pi0, pj0, tid, NT, sW);
     __syncthreads();
 
     // ---- phase 2: least-squares reconstruction + limiter -------------------
@@ -699,7 +785,7 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
                 mask = stencil_mask(ip, jp, ICu, JCu, bcW[jp], bcE[jp], bcS[ip], bcN[ip]);
             PS<FT> gx, gy, ph;
             if constexpr (O::first) ph = {FT(0), FT(0), FT(0), FT(0)};
-            else if (mask == 0xFFu)
+            else if (__builtin_expect(mask == 0xFFu, 1))
                 reconstruct<FT, O, true>(p, geo, phib, phim, e * XS, e * 8u, il, jl, 0xFFu, sW, sX, sY, gx, gy, ph);
             else reconstruct<FT, O, false>(p, geo, phib, phim, e * XS, e * 8u, il, jl, mask, sW, sX, sY, gx, gy, ph);
             if (phim == PHI_COMPUTE_STORE) {
