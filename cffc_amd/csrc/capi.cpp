@@ -996,18 +996,33 @@ extern "C" int cffc_create(const cffc_mesh_desc *md, const cffc_scheme_desc *sd,
             return e;
         }
     }
-    // default tile: for blocks at least 32 cells wide the autotuner's picks
-    // on the 16.8 M-cell and uneven quadtree workloads, 32 x 16 (FP64) and
-    // 32 x 8 (mixed), both ring-pass tiles; 16 x 8 for blocks 16 to 31
-    // cells wide (192 threads, three wavefronts); 8 x 8 for blocks narrower
-    // than 16 cells; in FP64, 4 x 4 (one wavefront per block) for blocks
-    // narrower than 8 cells
+    // Default tile.  A launch with fewer 16 x 8 tiles than compute units is
+    // latency-bound and takes 8 x 8 tiles; up to 1,280 of them (five
+    // resident workgroups on each of 256 units, 164 k cells) 16 x 8 spreads the
+    // work best; beyond, blocks at least 32 cells wide take the larger ring-pass
+    // tiles, which recompute fewer ring cells: 32 x 16 (FP64; mixed up to 1.5 M
+    // cells), 32 x 8 (mixed).  Narrower blocks stay with 16 x 8, in FP64 except
+    // for the stretch in which it has just begun a second round and 16 x 16 (four
+    // resident of half as many tiles) still fits one: 197 k cells of 16^2 blocks,
+    // five stages, 16x16 0.179 ms, 16x8 0.204.  Per RK4 step in blocks of 64^2, FP64: 16 k cells
+    // 8x8 0.071, 16x8 0.071, 32x16 0.094 ms; 66 k 16x8 0.078, 8x8 0.084, 32x16
+    // 0.095; 147 k 0.119 / 32x16 0.129; 262 k 32x16 0.140 / 16x8 0.163; 2.2 M
+    // 0.885 / 0.961.  Blocks of 16^2: 16 k cells 8x8 0.071, 16x8 0.075; 66 k
+    // 0.087 / 0.085.  Mixed, 64^2: 66 k 16x8 0.064, 32x8 0.068; 262 k 32x16
+    // 0.094, 32x8 0.100, 16x8 0.104; 2.2 M 32x8 0.506, 32x16 0.510.
+    // 8 x 8 for blocks narrower than 16 cells; in FP64, 4 x 4 (one wavefront
+    // per block) for blocks narrower than 8 cells.
     const bool fp64 = c->s.flux_precision == CFFC_FLUX_FP64;
     int ti = 16, tj = 8;
     int mini = 1 << 30;
-    for (auto &m : c->meta_h) mini = std::min(mini, m.ni);
-    if (mini >= 32) { ti = 32; tj = fp64 ? 16 : 8; }
-    if (mini < 16) ti = tj = 8;
+    int64_t n168 = 0;
+    for (auto &m : c->meta_h) {
+        mini = std::min(mini, m.ni);
+        n168 += (int64_t)((m.ni + 15) / 16) * ((m.nj + 7) / 8);
+    }
+    if (mini >= 32 && n168 > 1280) { ti = 32; tj = fp64 || c->ncell < 1500000 ? 16 : 8; }
+    else if (fp64 && n168 > 1280 && n168 <= 1700) tj = 16;
+    if (mini < 16 || n168 < 256) ti = tj = 8;
     if (mini < 8 && fp64) ti = tj = 4;
     if ((e = build_tiles(c, ti, tj))) {
         free_ctx(c);
