@@ -19,33 +19,9 @@
 #include "../../include/cffc_euler2d.h"
 #include "../../include/cffc_unet.h"
 
-typedef uint16_t bf16_t;
+#include "unet_kernels.hpp"
 
-extern "C" {
-hipError_t cffc_unet_launch_mfma_layout(float *out, hipStream_t st);
-hipError_t cffc_unet_launch_conv_fwd(const bf16_t *xA, int CA, const bf16_t *xB, int CB, int B, int H, int W,
-                                     const bf16_t *wt, int Kpad, const float *bias, int Cout, int relu, bf16_t *y,
-                                     float *y32, hipStream_t st);
-hipError_t cffc_unet_launch_conv_bwd_data(const float *dy, const bf16_t *yact, int Cout, int relu, int B, int H,
-                                          int W, const bf16_t *wd, int Kpad2, int CA, int CB, float *dxA, int accA,
-                                          float *dxB, int accB, hipStream_t st);
-hipError_t cffc_unet_launch_conv_bwd_weight(const float *dy, const bf16_t *yact, int Cout, int relu, const bf16_t *xA,
-                                            int CA, const bf16_t *xB, int CB, int B, int H, int W, float *dw,
-                                            float *db, hipStream_t st);
-hipError_t cffc_unet_launch_avgpool_fwd(const bf16_t *x, int B, int H, int W, int C, bf16_t *y, hipStream_t st);
-hipError_t cffc_unet_launch_avgpool_bwd(const float *dy, int B, int H, int W, int C, float *dx, hipStream_t st);
-hipError_t cffc_unet_launch_upsample_fwd(const bf16_t *x, int B, int H, int W, int C, bf16_t *y, hipStream_t st);
-hipError_t cffc_unet_launch_upsample_bwd(const float *dy, int B, int H, int W, int C, float *dx, hipStream_t st);
-hipError_t cffc_unet_launch_mse(const float *y32, int Cout, int nout, const float *t, int64_t P, float *dy,
-                                float *loss, hipStream_t st);
-hipError_t cffc_unet_launch_adam(float *w, const float *g, float *m, float *v, int Cout, int Cin, int Kpad, int Kpad2,
-                                 bf16_t *wt, bf16_t *wd, float lr, float b1, float b2, float eps, float c1, float c2,
-                                 int update, float *b, const float *gb, float *mb, float *vb, hipStream_t st);
-hipError_t cffc_unet_launch_gather_bf16(const bf16_t *src, const int32_t *idx, int nrows, int64_t row_elems,
-                                        bf16_t *dst, hipStream_t st);
-hipError_t cffc_unet_launch_gather_f32(const float *src, const int32_t *idx, int nrows, int64_t row_elems, float *dst,
-                                       hipStream_t st);
-}
+using namespace unetk;
 
 static thread_local std::string u_err;
 static int ufail(int code, const char *fmt, ...) {
@@ -64,43 +40,37 @@ static int ufail(int code, const char *fmt, ...) {
         if (e_ != hipSuccess) return ufail(CFFC_E_HIP, "%s: %s", #x, hipGetErrorString(e_));      \
     } while (0)
 
-static inline bf16_t host_f2bf(float f) {
-    uint32_t u;
-    memcpy(&u, &f, 4);
-    if ((u & 0x7F800000u) == 0x7F800000u) return (bf16_t)(u >> 16);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (bf16_t)(u >> 16);
-}
-
+// Activations, and the masked BF16 gradient of a convolution's output; gskip:
+// the FP32 gradient a skip connection brings to it.
 struct Tensor {
     int C, level;
-    bf16_t *act = nullptr;
-    float *grad = nullptr;
+    int producer = -1;   // conv that writes it
+    bf16_t *act = nullptr, *G = nullptr;
+    float *gskip = nullptr;
 };
 
 struct Conv {
-    int inA, inB, out;  // tensor ids (inB = -1: none)
+    int inA, inB, out;   // tensor ids (inB = -1: none); inA is read through the upsampling if upA
+    int upA;
+    int pool = -1;       // pooled copy of the output, or -1
     int CA, CB, Cout, level, relu;
+    int kind = -1, target = -1;   // where the input's gradient goes (BwdKind, tensor); -1: not needed
     int K, Kpad, Kpad2;
     float *w = nullptr, *b = nullptr, *m = nullptr, *v = nullptr, *mb = nullptr, *vb = nullptr;
     float *gw = nullptr, *gb = nullptr;
     bf16_t *wt = nullptr, *wd = nullptr;
+    float *part = nullptr, *dbp = nullptr;   // weight-gradient and bias-gradient partials
 };
 
-enum OpKind { OP_CONV, OP_POOL, OP_UP };
-struct Op {
-    OpKind kind;
-    int a, b;  // conv: layer index; pool/up: src tensor, dst tensor
-};
+constexpr int MSE_WG = 256;   // workgroups of the loss kernel
 
 struct cffc_unet {
     int H = 0, W = 0, maxB = 0;
     hipStream_t stream = nullptr;
     std::vector<Tensor> t;
     std::vector<Conv> L;
-    std::vector<Op> ops;
     int x0 = -1, yout = -1;
-    float *y32 = nullptr, *target = nullptr, *loss = nullptr;
+    float *y4 = nullptr, *target = nullptr, *loss = nullptr, *lossp = nullptr, *x32 = nullptr;
     int32_t *idx = nullptr;
     bf16_t *ds_in = nullptr;
     float *ds_tg = nullptr;
@@ -126,33 +96,39 @@ static int add_tensor(cffc_unet *n, int C, int level) {
     return (int)n->t.size() - 1;
 }
 
-static int add_conv(cffc_unet *n, int inA, int inB, int Cout, int relu) {
+static int add_conv(cffc_unet *n, int inA, int upA, int inB, int Cout, int relu) {
     Conv c;
     c.inA = inA;
+    c.upA = upA;
     c.inB = inB;
     c.CA = n->t[inA].C;
     c.CB = inB >= 0 ? n->t[inB].C : 0;
     c.Cout = Cout;
-    c.level = n->t[inA].level;
+    c.level = n->t[inA].level - upA;
     c.relu = relu;
     c.out = add_tensor(n, Cout, c.level);
+    n->t[c.out].producer = (int)n->L.size();
     c.K = 9 * (c.CA + c.CB);
     c.Kpad = (c.K + 31) / 32 * 32;
     c.Kpad2 = (9 * Cout + 31) / 32 * 32;
+    if (inA != n->x0) {
+        // the input's gradient: to the tensor, to the low-resolution tensor, or
+        // (a pooled input, which has no producer) to the tensor it was pooled from
+        c.kind = upA ? BWD_UP : BWD_SAME;
+        c.target = inA;
+        if (n->t[inA].producer < 0) {
+            c.kind = BWD_POOL;
+            for (const Conv &q : n->L)
+                if (q.pool == inA) c.target = q.out;
+        }
+    }
     n->L.push_back(c);
-    n->ops.push_back(Op{OP_CONV, (int)n->L.size() - 1, 0});
     return c.out;
 }
 
 static int add_pool(cffc_unet *n, int src) {
     const int dst = add_tensor(n, n->t[src].C, n->t[src].level + 1);
-    n->ops.push_back(Op{OP_POOL, src, dst});
-    return dst;
-}
-
-static int add_up(cffc_unet *n, int src) {
-    const int dst = add_tensor(n, n->t[src].C, n->t[src].level - 1);
-    n->ops.push_back(Op{OP_UP, src, dst});
+    n->L[n->t[src].producer].pool = dst;
     return dst;
 }
 
@@ -162,24 +138,33 @@ static void build_graph(cffc_unet *n) {
     int cur = n->x0;
     int skip[3];
     for (int l = 0; l < 4; ++l) {
-        cur = add_conv(n, cur, -1, ch[l], 1);
-        cur = add_conv(n, cur, -1, ch[l], 1);
+        cur = add_conv(n, cur, 0, -1, ch[l], 1);
+        cur = add_conv(n, cur, 0, -1, ch[l], 1);
         if (l < 3) {
             skip[l] = cur;
             cur = add_pool(n, cur);
         }
     }
     for (int l = 2; l >= 0; --l) {
-        cur = add_up(n, cur);
-        cur = add_conv(n, cur, skip[l], ch[l], 1);
-        cur = add_conv(n, cur, -1, ch[l], 1);
+        cur = add_conv(n, cur, 1, skip[l], ch[l], 1);
+        cur = add_conv(n, cur, 0, -1, ch[l], 1);
     }
-    n->yout = add_conv(n, cur, -1, 16, 0);
+    n->yout = add_conv(n, cur, 0, -1, 16, 0);
 }
 
-static int upload_weights_bf16(cffc_unet *n, Conv &c) {
-    UCHK(cffc_unet_launch_adam(c.w, c.gw, c.m, c.v, c.Cout, c.CA + c.CB, c.Kpad, c.Kpad2, c.wt, c.wd, 0.f, 0.f, 0.f,
-                               0.f, 1.f, 1.f, 0, c.b, c.gb, c.mb, c.vb, n->stream));
+// Adam on every layer, or (update 0) only the packed BF16 copies of layer
+// first .. last
+static int run_adam(cffc_unet *n, int first, int last, int update, float lr, float b1, float b2, float eps, float c1,
+                    float c2) {
+    AdamList A = {};
+    int wg = 0;
+    for (int l = first; l <= last; ++l) {
+        const Conv &c = n->L[l];
+        AdamLayer &a = A.l[A.count++];
+        a = {c.w, c.gw, c.m, c.v, c.b, c.gb, c.mb, c.vb, c.wt, c.wd, c.Cout, c.CA + c.CB, wg};
+        wg += (c.Cout * c.K + c.Cout + 255) / 256;
+    }
+    UCHK(cffc_unet_launch_adam(&A, wg, lr, b1, b2, eps, c1, c2, update, n->stream));
     return 0;
 }
 
@@ -207,11 +192,33 @@ extern "C" int cffc_unet_create(int H, int W, int max_batch, uint64_t seed, cffc
     int e = 0;
     for (auto &x : n->t) {
         const size_t np = (size_t)npix(n, x.level, max_batch) * x.C;
-        if ((e = ualloc(n, (void **)&x.act, np * sizeof(bf16_t))) || (e = ualloc(n, (void **)&x.grad, np * sizeof(float)))) {
+        if ((e = ualloc(n, (void **)&x.act, np * sizeof(bf16_t))) ||
+            (x.producer >= 0 && (e = ualloc(n, (void **)&x.G, np * sizeof(bf16_t))))) {
             cffc_unet_destroy(n);
             return e;
         }
     }
+    for (auto &c : n->L) {
+        if (c.inB < 0) continue;
+        Tensor &x = n->t[c.inB];
+        if ((e = ualloc(n, (void **)&x.gskip, (size_t)npix(n, x.level, max_batch) * x.C * sizeof(float)))) {
+            cffc_unet_destroy(n);
+            return e;
+        }
+    }
+    // rows of the bias-gradient partials of every convolution, written by the
+    // kernel that forms its output's gradient, for the largest batch and any
+    // smaller one (a smaller batch may take smaller tiles)
+    std::vector<size_t> dbrows(n->L.size(), MSE_WG), parts(n->L.size(), 0);
+    for (const Conv &c : n->L)
+        for (int B = 1; B <= max_batch; ++B) {
+            const int ch = H >> c.level, cw = W >> c.level, Cin = c.CA + c.CB;
+            size_t &p = parts[&c - n->L.data()];
+            p = std::max(p, (size_t)cffc_unet_wgrad_chunks(B, ch, cw, Cin, c.Cout));
+            if (c.target < 0) continue;
+            size_t &r = dbrows[n->t[c.target].producer];
+            r = std::max(r, (size_t)cffc_unet_conv_tiles(B, ch, cw, Cin));
+        }
     std::mt19937_64 rng(seed);
     for (size_t li = 0; li < n->L.size(); ++li) {
         Conv &c = n->L[li];
@@ -222,7 +229,9 @@ extern "C" int cffc_unet_create(int H, int W, int max_batch, uint64_t seed, cffc
             (e = ualloc(n, (void **)&c.b, c.Cout * 4)) || (e = ualloc(n, (void **)&c.mb, c.Cout * 4)) ||
             (e = ualloc(n, (void **)&c.vb, c.Cout * 4)) || (e = ualloc(n, (void **)&c.gb, c.Cout * 4)) ||
             (e = ualloc(n, (void **)&c.wt, (size_t)c.Cout * c.Kpad * 2)) ||
-            (e = ualloc(n, (void **)&c.wd, (size_t)Cin * c.Kpad2 * 2))) {
+            (e = ualloc(n, (void **)&c.wd, (size_t)((Cin + 15) / 16 * 16) * c.Kpad2 * 2)) ||
+            (e = ualloc(n, (void **)&c.part, parts[li] * nw * 4)) ||
+            (e = ualloc(n, (void **)&c.dbp, dbrows[li] * c.Cout * 4))) {
             cffc_unet_destroy(n);
             return e;
         }
@@ -233,14 +242,16 @@ extern "C" int cffc_unet_create(int H, int W, int max_batch, uint64_t seed, cffc
         std::normal_distribution<double> nd(0.0, sd);
         for (auto &x : hw) x = (float)nd(rng);
         UCHK(hipMemcpy(c.w, hw.data(), nw * 4, hipMemcpyHostToDevice));
-        if ((e = upload_weights_bf16(n, c))) {
-            cffc_unet_destroy(n);
-            return e;
-        }
+    }
+    if ((e = run_adam(n, 0, (int)n->L.size() - 1, 0, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f))) {
+        cffc_unet_destroy(n);
+        return e;
     }
     const size_t np0 = (size_t)npix(n, 0, max_batch);
-    if ((e = ualloc(n, (void **)&n->y32, np0 * 16 * 4)) || (e = ualloc(n, (void **)&n->target, np0 * CFFC_UNET_OUT * 4)) ||
-        (e = ualloc(n, (void **)&n->loss, 4)) || (e = ualloc(n, (void **)&n->idx, max_batch * 4))) {
+    if ((e = ualloc(n, (void **)&n->y4, np0 * CFFC_UNET_OUT * 4)) ||
+        (e = ualloc(n, (void **)&n->target, np0 * CFFC_UNET_OUT * 4)) ||
+        (e = ualloc(n, (void **)&n->x32, np0 * CFFC_UNET_IN * 4)) || (e = ualloc(n, (void **)&n->loss, 4)) ||
+        (e = ualloc(n, (void **)&n->lossp, MSE_WG * 4)) || (e = ualloc(n, (void **)&n->idx, max_batch * 4))) {
         cffc_unet_destroy(n);
         return e;
     }
@@ -271,7 +282,7 @@ extern "C" int cffc_unet_set_weights(cffc_unet *n, int l, const float *w, const 
     Conv &c = n->L[l];
     if (w) UCHK(hipMemcpy(c.w, w, (size_t)c.Cout * c.K * 4, hipMemcpyHostToDevice));
     if (b) UCHK(hipMemcpy(c.b, b, (size_t)c.Cout * 4, hipMemcpyHostToDevice));
-    if (int e = upload_weights_bf16(n, c)) return e;
+    if (int e = run_adam(n, l, l, 0, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f)) return e;
     UCHK(hipStreamSynchronize(n->stream));
     return 0;
 }
@@ -279,8 +290,6 @@ extern "C" int cffc_unet_set_weights(cffc_unet *n, int l, const float *w, const 
 extern "C" int cffc_unet_set_dataset(cffc_unet *n, int ns, const float *inputs, const float *targets) {
     if (!n || ns <= 0 || !inputs || !targets) return ufail(CFFC_E_ARG, "bad dataset");
     const size_t per_in = (size_t)n->H * n->W * CFFC_UNET_IN, per_tg = (size_t)n->H * n->W * CFFC_UNET_OUT;
-    std::vector<bf16_t> hin(per_in * ns);
-    for (size_t q = 0; q < hin.size(); ++q) hin[q] = host_f2bf(inputs[q]);
     if (n->ds_in) {
         (void)hipFree(n->ds_in);
         (void)hipFree(n->ds_tg);
@@ -288,57 +297,61 @@ extern "C" int cffc_unet_set_dataset(cffc_unet *n, int ns, const float *inputs, 
         n->allocs.erase(std::remove(n->allocs.begin(), n->allocs.end(), (void *)n->ds_tg), n->allocs.end());
     }
     int e;
-    if ((e = ualloc(n, (void **)&n->ds_in, hin.size() * 2)) || (e = ualloc(n, (void **)&n->ds_tg, per_tg * ns * 4))) return e;
-    UCHK(hipMemcpy(n->ds_in, hin.data(), hin.size() * 2, hipMemcpyHostToDevice));
-    UCHK(hipMemcpy(n->ds_tg, targets, per_tg * ns * 4, hipMemcpyHostToDevice));
+    if ((e = ualloc(n, (void **)&n->ds_in, per_in * ns * 2)) || (e = ualloc(n, (void **)&n->ds_tg, per_tg * ns * 4))) return e;
+    // rounded to BF16 on the device, max_batch samples at a time
+    for (int s = 0; s < ns; s += n->maxB) {
+        const size_t k = per_in * std::min(n->maxB, ns - s);
+        UCHK(hipMemcpyAsync(n->x32, inputs + per_in * s, k * 4, hipMemcpyHostToDevice, n->stream));
+        UCHK(cffc_unet_launch_to_bf16(n->x32, n->ds_in + per_in * s, (int64_t)k, n->stream));
+    }
+    UCHK(hipMemcpyAsync(n->ds_tg, targets, per_tg * ns * 4, hipMemcpyHostToDevice, n->stream));
+    UCHK(hipStreamSynchronize(n->stream));
     n->ds_n = ns;
     return 0;
 }
 
 static int forward(cffc_unet *n, int B) {
-    for (const Op &op : n->ops) {
-        if (op.kind == OP_CONV) {
-            Conv &c = n->L[op.a];
-            const int H = n->H >> c.level, W = n->W >> c.level;
-            const bf16_t *xb = c.inB >= 0 ? n->t[c.inB].act : nullptr;
-            UCHK(cffc_unet_launch_conv_fwd(n->t[c.inA].act, c.CA, xb, c.CB, B, H, W, c.wt, c.Kpad, c.b, c.Cout, c.relu,
-                                           n->t[c.out].act, c.out == n->yout ? n->y32 : nullptr, n->stream));
-        } else if (op.kind == OP_POOL) {
-            const Tensor &s = n->t[op.a];
-            UCHK(cffc_unet_launch_avgpool_fwd(s.act, B, n->H >> s.level, n->W >> s.level, s.C, n->t[op.b].act, n->stream));
-        } else {
-            const Tensor &s = n->t[op.a];
-            UCHK(cffc_unet_launch_upsample_fwd(s.act, B, n->H >> s.level, n->W >> s.level, s.C, n->t[op.b].act, n->stream));
-        }
+    for (const Conv &c : n->L) {
+        const int H = n->H >> c.level, W = n->W >> c.level;
+        UCHK(cffc_unet_launch_conv_fwd(n->t[c.inA].act, c.CA, c.upA, c.inB >= 0 ? n->t[c.inB].act : nullptr, c.CB, B, H,
+                                       W, c.wt, c.b, c.Cout, c.relu, n->t[c.out].act,
+                                       c.out == n->yout ? n->y4 : nullptr,
+                                       c.pool >= 0 ? n->t[c.pool].act : nullptr, n->stream));
     }
     return 0;
 }
 
+// Weight and input gradients from the last convolution to the first, then the
+// sums of all partials.  A skip tensor's gradient comes first through its
+// decoder (gskip), then through the pooling, where the two are added.
 static int backward(cffc_unet *n, int B) {
-    for (int q = (int)n->ops.size() - 1; q >= 0; --q) {
-        const Op &op = n->ops[q];
-        if (op.kind == OP_CONV) {
-            Conv &c = n->L[op.a];
-            const int H = n->H >> c.level, W = n->W >> c.level;
-            const bf16_t *xb = c.inB >= 0 ? n->t[c.inB].act : nullptr;
-            const Tensor &o = n->t[c.out];
-            UCHK(cffc_unet_launch_conv_bwd_weight(o.grad, o.act, c.Cout, c.relu, n->t[c.inA].act, c.CA, xb, c.CB, B, H, W,
-                                                  c.gw, c.gb, n->stream));
-            if (c.inA != n->x0) {
-                float *dxb = c.inB >= 0 ? n->t[c.inB].grad : nullptr;
-                UCHK(cffc_unet_launch_conv_bwd_data(o.grad, o.act, c.Cout, c.relu, B, H, W, c.wd, c.Kpad2, c.CA, c.CB,
-                                                    n->t[c.inA].grad, 0, dxb, 0, n->stream));
-            }
-        } else if (op.kind == OP_POOL) {
-            // the pooled tensor's source also feeds a skip connection whose
-            // gradient the decoder wrote first: accumulate
-            const Tensor &s = n->t[op.a];
-            UCHK(cffc_unet_launch_avgpool_bwd(n->t[op.b].grad, B, n->H >> s.level, n->W >> s.level, s.C, s.grad, n->stream));
-        } else {
-            const Tensor &s = n->t[op.a];
-            UCHK(cffc_unet_launch_upsample_bwd(n->t[op.b].grad, B, n->H >> s.level, n->W >> s.level, s.C, s.grad, n->stream));
-        }
+    SumList S = {};
+    auto sum = [&](const float *part, float *out, int len, int chunks) {
+        S.part[S.count] = part;
+        S.out[S.count] = out;
+        S.n[S.count] = len;
+        S.chunks[S.count] = chunks;
+        S.first[S.count + 1] = S.first[S.count] + (len + 31) / 32;
+        S.count++;
+    };
+    sum(n->lossp, n->loss, 1, MSE_WG);
+    sum(n->L.back().dbp, n->L.back().gb, n->L.back().Cout, MSE_WG);
+    for (int q = (int)n->L.size() - 1; q >= 0; --q) {
+        const Conv &c = n->L[q];
+        const int H = n->H >> c.level, W = n->W >> c.level, Cin = c.CA + c.CB;
+        const bf16_t *G = n->t[c.out].G;
+        UCHK(cffc_unet_launch_conv_bwd_weight(G, c.Cout, n->t[c.inA].act, c.CA, c.upA,
+                                              c.inB >= 0 ? n->t[c.inB].act : nullptr, c.CB, B, H, W, c.part,
+                                              n->stream));
+        sum(c.part, c.gw, c.Cout * c.K, cffc_unet_wgrad_chunks(B, H, W, Cin, c.Cout));
+        if (c.target < 0) continue;
+        const Tensor &t = n->t[c.target];
+        const Conv &pr = n->L[t.producer];
+        UCHK(cffc_unet_launch_conv_bwd_data(G, c.Cout, B, H, W, c.wd, Cin, c.CA, c.kind, t.act, t.G, pr.dbp,
+                                            c.inB >= 0 ? n->t[c.inB].gskip : nullptr, t.gskip, n->stream));
+        sum(pr.dbp, pr.gb, pr.Cout, cffc_unet_conv_tiles(B, H, W, Cin));
     }
+    UCHK(cffc_unet_launch_reduce(&S, n->stream));
     return 0;
 }
 
@@ -348,15 +361,14 @@ static int load_batch(cffc_unet *n, const int32_t *idx, int B) {
         if (idx[i] < 0 || idx[i] >= n->ds_n) return ufail(CFFC_E_ARG, "sample index out of range");
     UCHK(hipMemcpyAsync(n->idx, idx, B * 4, hipMemcpyHostToDevice, n->stream));
     const int64_t px = (int64_t)n->H * n->W;
-    UCHK(cffc_unet_launch_gather_bf16(n->ds_in, n->idx, B, px * CFFC_UNET_IN, n->t[n->x0].act, n->stream));
-    UCHK(cffc_unet_launch_gather_f32(n->ds_tg, n->idx, B, px * CFFC_UNET_OUT, n->target, n->stream));
+    UCHK(cffc_unet_launch_gather(n->ds_in, n->idx, B, px * CFFC_UNET_IN * 2, n->t[n->x0].act, n->stream));
+    UCHK(cffc_unet_launch_gather(n->ds_tg, n->idx, B, px * CFFC_UNET_OUT * 4, n->target, n->stream));
     return 0;
 }
 
 static int loss_and_grad(cffc_unet *n, int B, float *loss) {
-    UCHK(hipMemsetAsync(n->loss, 0, 4, n->stream));
-    UCHK(cffc_unet_launch_mse(n->y32, 16, CFFC_UNET_OUT, n->target, (int64_t)npix(n, 0, B), n->t[n->yout].grad, n->loss,
-                              n->stream));
+    UCHK(cffc_unet_launch_mse(n->y4, n->target, (int64_t)npix(n, 0, B), MSE_WG, n->t[n->yout].G, n->L.back().dbp,
+                              n->lossp, n->stream));
     if (int e = backward(n, B)) return e;
     if (loss) {
         UCHK(hipMemcpyAsync(loss, n->loss, 4, hipMemcpyDeviceToHost, n->stream));
@@ -373,9 +385,7 @@ extern "C" int cffc_unet_train_step(cffc_unet *n, const int32_t *idx, int B, flo
     n->step += 1;
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.f - std::pow(b1, (float)n->step), c2 = 1.f - std::pow(b2, (float)n->step);
-    for (Conv &c : n->L)
-        UCHK(cffc_unet_launch_adam(c.w, c.gw, c.m, c.v, c.Cout, c.CA + c.CB, c.Kpad, c.Kpad2, c.wt, c.wd, lr, b1, b2,
-                                   1e-8f, c1, c2, 1, c.b, c.gb, c.mb, c.vb, n->stream));
+    if (int e = run_adam(n, 0, (int)n->L.size() - 1, 1, lr, b1, b2, 1e-8f, c1, c2)) return e;
     UCHK(hipStreamSynchronize(n->stream));
     if (loss) *loss = l;
     return 0;
@@ -400,15 +410,13 @@ extern "C" int cffc_unet_loss_grad(cffc_unet *n, const int32_t *idx, int B, floa
 extern "C" int cffc_unet_predict(cffc_unet *n, const float *inputs, int B, float *outputs) {
     if (!n || B <= 0 || B > n->maxB || !inputs || !outputs) return ufail(CFFC_E_ARG, "bad batch");
     const size_t px = (size_t)n->H * n->W;
-    std::vector<bf16_t> hin(px * CFFC_UNET_IN * B);
-    for (size_t q = 0; q < hin.size(); ++q) hin[q] = host_f2bf(inputs[q]);
-    UCHK(hipMemcpyAsync(n->t[n->x0].act, hin.data(), hin.size() * 2, hipMemcpyHostToDevice, n->stream));
+    // rounded to BF16 on the device; the four FP32 output channels come back as
+    // the last convolution stores them
+    UCHK(hipMemcpyAsync(n->x32, inputs, px * CFFC_UNET_IN * B * 4, hipMemcpyHostToDevice, n->stream));
+    UCHK(cffc_unet_launch_to_bf16(n->x32, n->t[n->x0].act, (int64_t)px * CFFC_UNET_IN * B, n->stream));
     if (int e = forward(n, B)) return e;
-    std::vector<float> y(px * 16 * B);
-    UCHK(hipMemcpyAsync(y.data(), n->y32, y.size() * 4, hipMemcpyDeviceToHost, n->stream));
+    UCHK(hipMemcpyAsync(outputs, n->y4, px * CFFC_UNET_OUT * B * 4, hipMemcpyDeviceToHost, n->stream));
     UCHK(hipStreamSynchronize(n->stream));
-    for (size_t p = 0; p < px * B; ++p)
-        for (int c = 0; c < CFFC_UNET_OUT; ++c) outputs[p * CFFC_UNET_OUT + c] = y[p * 16 + c];
     return 0;
 }
 

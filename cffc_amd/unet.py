@@ -120,12 +120,10 @@ class UNet:
 
     def predict(self, X):
         X = np.ascontiguousarray(X, dtype=np.float32)
-        out = np.zeros(X.shape[:3] + (NOUT,), dtype=np.float32)
+        out = np.empty(X.shape[:3] + (NOUT,), dtype=np.float32)
         for s in range(0, X.shape[0], self.max_batch):
-            xb = np.ascontiguousarray(X[s:s + self.max_batch])
-            ob = np.zeros(xb.shape[:3] + (NOUT,), dtype=np.float32)
+            xb, ob = X[s:s + self.max_batch], out[s:s + self.max_batch]
             _check(_lib().cffc_unet_predict(self.h, _pf(xb), xb.shape[0], _pf(ob)), "predict")
-            out[s:s + xb.shape[0]] = ob
         return out
 
     def train(self, nsteps, batch, lr=2e-3, seed=0, log_every=0):
