@@ -67,6 +67,11 @@ constexpr int MSE_WG = 256;   // workgroups of the loss kernel
 struct cffc_unet {
     int H = 0, W = 0, maxB = 0;
     hipStream_t stream = nullptr;
+    // the weight gradients run beside the chain of input gradients, a few
+    // layers at a time: they wait for their outputs' gradients (ready), the sums
+    // wait for them (joined)
+    hipStream_t side = nullptr;
+    hipEvent_t ready[4] = {nullptr, nullptr, nullptr, nullptr}, joined = nullptr;
     std::vector<Tensor> t;
     std::vector<Conv> L;
     int x0 = -1, yout = -1;
@@ -171,7 +176,12 @@ static int run_adam(cffc_unet *n, int first, int last, int update, float lr, flo
 extern "C" void cffc_unet_destroy(cffc_unet *n) {
     if (!n) return;
     if (n->stream) (void)hipStreamSynchronize(n->stream);
+    if (n->side) (void)hipStreamSynchronize(n->side);
     for (void *p : n->allocs) (void)hipFree(p);
+    for (hipEvent_t e : n->ready)
+        if (e) (void)hipEventDestroy(e);
+    if (n->joined) (void)hipEventDestroy(n->joined);
+    if (n->side) (void)hipStreamDestroy(n->side);
     if (n->stream) (void)hipStreamDestroy(n->stream);
     delete n;
 }
@@ -189,6 +199,13 @@ extern "C" int cffc_unet_create(int H, int W, int max_batch, uint64_t seed, cffc
         return ufail(CFFC_E_HIP, "stream creation failed");
     }
     build_graph(n);
+    bool ok = hipStreamCreateWithFlags(&n->side, hipStreamNonBlocking) == hipSuccess &&
+              hipEventCreateWithFlags(&n->joined, hipEventDisableTiming) == hipSuccess;
+    for (hipEvent_t &ev : n->ready) ok = ok && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+        cffc_unet_destroy(n);
+        return ufail(CFFC_E_HIP, "stream or event creation failed");
+    }
     int e = 0;
     for (auto &x : n->t) {
         const size_t np = (size_t)npix(n, x.level, max_batch) * x.C;
@@ -336,21 +353,34 @@ static int backward(cffc_unet *n, int B) {
     };
     sum(n->lossp, n->loss, 1, MSE_WG);
     sum(n->L.back().dbp, n->L.back().gb, n->L.back().Cout, MSE_WG);
-    for (int q = (int)n->L.size() - 1; q >= 0; --q) {
+    const int nl = (int)n->L.size();
+    int pending = nl - 1, group = 0;   // weight gradients not launched yet: layers q..pending
+    for (int q = nl - 1; q >= 0; --q) {
         const Conv &c = n->L[q];
-        const int H = n->H >> c.level, W = n->W >> c.level, Cin = c.CA + c.CB;
-        const bf16_t *G = n->t[c.out].G;
-        UCHK(cffc_unet_launch_conv_bwd_weight(G, c.Cout, n->t[c.inA].act, c.CA, c.upA,
-                                              c.inB >= 0 ? n->t[c.inB].act : nullptr, c.CB, B, H, W, c.part,
-                                              n->stream));
-        sum(c.part, c.gw, c.Cout * c.K, cffc_unet_wgrad_chunks(B, H, W, Cin, c.Cout));
+        if (q == 0 || (q & 3) == 3) {
+            // every gradient down to layer q's output is in the stream
+            UCHK(hipEventRecord(n->ready[group], n->stream));
+            UCHK(hipStreamWaitEvent(n->side, n->ready[group], 0));
+            group++;
+            for (; pending >= q; --pending) {
+                const Conv &w = n->L[pending];
+                const int H = n->H >> w.level, W = n->W >> w.level;
+                UCHK(cffc_unet_launch_conv_bwd_weight(n->t[w.out].G, w.Cout, n->t[w.inA].act, w.CA, w.upA,
+                                                      w.inB >= 0 ? n->t[w.inB].act : nullptr, w.CB, B, H, W, w.part,
+                                                      n->side));
+                sum(w.part, w.gw, w.Cout * w.K, cffc_unet_wgrad_chunks(B, H, W, w.CA + w.CB, w.Cout));
+            }
+        }
         if (c.target < 0) continue;
+        const int H = n->H >> c.level, W = n->W >> c.level, Cin = c.CA + c.CB;
         const Tensor &t = n->t[c.target];
         const Conv &pr = n->L[t.producer];
-        UCHK(cffc_unet_launch_conv_bwd_data(G, c.Cout, B, H, W, c.wd, Cin, c.CA, c.kind, t.act, t.G, pr.dbp,
+        UCHK(cffc_unet_launch_conv_bwd_data(n->t[c.out].G, c.Cout, B, H, W, c.wd, Cin, c.CA, c.kind, t.act, t.G, pr.dbp,
                                             c.inB >= 0 ? n->t[c.inB].gskip : nullptr, t.gskip, n->stream));
         sum(pr.dbp, pr.gb, pr.Cout, cffc_unet_conv_tiles(B, H, W, Cin));
     }
+    UCHK(hipEventRecord(n->joined, n->side));
+    UCHK(hipStreamWaitEvent(n->stream, n->joined, 0));
     UCHK(cffc_unet_launch_reduce(&S, n->stream));
     return 0;
 }

@@ -143,21 +143,34 @@ __global__ __launch_bounds__(256) void conv_tile_kernel(ConvArgs a) {
     const int ntx = (a.W + TW - 1) / TW, nty = (a.H + TH - 1) / TH;
     const int tx = blockIdx.x % ntx, ty = (blockIdx.x / ntx) % nty, b = blockIdx.x / (ntx * nty);
     const int x0 = tx * TW, y0 = ty * TH;
-    for (int u = tid; u < (TH + 2) * HW * C8; u += 256) {
-        const int pix = u / C8, c = (u - pix * C8) * 8;
-        const int row = pix / HW, yy = y0 + row - 1, xx = x0 + (pix - row * HW) - 1;
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (yy >= 0 && yy < a.H && xx >= 0 && xx < a.W) {
-            if (c < a.CA) {
-                const int64_t q = a.upA ? ((int64_t)b * (a.H >> 1) + (yy >> 1)) * (a.W >> 1) + (xx >> 1)
-                                        : ((int64_t)b * a.H + yy) * a.W + xx;
-                v = *(const uint4 *)(a.xA + q * a.CA + c);
-            } else {
-                const int64_t q = ((int64_t)b * a.H + yy) * a.W + xx;
-                v = *(const uint4 *)(a.xB + q * (CIN - a.CA) + (c - a.CA));
+    // six 16-byte loads in flight per thread before their LDS stores: one after
+    // the other, the 17 of a 192-channel tile are 17 memory latencies
+    constexpr int NU = (TH + 2) * HW * C8, NIT = (NU + 255) / 256, UB = NIT < 6 ? NIT : 6;
+    for (int k0 = 0; k0 < NIT; k0 += UB) {
+        uint4 v[UB];
+#pragma unroll
+        for (int k = 0; k < UB; ++k) {
+            const int u = tid + (k0 + k) * 256;
+            const int pix = u / C8, c = (u - pix * C8) * 8;
+            const int row = pix / HW, yy = y0 + row - 1, xx = x0 + (pix - row * HW) - 1;
+            v[k] = make_uint4(0, 0, 0, 0);
+            if (u < NU && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W) {
+                if (c < a.CA) {
+                    const int64_t q = a.upA ? ((int64_t)b * (a.H >> 1) + (yy >> 1)) * (a.W >> 1) + (xx >> 1)
+                                            : ((int64_t)b * a.H + yy) * a.W + xx;
+                    v[k] = *(const uint4 *)(a.xA + q * a.CA + c);
+                } else {
+                    const int64_t q = ((int64_t)b * a.H + yy) * a.W + xx;
+                    v[k] = *(const uint4 *)(a.xB + q * (CIN - a.CA) + (c - a.CA));
+                }
             }
         }
-        *(uint4 *)(sx + pix * CS + c) = v;
+#pragma unroll
+        for (int k = 0; k < UB; ++k) {
+            const int u = tid + (k0 + k) * 256;
+            const int pix = u / C8, c = (u - pix * C8) * 8;
+            if (u < NU) *(uint4 *)(sx + pix * CS + c) = v[k];
+        }
     }
     __syncthreads();
     const int px = lane & 15, kg = lane >> 4;
@@ -300,8 +313,8 @@ __global__ __launch_bounds__(256) void conv_tile_kernel(ConvArgs a) {
 // (ds_read_b64_tr_b16: four pixels by 16 channels per 16 lanes), each tap a
 // shifted address in the same tile.  COB < 4: the four waves also split a tile's
 // pixels and add up at the end.  C8: an 8-channel input, two taps per 16 columns.
-// Against per-tap gathers, transposing stores and atomics (86 us a layer of a
-// 16-image batch) the operands are read once per tile.
+// Per layer of a 16-image batch of 64 x 192: 8 to 11 us; with per-tap gathers,
+// transposing stores and atomics it was 86 us.
 struct WgradArgs {
     const bf16_t *G;
     int Cout;
@@ -340,27 +353,49 @@ __global__ __launch_bounds__(256) void conv_wgrad_kernel(WgradArgs a) {
     f32x4 acc[NBK];
 #pragma unroll
     for (int n = 0; n < NBK; ++n) acc[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
+    // the next tile's operands are loaded into registers while this one's are
+    // multiplied
+    constexpr int NUG = TH * TW * COB * 2 / 256, NUX = ((TH + 2) * HW * (NX / 8) + 255) / 256;
+    uint4 vg[NUG], vx[NUX];
+    auto load_tile = [&](int t) {
         const int x0 = (t % ntx) * TW, y0 = ((t / ntx) % nty) * TH, b = t / (ntx * nty);
-        for (int u = tid; u < TH * TW * COB * 2; u += 256) {
+#pragma unroll
+        for (int k = 0; k < NUG; ++k) {
+            const int u = tid + k * 256;
             const int pix = u / (COB * 2), c = (u - pix * (COB * 2)) * 8;
             const int yy = y0 + (pix >> 4), xx = x0 + (pix & 15);
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (yy < a.H && xx < a.W) v = *(const uint4 *)(a.G + (((int64_t)b * a.H + yy) * a.W + xx) * a.Cout + co0 + c);
-            *(uint4 *)(sG + pix * GS + c) = v;
+            vg[k] = make_uint4(0, 0, 0, 0);
+            if (yy < a.H && xx < a.W)
+                vg[k] = *(const uint4 *)(a.G + (((int64_t)b * a.H + yy) * a.W + xx) * a.Cout + co0 + c);
         }
-        for (int u = tid; u < (TH + 2) * HW * (NX / 8); u += 256) {
+#pragma unroll
+        for (int k = 0; k < NUX; ++k) {
+            const int u = tid + k * 256;
             const int pix = u / (NX / 8), c = (u - pix * (NX / 8)) * 8;
             const int row = pix / HW, yy = y0 + row - 1, xx = x0 + (pix - row * HW) - 1;
-            uint4 v = make_uint4(0, 0, 0, 0);
-            if (yy >= 0 && yy < a.H && xx >= 0 && xx < a.W) {
+            vx[k] = make_uint4(0, 0, 0, 0);
+            if (row < TH + 2 && yy >= 0 && yy < a.H && xx >= 0 && xx < a.W) {
                 const int64_t q = up ? ((int64_t)b * (a.H >> 1) + (yy >> 1)) * (a.W >> 1) + (xx >> 1)
                                      : ((int64_t)b * a.H + yy) * a.W + xx;
-                v = *(const uint4 *)(x + q * xc + xc0 + c);
+                vx[k] = *(const uint4 *)(x + q * xc + xc0 + c);
             }
-            *(uint4 *)(sX + pix * NX + c) = v;
+        }
+    };
+    if ((int)blockIdx.x < a.ntiles) load_tile(blockIdx.x);
+    for (int t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
+#pragma unroll
+        for (int k = 0; k < NUG; ++k) {
+            const int u = tid + k * 256;
+            const int pix = u / (COB * 2), c = (u - pix * (COB * 2)) * 8;
+            *(uint4 *)(sG + pix * GS + c) = vg[k];
+        }
+#pragma unroll
+        for (int k = 0; k < NUX; ++k) {
+            const int u = tid + k * 256;
+            if (u < (TH + 2) * HW * (NX / 8)) *(uint4 *)(sX + u * 8) = vx[k];   // rows of NX, no padding
         }
         __syncthreads();
+        if (t + (int)gridDim.x < a.ntiles) load_tile(t + gridDim.x);
         // 32 pixels a step: two rows of 16; lane group g takes pixels 8g..8g+7,
         // four of them (row, 8*(g&1) + 4h + ...) with each of two reads
 #pragma unroll
@@ -573,7 +608,8 @@ template <int CIN, bool BWD> static hipError_t launch_conv(const ConvArgs &a, hi
 }
 
 // pixel chunks (partials) of a weight gradient: about 256 workgroups over the
-// channel blocks
+// channel blocks (a training pass of 16 images: 430 us; with 128 workgroups
+// 481 us, with 512, whose partials take longer to add, 451 us)
 static int wgrad_chunks(int B, int H, int W, int Cin, int Cout) {
     const int tiles = B * ((W + 15) / 16) * ((H + 7) / 8);
     const int blocks = ((Cin + 15) / 16) * (Cout >= 64 ? Cout / 64 : 1);
