@@ -101,7 +101,7 @@ struct cffc_ctx {
     // the fused stage kernel forms the physical ghosts in its own window: one
     // level (the coarse-to-fine messages read them from HBM) and no periodic
     // boundary (its ghosts come from the far side of the block)
-    bool window_bcs = false;
+    bool windowable = false, window_bcs = false;   // could, and does where it is faster
     int nbc = 0;
     int32_t *bc_blocks = nullptr;
     // resolution changes (quadtree meshes): level-change legs of the exchange
@@ -888,6 +888,7 @@ extern "C" int cffc_create(const cffc_mesh_desc *md, const cffc_scheme_desc *sd,
         // 262 k cells, 0.820 against 0.824 at 2.0 M, 1.634 against 1.603 at
         // 4.2 M; mixed 0.237 against 0.253 ms at 1.0 M, 1.396 against 1.407 at
         // 6.6 M.
+        c->windowable = windowed;
         c->window_bcs = windowed && (c->s.flux_precision == CFFC_FLUX_FP32 || c->ncell <= (int64_t)1 << 21);
         c->nbc = (int)bl.size();
         if (!bl.empty()) {
@@ -1324,7 +1325,7 @@ extern "C" int cffc_cfl(cffc_ctx *c, double *dt_min, int set_global) {
     if (!c) return fail(CFFC_E_ARG, "null context");
     HIPCHK(cffc_launch_set_u64(c->scal, MILLION_BITS, 0, 1, c->stream));
     HIPCHK(cffc_launch_cfl(c->meta, c->tiles, c->ntiles, c->ti, c->tj, c->W[c->wcur], c->geom, c->ncp, c->dt, c->scal,
-                           c->stream));
+                           nullptr, nullptr, nullptr, c->stream));
     if (set_global) HIPCHK(cffc_launch_set_global_dt(c->meta, c->nblk, c->max_int, c->dt, c->scal, c->stream));
     unsigned long long bits = 0;
     HIPCHK(hipMemcpyAsync(&bits, c->scal, sizeof bits, hipMemcpyDeviceToHost, c->stream));
@@ -1440,7 +1441,7 @@ extern "C" int cffc_update_stage(cffc_ctx *c, int i_stage, int64_t *bad_cell) {
 extern "C" int cffc_residual_norms(cffc_ctx *c, int var, double out[3]) {
     if (!c || !out || var < 1 || var > 4) return fail(CFFC_E_ARG, "bad argument");
     HIPCHK(cffc_launch_norms(c->meta, c->tiles, c->ntiles, c->ti, c->tj, c->dUdt[0], c->ncp, var, c->norm_part,
-                             c->norm_small, c->stream));
+                             c->norm_small, nullptr, c->stream));
     HIPCHK(hipMemcpyAsync(out, c->norm_small, 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return 0;
@@ -1635,7 +1636,7 @@ static int begin_run(cffc_ctx *c, int nsteps) {
     // CFL of the first step from the current state (slot 0)
     HIPCHK(cffc_launch_set_u64(c->scal, MILLION_BITS, MILLION_BITS, 2, c->stream));
     HIPCHK(cffc_launch_cfl(c->meta, c->tiles, c->ntiles, c->ti, c->tj, c->W[c->wcur], c->geom, c->ncp, c->dt, c->scal,
-                           c->stream));
+                           nullptr, nullptr, nullptr, c->stream));
     if (c->Wf[0]) {
         // the fused mixed path keeps W in FP32: derive it from U
         HIPCHK(cffc_launch_w_from_u(c->meta, c->nblk, c->max_int, c->U, nullptr, c->Wf[c->wcur], c->ncp, c->stream));
@@ -2110,7 +2111,6 @@ struct cffc_mg {
     std::vector<cffc_ctx *> lv;
     cffc_mg_desc d{};
     std::vector<double *> P, uo;     // per level (P unused on level 0)
-    std::vector<int> max_edge;       // per level: max ni + nj over blocks
     std::vector<double> Ahost;       // scratch: fine-level areas for the Wo restriction
     double rs_eps = 0.0;
     int rs_iters = 0;
@@ -2123,7 +2123,12 @@ struct cffc_mg {
     bool use_graph = true;
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
-    int graph_frozen = -1, graph_top = -1;
+    int graph_frozen = -1, graph_top = -1, graph_base = -1;
+    // norms of the top level and the levels' error keys of the last check, and
+    // the parts' norms, in pinned host memory (written by the kernels)
+    double *status = nullptr;
+    ErrorKeys keys{};
+    int base = 0;   // W buffer of the top level at the start of a cycle
     // per-case stopping (cffc_mg_set_parts): part q owns level-0 blocks
     // part_block0[q] .. part_block0[q+1]-1; per part its tolerance, freeze
     // level, last checked L2 norm and the regular cycles done when its norm
@@ -2153,7 +2158,8 @@ static void mg_free(cffc_mg *mg) {
     if (!mg) return;
     for (int32_t *q : {mg->d_tile0, mg->d_part_of_block, mg->d_part_frozen})
         if (q) (void)hipFree(q);
-    if (mg->d_part_l2) (void)hipFree(mg->d_part_l2);
+    if (mg->d_part_l2) (void)hipHostFree(mg->d_part_l2);
+    if (mg->status) (void)hipHostFree(mg->status);
     if (mg->gexec) (void)hipGraphExecDestroy(mg->gexec);
     if (mg->graph) (void)hipGraphDestroy(mg->graph);
     for (size_t l = 0; l < mg->lv.size(); ++l) {
@@ -2209,7 +2215,6 @@ extern "C" int cffc_mg_create(const cffc_mesh_desc *levels, int nlevels, const c
     mg->lv.assign(nlevels, nullptr);
     mg->P.assign(nlevels, nullptr);
     mg->uo.assign(nlevels, nullptr);
-    mg->max_edge.assign(nlevels, 0);
     for (int l = 0; l < nlevels; ++l) {
         if (int e = cffc_create(&levels[l], smoother, &mg->lv[l])) {
             mg_free(mg);
@@ -2235,7 +2240,12 @@ extern "C" int cffc_mg_create(const cffc_mesh_desc *levels, int nlevels, const c
             mg_free(mg);
             return fail(CFFC_E_HIP, "hipMemsetAsync failed");
         }
-        for (int b = 0; b < c->nblk; ++b) mg->max_edge[l] = std::max(mg->max_edge[l], c->meta_h[b].ni + c->meta_h[b].nj);
+    }
+    mg->keys.n = std::min(nlevels, MAX_KEYS);   // a level halves the blocks: 32 are out of reach
+    for (int l = 0; l < mg->keys.n; ++l) mg->keys.key[l] = mg->lv[l]->scal + 2;
+    if (hipHostMalloc((void **)&mg->status, (3 + MAX_KEYS) * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        mg_free(mg);
+        return fail(CFFC_E_NOMEM, "hipHostMalloc failed");
     }
     mg_set_top(mg, 0);
     if (hipStreamSynchronize(mg->lv[0]->stream) != hipSuccess) {
@@ -2253,6 +2263,8 @@ extern "C" int cffc_mg_set_residual_smoothing(cffc_mg *mg, double epsilon, int i
     return 0;
 }
 
+static const double *area(const cffc_ctx *c) { return c->geom + (size_t)GEO_A * c->ncp; }
+
 // Exchange_Solution_Information + BCs of one level (U sent, W = W(U))
 static int mg_exchange(cffc_ctx *c) {
     ExchangeParams p = exchange_params(c, 1, nullptr);
@@ -2261,11 +2273,9 @@ static int mg_exchange(cffc_ctx *c) {
     return 0;
 }
 
-static const double *area(const cffc_ctx *c) { return c->geom + (size_t)GEO_A * c->ncp; }
-
 // one granular FP64 stage kernel: a smoothing stage (residual = 0) or
 // dUdt_Residual_Evaluation into dUdt[0] (residual = 1); P: forcing term or null
-static int mg_stage(cffc_ctx *c, int i_stage, int residual, const double *P) {
+static int mg_stage(cffc_ctx *c, int i_stage, int residual, const double *P, double *Psub = nullptr) {
     StageParams p = base_stage_params(c);
     p.Win = c->W[c->wcur];
     p.Wout = c->W[c->wcur];
@@ -2282,36 +2292,86 @@ static int mg_stage(cffc_ctx *c, int i_stage, int residual, const double *P) {
     p.hlle = c->s.i_flux_function == CFFC_FLUX_FUNCTION_HLLE;
     p.residual = residual;
     p.P = P;
+    p.Psub = Psub;
     HIPCHK(cffc_launch_stage_fp64(&p, c->ti, c->tj, 0, c->stream));
     return 0;
 }
 
-// Smooth :2865-3110
-static int mg_smooth(cffc_mg *mg, int top, int l) {
+// Whether a level's smoothing stages can each be one launch (SK_STEP): the
+// kernel fills its own ghost cells (no periodic boundary), every stage starts
+// from a zero residual (multistage optimal smoothing) and nothing runs between
+// the residual and the update.
+static bool mg_one_launch(const cffc_mg *mg, const cffc_ctx *c) {
+    const bool hlle = c->s.i_flux_function == CFFC_FLUX_FUNCTION_HLLE;
+    return c->windowable && mg->rs_iters == 0 && !c->s.axisymmetric &&
+           c->s.i_time_integration == CFFC_TIME_STEPPING_MULTISTAGE_OPTIMAL_SMOOTHING &&
+           (hlle ? c->s.i_limiter == CFFC_LIMITER_ZERO && !c->freeze
+                 : c->s.i_limiter == CFFC_LIMITER_VENKATAKRISHNAN);
+}
+
+// one smoothing stage from the level's W buffer to its other one; pull: the
+// ghost cells in the buffer are not current, the kernel forms its window's
+static int mg_step(cffc_ctx *c, int i_stage, int pull, const double *P) {
+    StageParams p = base_stage_params(c);
+    p.Win = c->W[c->wcur];
+    p.Wout = c->W[1 - c->wcur];
+    p.Uo = c->Uo;
+    p.first_stage = i_stage == 1;
+    p.pull = pull;
+    p.halve = c->s.local_time_stepping == CFFC_SCALAR_LOCAL_TIME_STEPPING;
+    p.omega = stage_omega(c->s, i_stage);
+    p.dtmin_in = c->scal;
+    p.lts = 1;
+    // the limiters of the residual that ends the smoothing are the ones kept
+    p.phi_mode = c->freeze ? PHI_LOAD : PHI_COMPUTE;
+    p.part_of_block = c->mg_part_of_block;
+    p.part_frozen = c->mg_part_frozen;
+    p.hlle = c->s.i_flux_function == CFFC_FLUX_FUNCTION_HLLE;
+    p.P = P;
+    HIPCHK(cffc_launch_mg_step(&p, c->ti, c->tj, c->stream));
+    c->wcur = 1 - c->wcur;
+    return 0;
+}
+
+// Smooth :2865-3110, n times.  Only the last one's closing exchange and
+// residual are evaluated: the next smoothing's stages replace both.
+static int mg_smooth(cffc_mg *mg, int top, int l, int n) {
     cffc_ctx *c = mg->lv[l];
-    // local time steps only (the levels' stages read dt per cell): no global
-    // minimum is formed
-    HIPCHK(cffc_launch_cfl(c->meta, c->tiles, c->ntiles, c->ti, c->tj, c->W[c->wcur], c->geom, c->ncp, c->dt, nullptr,
-                           c->stream));
-    if (l > top) {
-        cffc_ctx *f = mg->lv[l - 1];
-        HIPCHK(cffc_launch_mg_cfl(f->meta, c->meta, c->nblk, c->max_int, f->dt, area(f), c->dt, area(c), c->stream));
+    const double *P = l > top ? mg->P[l] : nullptr;
+    for (int nu = 0; nu < n; ++nu) {
+        // local time steps only (the levels' stages read dt per cell): no
+        // global minimum is formed
+        const cffc_ctx *f = l > top ? mg->lv[l - 1] : nullptr;
+        HIPCHK(cffc_launch_cfl(c->meta, c->tiles, c->ntiles, c->ti, c->tj, c->W[c->wcur], c->geom, c->ncp, c->dt,
+                               nullptr, f ? f->meta : nullptr, f ? f->dt : nullptr, f ? area(f) : nullptr, c->stream));
+        if (mg_one_launch(mg, c)) {
+            // Stage 1 of the first smoothing reads the ghosts that the exchange
+            // after the restriction or prolongation filled; the top level, whose
+            // state may have been set since, exchanges first (ghosts = W(U))
+            if (nu == 0 && l == top)
+                if (int e = mg_exchange(c)) return e;
+            for (int st = 1; st <= c->s.n_stage; ++st)
+                if (int e = mg_step(c, st, nu > 0 || st > 1, P)) return e;
+            continue;
+        }
+        for (int st = 1; st <= c->s.n_stage; ++st) {
+            if (int e = mg_exchange(c)) return e;
+            if (st == 1)
+                HIPCHK(cffc_launch_copy_interior(c->meta, c->nblk, c->max_int, c->U, c->Uo, c->ncp, c->stream));
+            if (int e = mg_stage(c, st, 0, P)) return e;
+            if (mg->rs_iters > 0)
+                HIPCHK(cffc_launch_residual_smoothing(c->meta, c->nblk, c->dUdt[0], c->dUdt[1], c->ncp, mg->rs_eps,
+                                                      mg->rs_iters, nullptr, nullptr, c->stream));
+            const int k = k_residual(c->s, st);
+            HIPCHK(cffc_launch_update(c->meta, c->nblk, c->max_int, c->W[c->wcur], c->U, c->Uo, c->dUdt[k], c->dt,
+                                      c->ncp, stage_omega(c->s, st),
+                                      c->s.local_time_stepping == CFFC_SCALAR_LOCAL_TIME_STEPPING, c->scal + 2,
+                                      c->stream));
+        }
     }
-    for (int st = 1; st <= c->s.n_stage; ++st) {
-        if (int e = mg_exchange(c)) return e;
-        if (st == 1) HIPCHK(cffc_launch_copy_interior(c->meta, c->nblk, c->max_int, c->U, c->Uo, c->ncp, c->stream));
-        if (int e = mg_stage(c, st, 0, l > top ? mg->P[l] : nullptr)) return e;
-        if (mg->rs_iters > 0)
-            HIPCHK(cffc_launch_residual_smoothing(c->meta, c->nblk, c->dUdt[0], c->dUdt[1], c->ncp, mg->rs_eps,
-                                                  mg->rs_iters, nullptr, nullptr, c->stream));
-        const int k = k_residual(c->s, st);
-        HIPCHK(cffc_launch_update(c->meta, c->nblk, c->max_int, c->W[c->wcur], c->U, c->Uo, c->dUdt[k], c->dt, c->ncp,
-                                  stage_omega(c->s, st),
-                                  c->s.local_time_stepping == CFFC_SCALAR_LOCAL_TIME_STEPPING, c->scal + 2,
-                                  c->stream));
-    }
+    if (n == 0) return 0;
     if (int e = mg_exchange(c)) return e;
-    if (int e = mg_stage(c, 1, 1, l > top ? mg->P[l] : nullptr)) return e;
+    if (int e = mg_stage(c, 1, 1, P)) return e;
     if (!c->freeze) c->phi_valid = 1;
     return 0;
 }
@@ -2322,48 +2382,42 @@ static int mg_store_uo(cffc_mg *mg, int l) {
     return 0;
 }
 
-// Coarse_Grid_Correction :3118-3370
+// Coarse_Grid_Correction :3118-3370.  A smoothing with an odd stage count ends
+// in the other W buffer; restriction (coarse level) and prolongation (this
+// level), which form every interior W again, put it back into the first, so
+// that a captured cycle ends where it began.
 static int mg_cgc(cffc_mg *mg, int top, int l) {
     const cffc_mg_desc &d = mg->d;
     const int L = (int)mg->lv.size();
     cffc_ctx *c = mg->lv[l];
+    const int base = l == top ? mg->base : 0;
     int e;
     if (l == L - 1) {
-        if ((e = mg_store_uo(mg, l))) return e;
-        for (int nu = 1; nu <= d.smooths_on_coarsest_level; ++nu)
-            if ((e = mg_smooth(mg, top, l))) return e;
+        if (l != top && (e = mg_store_uo(mg, l))) return e;
+        if ((e = mg_smooth(mg, top, l, d.smooths_on_coarsest_level))) return e;
     } else {
         cffc_ctx *cc = mg->lv[l + 1];
         // the W cycle's two passes apply below the finest level, whatever
         // the top level (:3151-3158)
         const int m_cycle = (d.i_cycle == CFFC_MULTIGRID_V_CYCLE || l == 0) ? 1 : 2;
         for (int m = 1; m <= m_cycle; ++m) {
-            if ((e = mg_store_uo(mg, l))) return e;
-            const int n_pre = l == top ? d.smooths_on_finest_level : d.pre_smooths;
-            for (int nu = 0; nu < n_pre; ++nu)
-                if ((e = mg_smooth(mg, top, l))) return e;
-            HIPCHK(cffc_launch_mg_restrict(c->meta, cc->meta, c->nblk, cc->max_int, c->U, area(c), c->ncp, cc->U,
-                                           area(cc), cc->ncp, c->stream));
-            HIPCHK(cffc_launch_mg_primitive(cc->meta, cc->nblk, cc->max_int, cc->U, cc->W[cc->wcur], cc->ncp,
-                                            c->stream));
+            // uo serves the change that a level returns, which the top does not
+            if (l != top && (e = mg_store_uo(mg, l))) return e;
+            if ((e = mg_smooth(mg, top, l, l == top ? d.smooths_on_finest_level : d.pre_smooths))) return e;
+            cc->wcur = 0;
+            HIPCHK(cffc_launch_mg_restrict(c->meta, cc->meta, c->nblk, cc->max_int, c->U,
+                                           d.defect_correction ? c->dUdt[0] : nullptr, area(c), c->ncp, cc->U,
+                                           cc->W[0], mg->P[l + 1], area(cc), cc->ncp, c->stream));
             if ((e = mg_exchange(cc))) return e;
-            if (d.defect_correction) {
-                HIPCHK(cffc_launch_mg_restrict(c->meta, cc->meta, c->nblk, cc->max_int, c->dUdt[0], area(c), c->ncp,
-                                               mg->P[l + 1], area(cc), cc->ncp, c->stream));
-                if ((e = mg_stage(cc, 1, 1, nullptr))) return e;
-                HIPCHK(cffc_launch_mg_subtract(cc->meta, cc->nblk, cc->max_int, mg->P[l + 1], cc->dUdt[0], cc->ncp,
-                                               c->stream));
-            }
+            if (d.defect_correction && (e = mg_stage(cc, 1, 1, nullptr, mg->P[l + 1]))) return e;
             if ((e = mg_cgc(mg, top, l + 1))) return e;
-            HIPCHK(cffc_launch_mg_prolong(cc->meta, c->meta, c->nblk, cc->max_int, mg->max_edge[l + 1], cc->bc, cc->U,
-                                          cc->geom, cc->ncp, c->U, c->geom, c->ncp, !d.prolong_using_injection,
+            c->wcur = base;
+            HIPCHK(cffc_launch_mg_prolong(cc->meta, c->meta, c->nblk, cc->max_int, cc->bc, cc->U, cc->geom, cc->ncp, c->U,
+                                          c->W[base], c->geom, c->ncp, !d.prolong_using_injection,
                                           d.injection_at_dirichlet, d.prolong_using_injection,
                                           d.update_stability_switch, d.max_update_reductions, 0, c->stream));
-            HIPCHK(cffc_launch_mg_primitive(c->meta, c->nblk, c->max_int, c->U, c->W[c->wcur], c->ncp, c->stream));
             if ((e = mg_exchange(c))) return e;
-            const int n_post = l == top ? 0 : d.post_smooths;
-            for (int nu = 0; nu < n_post; ++nu)
-                if ((e = mg_smooth(mg, top, l))) return e;
+            if ((e = mg_smooth(mg, top, l, l == top ? 0 : d.post_smooths))) return e;
         }
     }
     if (l != top) HIPCHK(cffc_launch_mg_changes(c->meta, c->nblk, c->max_cells, c->U, mg->uo[l], c->ncp, c->stream));
@@ -2443,9 +2497,8 @@ extern "C" int cffc_mg_initialize(cffc_mg *mg) {
     if (int e = mg_exchange(mg->lv[0])) return e;
     for (size_t l = 1; l < mg->lv.size(); ++l) {
         cffc_ctx *f = mg->lv[l - 1], *c = mg->lv[l];
-        HIPCHK(cffc_launch_mg_restrict(f->meta, c->meta, c->nblk, c->max_int, f->U, area(f), f->ncp, c->U, area(c),
-                                       c->ncp, c->stream));
-        HIPCHK(cffc_launch_mg_primitive(c->meta, c->nblk, c->max_int, c->U, c->W[c->wcur], c->ncp, c->stream));
+        HIPCHK(cffc_launch_mg_restrict(f->meta, c->meta, c->nblk, c->max_int, f->U, nullptr, area(f), f->ncp, c->U,
+                                       c->W[c->wcur], nullptr, area(c), c->ncp, c->stream));
         if (int e = mg_restrict_wo(mg, (int)l - 1)) return e;
         if (int e = mg_exchange(c)) return e;
     }
@@ -2454,7 +2507,7 @@ extern "C" int cffc_mg_initialize(cffc_mg *mg) {
 }
 
 static int mg_reset_errors(cffc_mg *mg) {
-    for (cffc_ctx *c : mg->lv) HIPCHK(cffc_launch_set_u64(c->scal + 2, ERR_NONE, 0, 1, c->stream));
+    HIPCHK(cffc_launch_reset_keys(&mg->keys, mg->lv[0]->stream));
     return 0;
 }
 // the first failing update of the last cycle, finest level first: level in
@@ -2478,6 +2531,7 @@ static int mg_check_errors(cffc_mg *mg, int64_t *bad_cell) {
 extern "C" int cffc_mg_cycle(cffc_mg *mg, int64_t *bad_cell) {
     if (!mg) return fail(CFFC_E_ARG, "null multigrid solver");
     mg_set_top(mg, 0);
+    mg->base = mg->lv[0]->wcur;
     if (int e = mg_reset_errors(mg)) return e;
     if (int e = mg_cgc(mg, 0, 0)) return e;
     return mg_check_errors(mg, bad_cell);
@@ -2494,11 +2548,12 @@ extern "C" int cffc_mg_set_graph(cffc_mg *mg, int on) {
 // changes), or the launches themselves
 static int mg_enqueue_cycle(cffc_mg *mg, int top) {
     cffc_ctx *f = mg->lv[0];
+    mg->base = mg->lv[top]->wcur;
     if (!mg->use_graph) {
         if (int e = mg_reset_errors(mg)) return e;
         return mg_cgc(mg, top, top);
     }
-    if (!mg->gexec || mg->graph_frozen != (int)mg->frozen || mg->graph_top != top) {
+    if (!mg->gexec || mg->graph_frozen != (int)mg->frozen || mg->graph_top != top || mg->graph_base != mg->base) {
         if (mg->gexec) (void)hipGraphExecDestroy(mg->gexec);
         if (mg->graph) (void)hipGraphDestroy(mg->graph);
         mg->gexec = nullptr;
@@ -2512,6 +2567,7 @@ static int mg_enqueue_cycle(cffc_mg *mg, int top) {
         HIPCHK(hipGraphInstantiate(&mg->gexec, mg->graph, nullptr, nullptr, 0));
         mg->graph_frozen = (int)mg->frozen;
         mg->graph_top = top;
+        mg->graph_base = mg->base;
     }
     HIPCHK(hipGraphLaunch(mg->gexec, f->stream));
     return 0;
@@ -2584,10 +2640,11 @@ extern "C" int cffc_mg_set_parts(cffc_mg *mg, int npart, const int32_t *first_bl
         }
     for (int32_t **q : {&mg->d_tile0, &mg->d_part_of_block, &mg->d_part_frozen})
         if (*q) { (void)hipFree(*q); *q = nullptr; }
-    if (mg->d_part_l2) (void)hipFree(mg->d_part_l2);
+    if (mg->d_part_l2) (void)hipHostFree(mg->d_part_l2);
     mg->d_part_l2 = nullptr;
     if (int e = dalloc(&mg->d_tile0, npart + 1)) return e;
-    if (int e = dalloc(&mg->d_part_l2, npart)) return e;
+    if (hipHostMalloc((void **)&mg->d_part_l2, npart * sizeof(double), hipHostMallocDefault) != hipSuccess)
+        return fail(CFFC_E_NOMEM, "hipHostMalloc failed");
     if (int e = dalloc(&mg->d_part_of_block, f->nblk)) return e;
     if (int e = dalloc(&mg->d_part_frozen, npart)) return e;
     HIPCHK(hipMemcpy(mg->d_part_of_block, pob.data(), pob.size() * sizeof(int32_t), hipMemcpyHostToDevice));
@@ -2641,7 +2698,6 @@ extern "C" int cffc_mg_execute(cffc_mg *mg, int max_cycles, double freeze_level,
     const int L = (int)mg->lv.size();
     bool first_step = true;
     int n = 0, nchk = 0, rc = 0;
-    std::vector<unsigned long long> keys(mg->lv.size());
     if (int e = mg_reset_errors(mg)) return e;
     if (mg->npart)
         if (int e = mg_part_tiles(mg)) return e;
@@ -2658,20 +2714,18 @@ extern "C" int cffc_mg_execute(cffc_mg *mg, int max_cycles, double freeze_level,
         for (long long cycles = 1; cycles <= ncyc; ++cycles) {
             double nr[3];
             HIPCHK(cffc_launch_norms(t->meta, t->tiles, t->ntiles, t->ti, t->tj, t->dUdt[0], t->ncp, 1,
-                                     t->norm_part, t->norm_small, t->stream));
-            HIPCHK(hipMemcpyAsync(nr, t->norm_small, 3 * sizeof(double), hipMemcpyDeviceToHost, t->stream));
+                                     t->norm_part, mg->status, &mg->keys, t->stream));
             const bool parts = mg->npart && top == 0;
-            if (parts) {
+            if (parts)
                 HIPCHK(cffc_launch_part_norms(t->norm_part, mg->d_tile0, mg->npart, mg->d_part_l2, t->stream));
-                HIPCHK(hipMemcpyAsync(mg->part_l2.data(), mg->d_part_l2, mg->npart * sizeof(double),
-                                      hipMemcpyDeviceToHost, t->stream));
-            }
-            for (size_t l = 0; l < mg->lv.size(); ++l)
-                HIPCHK(hipMemcpyAsync(&keys[l], mg->lv[l]->scal + 2, sizeof(unsigned long long),
-                                      hipMemcpyDeviceToHost, t->stream));
             HIPCHK(hipStreamSynchronize(t->stream));
-            for (size_t l = 0; l < keys.size() && !rc; ++l)
-                if (keys[l] != ERR_NONE) rc = (int)(keys[l] & 0xFFFF);
+            memcpy(nr, mg->status, sizeof nr);
+            if (parts) memcpy(mg->part_l2.data(), mg->d_part_l2, mg->npart * sizeof(double));
+            for (int l = 0; l < mg->keys.n && !rc; ++l) {
+                unsigned long long key;
+                memcpy(&key, mg->status + 3 + l, sizeof key);
+                if (key != ERR_NONE) rc = (int)(key & 0xFFFF);
+            }
             if (rc) break;
             if (norms) memcpy(norms + 3 * nchk, nr, sizeof nr);
             nchk++;
@@ -2722,9 +2776,9 @@ extern "C" int cffc_mg_execute(cffc_mg *mg, int max_cycles, double freeze_level,
         }
         if (top != 0 && !rc) {
             cffc_ctx *f = mg->lv[top - 1];
-            HIPCHK(cffc_launch_mg_prolong(t->meta, f->meta, t->nblk, t->max_int, mg->max_edge[top], t->bc, t->U,
-                                          t->geom, t->ncp, f->U, f->geom, f->ncp, 0, 0, mg->d.prolong_using_injection,
-                                          0, 0, 1, t->stream));
+            HIPCHK(cffc_launch_mg_prolong(t->meta, f->meta, t->nblk, t->max_int, t->bc, t->U, t->geom, t->ncp, f->U,
+                                          nullptr, f->geom, f->ncp, 0, 0, mg->d.prolong_using_injection, 0, 0, 1,
+                                          t->stream));
             if (int e = mg_exchange(f)) return e;
         }
     }

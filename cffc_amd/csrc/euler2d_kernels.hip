@@ -344,10 +344,13 @@ __global__ __launch_bounds__(256) void exchange_bc_kernel(ExchangeParams p) {
 // ---------------------------------------------------------------------------
 // CFL over the interior cells of each tile; global minimum with atomicMin on
 // the bit pattern (positive doubles order like their bits), unless dtmin is
-// null (local time steps only).
+// null (local time steps only).  A coarse multigrid level (mf: the finer level's
+// blocks) then takes the minimum with its four fine cells' time steps scaled by
+// the square root of the area ratio (CFL_Multigrid, FASMultigrid2D.h:2364-2407).
 __global__ __launch_bounds__(256) void cfl_kernel(const BlockMeta *meta, const TileDesc *tiles, int ti, int tj,
                                                   const double *W, const double *geom, int64_t ncp, double *dt,
-                                                  unsigned long long *dtmin) {
+                                                  unsigned long long *dtmin, const BlockMeta *mf, const double *dtf,
+                                                  const double *Af) {
     __shared__ double sm[4];
     const TileDesc t = tiles[blockIdx.x];
     const BlockMeta m = meta[t.b];
@@ -369,7 +372,17 @@ __global__ __launch_bounds__(256) void cfl_kernel(const BlockMeta *meta, const T
         const double v_i = 0.5 * (Wc.vx * (G[GEO_NEX * ncp + c] - nWx) + Wc.vy * (G[GEO_NEY * ncp + c] - nWy));
         const double v_j = 0.5 * (Wc.vx * (G[GEO_NNX * ncp + c] - nSx) + Wc.vy * (G[GEO_NNY * ncp + c] - nSy));
         const double a = W_a(Wc);
-        const double d = dmin(qdiv(d_i, a + fabs(v_i)), qdiv(d_j, a + fabs(v_j)));
+        double d = dmin(qdiv(d_i, a + fabs(v_i)), qdiv(d_j, a + fabs(v_j)));
+        if (mf) {
+            const BlockMeta f = mf[t.b];
+            const int64_t sw = f.coff + (int64_t)(2 * (jp - 2) + 2) * f.pitch + 2 * (ip - 2) + 2;
+            const int64_t se = sw + 1, nw = sw + f.pitch, ne = nw + 1;
+            const double dt_NE = qsqrt(qdiv(A, Af[ne])) * dtf[ne];
+            const double dt_SE = qsqrt(qdiv(A, Af[se])) * dtf[se];
+            const double dt_NW = qsqrt(qdiv(A, Af[nw])) * dtf[nw];
+            const double dt_SW = qsqrt(qdiv(A, Af[sw])) * dtf[sw];
+            d = dmin(d, dmin(dt_NE, dmin(dt_SE, dmin(dt_NW, dt_SW))));
+        }
         dt[c] = d;
         dmn = dmin(dmn, d);
     }
@@ -467,8 +480,10 @@ __global__ __launch_bounds__(256) void norm_partial_kernel(const BlockMeta *meta
     }
 }
 
-__global__ __launch_bounds__(256) void norm_final_kernel(const double *part, int n, double *out) {
+// keys (multigrid): the levels' error keys, copied after the norms
+__global__ __launch_bounds__(256) void norm_final_kernel(const double *part, int n, double *out, ErrorKeys keys) {
     __shared__ double sm[4][3];
+    if ((int)threadIdx.x < keys.n) out[3 + threadIdx.x] = bitsd(*keys.key[threadIdx.x]);
     double a = 0.0, b = 0.0, mx = 0.0;
     for (int q = threadIdx.x; q < n; q += blockDim.x) { a += part[3 * q]; b += part[3 * q + 1]; mx = dmax(mx, part[3 * q + 2]); }
     for (int off = 32; off > 0; off >>= 1) {
@@ -718,6 +733,11 @@ __global__ __launch_bounds__(CHUNK_NT) void chunk_partial_kernel(const double *p
     }
 }
 
+// every level's error key to "none" (graph-safe, no memset nodes)
+__global__ void reset_keys_kernel(ErrorKeys keys) {
+    if ((int)threadIdx.x < keys.n) *keys.key[threadIdx.x] = ~0ull;
+}
+
 // small device-side scalar writes (graph-safe, no memset nodes)
 __global__ void set_u64_kernel(unsigned long long *dst, unsigned long long v0, unsigned long long v1, int n) {
     if (threadIdx.x == 0) { dst[0] = v0; if (n > 1) dst[1] = v1; }
@@ -745,6 +765,28 @@ __global__ void arith_check_kernel(const double *a, const double *b, int64_t n, 
     o[5] = fmin(x, y);
     o[6] = vmax64(x, y);
     o[7] = fmax(x, y);
+}
+
+static hipError_t launch_stage_kind(const StageParams *p, int ti, int tj, int kind, hipStream_t st) {
+#define L(TI, TJ)                                                                                          \
+    if (ti == TI && tj == TJ) {                                                                            \
+        switch (kind) {                                                                                    \
+        case SK_PLAIN: launch_stage_kernel<double, TI, TJ, SK_PLAIN>(p, st); break;                            \
+        case SK_WINDOW: launch_stage_kernel<double, TI, TJ, SK_WINDOW>(p, st); break;                          \
+        case SK_LEVELS: launch_stage_kernel<double, TI, TJ, SK_LEVELS>(p, st); break;                          \
+        case SK_MG: launch_stage_kernel<double, TI, TJ, SK_MG>(p, st); break;                              \
+        case SK_MG_FIRST: launch_stage_kernel<double, TI, TJ, SK_MG_FIRST>(p, st); break;                  \
+        case SK_STEP: launch_stage_kernel<double, TI, TJ, SK_STEP>(p, st); break;                          \
+        case SK_STEP_FIRST: launch_stage_kernel<double, TI, TJ, SK_STEP_FIRST>(p, st); break;              \
+        case SK_FUSED: launch_stage_kernel<double, TI, TJ, SK_FUSED>(p, st); break;                            \
+        default: launch_stage_kernel<double, TI, TJ, SK_GRANULAR>(p, st); break;                               \
+        }                                                                                                  \
+        return hipGetLastError();                                                                          \
+    }
+    CFFC_TILE_LIST(L)
+    CFFC_SMALL_TILE_LIST(L)
+#undef L
+    return hipErrorInvalidValue;
 }
 
 extern "C" {
@@ -794,10 +836,12 @@ hipError_t cffc_launch_widen(const float *src, double *dst, int64_t n, hipStream
     return hipGetLastError();
 }
 hipError_t cffc_launch_cfl(const BlockMeta *meta, const TileDesc *tiles, int ntiles, int ti, int tj, const double *W,
-                           const double *geom, int64_t ncp, double *dt, unsigned long long *dtmin, hipStream_t st) {
+                           const double *geom, int64_t ncp, double *dt, unsigned long long *dtmin, const BlockMeta *mf,
+                           const double *dtf, const double *Af, hipStream_t st) {
     // one thread per tile cell, in whole wavefronts up to 256
     const int nt = ti * tj <= 64 ? 64 : ti * tj <= 128 ? 128 : 256;
-    hipLaunchKernelGGL(cfl_kernel, dim3(ntiles), dim3(nt), 0, st, meta, tiles, ti, tj, W, geom, ncp, dt, dtmin);
+    hipLaunchKernelGGL(cfl_kernel, dim3(ntiles), dim3(nt), 0, st, meta, tiles, ti, tj, W, geom, ncp, dt, dtmin, mf, dtf,
+                       Af);
     return hipGetLastError();
 }
 hipError_t cffc_launch_set_global_dt(const BlockMeta *meta, int nblk, int max_int, double *dt,
@@ -820,9 +864,14 @@ hipError_t cffc_launch_copy_interior(const BlockMeta *meta, int nblk, int max_in
     return hipGetLastError();
 }
 hipError_t cffc_launch_norms(const BlockMeta *meta, const TileDesc *tiles, int ntiles, int ti, int tj,
-                             const double *dU, int64_t ncp, int var, double *part, double *out, hipStream_t st) {
+                             const double *dU, int64_t ncp, int var, double *part, double *out, const ErrorKeys *keys,
+                             hipStream_t st) {
     hipLaunchKernelGGL(norm_partial_kernel, dim3(ntiles), dim3(256), 0, st, meta, tiles, ti, tj, dU, ncp, var, part);
-    hipLaunchKernelGGL(norm_final_kernel, dim3(1), dim3(256), 0, st, part, ntiles, out);
+    hipLaunchKernelGGL(norm_final_kernel, dim3(1), dim3(256), 0, st, part, ntiles, out, keys ? *keys : ErrorKeys{});
+    return hipGetLastError();
+}
+hipError_t cffc_launch_reset_keys(const ErrorKeys *keys, hipStream_t st) {
+    hipLaunchKernelGGL(reset_keys_kernel, dim3(1), dim3(64), 0, st, *keys);
     return hipGetLastError();
 }
 hipError_t cffc_launch_set_u64(unsigned long long *dst, unsigned long long v0, unsigned long long v1, int n,
@@ -869,24 +918,12 @@ hipError_t cffc_launch_finish(const FinishParams *p, double *chunk_part, int nch
 }
 
 hipError_t cffc_launch_stage_fp64(const StageParams *p, int ti, int tj, int fused, hipStream_t st) {
-    int kind = stage_kind(*p, fused);
-#define L(TI, TJ)                                                                                          \
-    if (ti == TI && tj == TJ) {                                                                            \
-        switch (kind) {                                                                                    \
-        case SK_PLAIN: launch_stage_kernel<double, TI, TJ, SK_PLAIN>(p, st); break;                            \
-        case SK_WINDOW: launch_stage_kernel<double, TI, TJ, SK_WINDOW>(p, st); break;                          \
-        case SK_LEVELS: launch_stage_kernel<double, TI, TJ, SK_LEVELS>(p, st); break;                          \
-        case SK_MG: launch_stage_kernel<double, TI, TJ, SK_MG>(p, st); break;                              \
-        case SK_MG_FIRST: launch_stage_kernel<double, TI, TJ, SK_MG_FIRST>(p, st); break;                  \
-        case SK_FUSED: launch_stage_kernel<double, TI, TJ, SK_FUSED>(p, st); break;                            \
-        default: launch_stage_kernel<double, TI, TJ, SK_GRANULAR>(p, st); break;                               \
-        }                                                                                                  \
-        return hipGetLastError();                                                                          \
-    }
-    CFFC_TILE_LIST(L)
-    CFFC_SMALL_TILE_LIST(L)
-#undef L
-    return hipErrorInvalidValue;
+    return launch_stage_kind(p, ti, tj, stage_kind(*p, fused), st);
+}
+// one smoothing stage of a multigrid level (SK_STEP): ghosts, residual, forcing
+// term and update, from W (Win) to the level's other buffer (Wout)
+hipError_t cffc_launch_mg_step(const StageParams *p, int ti, int tj, hipStream_t st) {
+    return launch_stage_kind(p, ti, tj, p->hlle ? SK_STEP_FIRST : SK_STEP, st);
 }
 
 }  // extern "C"

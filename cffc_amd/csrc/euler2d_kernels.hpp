@@ -67,6 +67,13 @@ struct FinishParams {
     int32_t *part_best_step;                // [npart] step of that L2
 };
 
+// the error keys of a multigrid solver's levels
+constexpr int MAX_KEYS = 32;
+struct ErrorKeys {
+    unsigned long long *key[MAX_KEYS];
+    int n;
+};
+
 }  // namespace cffc
 
 // tile shapes the stage kernel is instantiated for (TI x TJ interior cells)
@@ -91,7 +98,7 @@ hipError_t cffc_launch_gather(const cffc::BlockMeta *meta, int nblk, int max_int
 hipError_t cffc_launch_exchange(const cffc::ExchangeParams *p, int nblk, hipStream_t st);
 hipError_t cffc_launch_cfl(const cffc::BlockMeta *meta, const cffc::TileDesc *tiles, int ntiles, int ti, int tj,
                            const double *W, const double *geom, int64_t ncp, double *dt, unsigned long long *dtmin,
-                           hipStream_t st);
+                           const cffc::BlockMeta *mf, const double *dtf, const double *Af, hipStream_t st);
 hipError_t cffc_launch_set_global_dt(const cffc::BlockMeta *meta, int nblk, int max_int, double *dt,
                                      const unsigned long long *dtmin, hipStream_t st);
 hipError_t cffc_launch_update(const cffc::BlockMeta *meta, int nblk, int max_int, double *W, double *U,
@@ -100,7 +107,10 @@ hipError_t cffc_launch_update(const cffc::BlockMeta *meta, int nblk, int max_int
 hipError_t cffc_launch_copy_interior(const cffc::BlockMeta *meta, int nblk, int max_int, const double *src,
                                      double *dst, int64_t ncp, hipStream_t st);
 hipError_t cffc_launch_norms(const cffc::BlockMeta *meta, const cffc::TileDesc *tiles, int ntiles, int ti, int tj,
-                             const double *dU, int64_t ncp, int var, double *part, double *out, hipStream_t st);
+                             const double *dU, int64_t ncp, int var, double *part, double *out,
+                             const cffc::ErrorKeys *keys, hipStream_t st);
+hipError_t cffc_launch_reset_keys(const cffc::ErrorKeys *keys, hipStream_t st);
+hipError_t cffc_launch_mg_step(const cffc::StageParams *p, int ti, int tj, hipStream_t st);
 hipError_t cffc_launch_set_u64(unsigned long long *dst, unsigned long long v0, unsigned long long v1, int n,
                                hipStream_t st);
 hipError_t cffc_launch_finish(const cffc::FinishParams *p, double *chunk_part, int nchunk, hipStream_t st);
@@ -124,21 +134,15 @@ hipError_t cffc_launch_flux_fix(const cffc::FluxFixOp *ops, int nops, double *S,
 hipError_t cffc_launch_stage_fp64(const cffc::StageParams *p, int ti, int tj, int fused, hipStream_t st);
 // multigrid level transfers (euler2d_mg.hip)
 hipError_t cffc_launch_mg_restrict(const cffc::BlockMeta *mf, const cffc::BlockMeta *mc, int nblk, int max_int_c,
-                                   const double *src, const double *Af, int64_t ncpf, double *dst, const double *Ac,
-                                   int64_t ncpc, hipStream_t st);
-hipError_t cffc_launch_mg_primitive(const cffc::BlockMeta *meta, int nblk, int max_int, const double *U, double *W,
-                                    int64_t ncp, hipStream_t st);
-hipError_t cffc_launch_mg_subtract(const cffc::BlockMeta *meta, int nblk, int max_int, double *P, const double *R,
-                                   int64_t ncp, hipStream_t st);
-hipError_t cffc_launch_mg_cfl(const cffc::BlockMeta *mf, const cffc::BlockMeta *mc, int nblk, int max_int_c,
-                              const double *dtf, const double *Af, double *dtc, const double *Ac, hipStream_t st);
+                                   const double *U, const double *R, const double *Af, int64_t ncpf, double *Uc,
+                                   double *Wc, double *P, const double *Ac, int64_t ncpc, hipStream_t st);
 hipError_t cffc_launch_mg_changes(const cffc::BlockMeta *meta, int nblk, int max_cells, double *U, const double *uo,
                                   int64_t ncp, hipStream_t st);
 hipError_t cffc_launch_mg_copy(const cffc::BlockMeta *meta, int nblk, int max_cells, double *dst, const double *src,
                                int64_t ncp, hipStream_t st);
 hipError_t cffc_launch_mg_prolong(const cffc::BlockMeta *mc, const cffc::BlockMeta *mf, int nblk, int max_int_c,
-                                  int max_edge_c, const int32_t *bc, double *Uc, const double *gc, int64_t ncpc,
-                                  double *Uf, const double *gf, int64_t ncpf, int neumann, int inj_dirichlet,
+                                  const int32_t *bc, const double *Uc, const double *gc, int64_t ncpc, double *Uf,
+                                  double *Wf, const double *gf, int64_t ncpf, int neumann, int inj_dirichlet,
                                   int inj_always, int stability, int max_red, int assign, hipStream_t st);
 hipError_t cffc_launch_stage_mixed(const cffc::StageParams *p, int ti, int tj, int fused, hipStream_t st);
 }

@@ -29,11 +29,14 @@ __device__ __forceinline__ void stU(double *U, int64_t ncp, int64_t c, const CS<
     U[c] = u.d; U[ncp + c] = u.mx; U[2 * ncp + c] = u.my; U[3 * ncp + c] = u.E;
 }
 
-// Restrict_Solution_Blocks :996-1037 (src = U, dst = U) and
-// Restrict_Residuals :1053-1095 (src = dUdt[0], dst = P): the area-weighted
-// average of the four fine cells, SW, SE, NW, NE in that order
-__global__ void mg_restrict_kernel(const BlockMeta *mf, const BlockMeta *mc, const double *src, const double *Af,
-                                   int64_t ncpf, double *dst, const double *Ac, int64_t ncpc) {
+// Restrict_Solution_Blocks :996-1037 (U -> Uc, with Update_Primitive_Variables
+// :2423-2445 into Wc) and, where R is given, Restrict_Residuals :1053-1095
+// (R -> P): the area-weighted average of the four fine cells, SW, SE, NW, NE
+// in that order.  One pass: both averages share the areas and their quotients
+// the coarse area's reciprocal.
+__global__ void mg_restrict_kernel(const BlockMeta *mf, const BlockMeta *mc, const double *U, const double *R,
+                                   const double *Af, int64_t ncpf, double *Uc, double *Wc, double *P, const double *Ac,
+                                   int64_t ncpc) {
     const BlockMeta f = mf[blockIdx.y], c = mc[blockIdx.y];
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= c.ni * c.nj || c.skip) return;
@@ -43,49 +46,18 @@ __global__ void mg_restrict_kernel(const BlockMeta *mf, const BlockMeta *mc, con
     const double A0 = Af[q0], A1 = Af[q1], A2 = Af[q2], A3 = Af[q3];
     const int64_t cc = cell(c, ic, jc);
     const Recip<double> rA = recip(Ac[cc]);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
+    auto average = [&](const double *src, int v) {
         const double *s = src + v * ncpf;
-        dst[v * ncpc + cc] = rdiv(s[q0] * A0 + s[q1] * A1 + s[q2] * A2 + s[q3] * A3, rA);
-    }
-}
-
-// Update_Primitive_Variables :2423-2445
-__global__ void mg_primitive_kernel(const BlockMeta *meta, const double *U, double *W, int64_t ncp) {
-    const BlockMeta m = meta[blockIdx.y];
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= m.ni * m.nj || m.skip) return;
-    const int64_t c = cell(m, q % m.ni + 2, q / m.ni + 2);
-    const PS<double> w = W_of_U(ldU(U, ncp, c));
-    W[c] = w.d; W[ncp + c] = w.vx; W[2 * ncp + c] = w.vy; W[3 * ncp + c] = w.p;
-}
-
-// Subtract_dUdt_from_P :2331-2352
-__global__ void mg_subtract_kernel(const BlockMeta *meta, double *P, const double *R, int64_t ncp) {
-    const BlockMeta m = meta[blockIdx.y];
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= m.ni * m.nj || m.skip) return;
-    const int64_t c = cell(m, q % m.ni + 2, q / m.ni + 2);
+        return rdiv(s[q0] * A0 + s[q1] * A1 + s[q2] * A2 + s[q3] * A3, rA);
+    };
+    const CS<double> u = {average(U, 0), average(U, 1), average(U, 2), average(U, 3)};
+    stU(Uc, ncpc, cc, u);
+    const PS<double> w = W_of_U(u);
+    Wc[cc] = w.d; Wc[ncpc + cc] = w.vx; Wc[2 * ncpc + cc] = w.vy; Wc[3 * ncpc + cc] = w.p;
+    if (R) {
 #pragma unroll
-    for (int v = 0; v < 4; ++v) P[v * ncp + c] -= R[v * ncp + c];
-}
-
-// CFL_Multigrid :2364-2407
-__global__ void mg_cfl_kernel(const BlockMeta *mf, const BlockMeta *mc, const double *dtf, const double *Af,
-                              double *dtc, const double *Ac) {
-    const BlockMeta f = mf[blockIdx.y], c = mc[blockIdx.y];
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= c.ni * c.nj || c.skip) return;
-    const int ic = q % c.ni + 2, jc = q / c.ni + 2;
-    const int i0 = 2 * (ic - 2) + 2, j0 = 2 * (jc - 2) + 2;
-    const int64_t sw = cell(f, i0, j0), se = sw + 1, nw = sw + f.pitch, ne = nw + 1;
-    const int64_t cc = cell(c, ic, jc);
-    const double A = Ac[cc];
-    const double dt_NE = qsqrt(qdiv(A, Af[ne])) * dtf[ne];
-    const double dt_SE = qsqrt(qdiv(A, Af[se])) * dtf[se];
-    const double dt_NW = qsqrt(qdiv(A, Af[nw])) * dtf[nw];
-    const double dt_SW = qsqrt(qdiv(A, Af[sw])) * dtf[sw];
-    dtc[cc] = dmin(dtc[cc], dmin(dt_NE, dmin(dt_SE, dmin(dt_NW, dt_SW))));
+        for (int v = 0; v < 4; ++v) P[v * ncpc + cc] = average(R, v);
+    }
 }
 
 // Evaluate_Solution_Changes :2454-2478 over every cell of each block,
@@ -109,26 +81,6 @@ __global__ void mg_copy_kernel(const BlockMeta *meta, double *dst, const double 
     const int64_t c = cell(m, q % m.nci, q / m.nci);
 #pragma unroll
     for (int v = 0; v < 4; ++v) dst[v * ncp + c] = src[v * ncp + c];
-}
-
-// Neumann conditions on the coarse solution change before bilinear
-// prolongation (:1640-1669): ghost = interior next to constant-extrapolation
-// boundaries; one thread per boundary cell of the interior span
-__global__ void mg_neumann_kernel(const BlockMeta *meta, const int32_t *bc, double *U, int64_t ncp) {
-    const BlockMeta m = meta[blockIdx.y];
-    if (m.skip) return;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int32_t *bW = bc + m.bcoff, *bE = bW + m.ncj, *bS = bE + m.ncj, *bN = bS + m.nci;
-    if (t < m.nj) {
-        const int j = t + 2;
-        // E before W, as the reference loop does; the two never share a cell
-        if (bE[j] == 4001) stU(U, ncp, cell(m, m.ni + 2, j), ldU(U, ncp, cell(m, m.ni + 1, j)));
-        if (bW[j] == 4001) stU(U, ncp, cell(m, 1, j), ldU(U, ncp, cell(m, 2, j)));
-    } else if (t < m.nj + m.ni) {
-        const int i = t - m.nj + 2;
-        if (bS[i] == 4001) stU(U, ncp, cell(m, i, 1), ldU(U, ncp, cell(m, i, 2)));
-        if (bN[i] == 4001) stU(U, ncp, cell(m, i, m.nj + 2), ldU(U, ncp, cell(m, i, m.nj + 1)));
-    }
 }
 
 // Bilinear_Interpolation, CFD.h:1367-1416 (Zingg and Yarrow)
@@ -181,14 +133,19 @@ __constant__ int8_t kQuad[4][4][2] = {
 // first quadrilateral that contains it, and a cell none contains restarts
 // the coarse cell with injection from the SW fine cell (cells already
 // updated are updated again, as in the reference).  Updates that leave the
-// state unphysical are halved up to max_red times, then dropped.
+// state unphysical are halved up to max_red times, then dropped.  Wf (if not
+// null) takes the fine cells' W(U) (Update_Primitive_Variables).
+//
+// neumann: a ghost cell of the interior span next to a constant-extrapolation
+// boundary takes the adjacent interior change (:1640-1669).
 //
 // assign (Prolong_Solution_Blocks :1200-1625, full multigrid): Uc is the
 // coarse solution; the fine cells take it (same quadrilateral order and
 // injection fall-back), with neither Dirichlet injection nor reduction.
 __global__ void mg_prolong_kernel(const BlockMeta *mc, const BlockMeta *mf, const int32_t *bc, const double *Uc,
-                                  const double *gc, int64_t ncpc, double *Uf, const double *gf, int64_t ncpf,
-                                  int inj_dirichlet, int inj_always, int stability, int max_red, int assign) {
+                                  const double *gc, int64_t ncpc, double *Uf, double *Wf, const double *gf,
+                                  int64_t ncpf, int neumann, int inj_dirichlet, int inj_always, int stability,
+                                  int max_red, int assign) {
     const BlockMeta c = mc[blockIdx.y], f = mf[blockIdx.y];
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= c.ni * c.nj || c.skip) return;
@@ -196,6 +153,24 @@ __global__ void mg_prolong_kernel(const BlockMeta *mc, const BlockMeta *mf, cons
     const int i0 = 2 * (ic - 2) + 2, j0 = 2 * (jc - 2) + 2;
     const int32_t *bW = bc + c.bcoff, *bE = bW + c.ncj, *bS = bE + c.ncj, *bN = bS + c.nci;
     const CS<double> Ucc = ldU(Uc, ncpc, cell(c, ic, jc));
+    // the coarse change at (a, e)
+    auto change = [&](int a, int e) {
+        if (neumann) {
+            if (e >= 2 && e <= c.nj + 1) {
+                if (a == c.ni + 2 && bE[e] == 4001) a = c.ni + 1;
+                else if (a == 1 && bW[e] == 4001) a = 2;
+            } else if (a >= 2 && a <= c.ni + 1) {
+                if (e == 1 && bS[a] == 4001) e = 2;
+                else if (e == c.nj + 2 && bN[a] == 4001) e = c.nj + 1;
+            }
+        }
+        return ldU(Uc, ncpc, cell(c, a, e));
+    };
+    auto primitive = [&](int64_t fc, const CS<double> &u) {
+        if (!Wf) return;
+        const PS<double> w = W_of_U(u);
+        Wf[fc] = w.d; Wf[ncpf + fc] = w.vx; Wf[2 * ncpf + fc] = w.vy; Wf[3 * ncpf + fc] = w.p;
+    };
     const int fdi[4] = {0, 1, 1, 0}, fdj[4] = {0, 0, 1, 1};
     const bool dirichlet = (ic == 2 && bW[jc] == 11000) || (ic == c.ni + 1 && bE[jc] == 11000) ||
                            (jc == 2 && bS[ic] == 11000) || (jc == c.nj + 1 && bN[ic] == 11000);
@@ -205,6 +180,7 @@ __global__ void mg_prolong_kernel(const BlockMeta *mc, const BlockMeta *mf, cons
             CS<double> u = ldU(Uf, ncpf, fc);
             u.d += Ucc.d; u.mx += Ucc.mx; u.my += Ucc.my; u.E += Ucc.E;
             stU(Uf, ncpf, fc, u);
+            primitive(fc, u);
         }
         return;
     }
@@ -218,8 +194,8 @@ __global__ void mg_prolong_kernel(const BlockMeta *mc, const BlockMeta *mf, cons
             for (int t = 0; t < 4 && !ok; ++t) {
                 const int a = ic + kQuad[k][t][0], e = jc + kQuad[k][t][1];
                 const int64_t p1 = cell(c, a, e), p2 = p1 + c.pitch, p3 = p2 + 1, p4 = p1 + 1;
-                ok = bilinear(ldU(Uc, ncpc, p1), xc[p1], yc[p1], ldU(Uc, ncpc, p2), xc[p2], yc[p2], ldU(Uc, ncpc, p3),
-                              xc[p3], yc[p3], ldU(Uc, ncpc, p4), xc[p4], yc[p4], gf[GEO_XC * ncpf + fc],
+                ok = bilinear(change(a, e), xc[p1], yc[p1], change(a, e + 1), xc[p2], yc[p2], change(a + 1, e + 1),
+                              xc[p3], yc[p3], change(a + 1, e), xc[p4], yc[p4], gf[GEO_XC * ncpf + fc],
                               gf[GEO_YC * ncpf + fc], dU);
             }
             if (!ok) {
@@ -250,6 +226,7 @@ __global__ void mg_prolong_kernel(const BlockMeta *mc, const BlockMeta *mf, cons
         }
         u.d += dU.d; u.mx += dU.mx; u.my += dU.my; u.E += dU.E;
         stU(Uf, ncpf, fc, u);
+        primitive(fc, u);   // a restarted cell's last write is its final state
     }
 }
 
@@ -259,28 +236,11 @@ __global__ void mg_prolong_kernel(const BlockMeta *mc, const BlockMeta *mf, cons
 using namespace cffc;
 
 extern "C" hipError_t cffc_launch_mg_restrict(const BlockMeta *mf, const BlockMeta *mc, int nblk, int max_int_c,
-                                   const double *src, const double *Af, int64_t ncpf, double *dst, const double *Ac,
-                                   int64_t ncpc, hipStream_t st) {
+                                   const double *U, const double *R, const double *Af, int64_t ncpf, double *Uc,
+                                   double *Wc, double *P, const double *Ac, int64_t ncpc, hipStream_t st) {
     dim3 grid((max_int_c + 255) / 256, nblk);
-    hipLaunchKernelGGL(mg_restrict_kernel, grid, dim3(256), 0, st, mf, mc, src, Af, ncpf, dst, Ac, ncpc);
-    return hipGetLastError();
-}
-extern "C" hipError_t cffc_launch_mg_primitive(const BlockMeta *meta, int nblk, int max_int, const double *U, double *W,
-                                    int64_t ncp, hipStream_t st) {
-    dim3 grid((max_int + 255) / 256, nblk);
-    hipLaunchKernelGGL(mg_primitive_kernel, grid, dim3(256), 0, st, meta, U, W, ncp);
-    return hipGetLastError();
-}
-extern "C" hipError_t cffc_launch_mg_subtract(const BlockMeta *meta, int nblk, int max_int, double *P, const double *R,
-                                   int64_t ncp, hipStream_t st) {
-    dim3 grid((max_int + 255) / 256, nblk);
-    hipLaunchKernelGGL(mg_subtract_kernel, grid, dim3(256), 0, st, meta, P, R, ncp);
-    return hipGetLastError();
-}
-extern "C" hipError_t cffc_launch_mg_cfl(const BlockMeta *mf, const BlockMeta *mc, int nblk, int max_int_c, const double *dtf,
-                              const double *Af, double *dtc, const double *Ac, hipStream_t st) {
-    dim3 grid((max_int_c + 255) / 256, nblk);
-    hipLaunchKernelGGL(mg_cfl_kernel, grid, dim3(256), 0, st, mf, mc, dtf, Af, dtc, Ac);
+    hipLaunchKernelGGL(mg_restrict_kernel, grid, dim3(max_int_c <= 64 ? 64 : 256), 0, st, mf, mc, U, R, Af, ncpf, Uc,
+                       Wc, P, Ac, ncpc);
     return hipGetLastError();
 }
 extern "C" hipError_t cffc_launch_mg_changes(const BlockMeta *meta, int nblk, int max_cells, double *U,
@@ -293,13 +253,13 @@ extern "C" hipError_t cffc_launch_mg_copy(const BlockMeta *meta, int nblk, int m
     hipLaunchKernelGGL(mg_copy_kernel, dim3((max_cells + 255) / 256, nblk), dim3(256), 0, st, meta, dst, src, ncp);
     return hipGetLastError();
 }
-extern "C" hipError_t cffc_launch_mg_prolong(const BlockMeta *mc, const BlockMeta *mf, int nblk, int max_int_c, int max_edge_c,
-                                  const int32_t *bc, double *Uc, const double *gc, int64_t ncpc, double *Uf,
-                                  const double *gf, int64_t ncpf, int neumann, int inj_dirichlet, int inj_always,
-                                  int stability, int max_red, int assign, hipStream_t st) {
-    if (neumann)
-        hipLaunchKernelGGL(mg_neumann_kernel, dim3((max_edge_c + 255) / 256, nblk), dim3(256), 0, st, mc, bc, Uc, ncpc);
-    hipLaunchKernelGGL(mg_prolong_kernel, dim3((max_int_c + 255) / 256, nblk), dim3(256), 0, st, mc, mf, bc, Uc, gc,
-                       ncpc, Uf, gf, ncpf, inj_dirichlet, inj_always, stability, max_red, assign);
+extern "C" hipError_t cffc_launch_mg_prolong(const BlockMeta *mc, const BlockMeta *mf, int nblk, int max_int_c,
+                                  const int32_t *bc, const double *Uc, const double *gc, int64_t ncpc, double *Uf,
+                                  double *Wf, const double *gf, int64_t ncpf, int neumann, int inj_dirichlet,
+                                  int inj_always, int stability, int max_red, int assign, hipStream_t st) {
+    // one thread per coarse cell, in the smallest workgroup that holds a block's
+    const int nt = max_int_c <= 64 ? 64 : max_int_c <= 128 ? 128 : 256;
+    hipLaunchKernelGGL(mg_prolong_kernel, dim3((max_int_c + nt - 1) / nt, nblk), dim3(nt), 0, st, mc, mf, bc, Uc, gc,
+                       ncpc, Uf, Wf, gf, ncpf, neumann, inj_dirichlet, inj_always, stability, max_red, assign);
     return hipGetLastError();
 }

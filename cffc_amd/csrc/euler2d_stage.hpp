@@ -76,6 +76,10 @@ struct StageParams {
     int32_t hlle;           // HLLE flux instead of Roe
     int32_t residual;       // steady residual (F*l)/A, no CFL*dt factor (dUdt_Residual_Evaluation)
     const double *P;        // forcing term added after the fluxes: +(CFL*dt)*P, or +P with residual
+    double *Psub;           // residual: also P -= R here (Subtract_dUdt_from_P), or null
+    double *Uo;             // one multistage step of a multigrid level: U at its start, written at stage 1
+    int32_t first_stage, halve;   // ... stage 1; halve unphysical updates (local time stepping)
+    int32_t pull;           // ... form the window's ghost cells (0: those in Win are current)
     int32_t axisym;         // axisymmetric source (CFL*dt)*S(W, Xc) after the east face
 };
 
@@ -232,14 +236,17 @@ enum StageKind {
     SK_WINDOW = 3,     // the same, physical ghosts formed in the tile's window
     SK_LEVELS = 4,     // SK_PLAIN with resolution changes
     SK_MG = 5,         // granular: one level, planar, Venkatakrishnan, Roe
-    SK_MG_FIRST = 6    // granular multigrid stage of a first-order level: zero limiter, so no reconstruction
+    SK_MG_FIRST = 6,   // granular multigrid stage of a first-order level: zero limiter, so no reconstruction
+    SK_STEP = 7,       // SK_MG with its ghost cells and its update: one launch per smoothing stage
+    SK_STEP_FIRST = 8  // the same on a first-order level
 };
 template <int K> struct StageOpt {
     static constexpr bool fused = K == SK_FUSED || K == SK_PLAIN || K == SK_WINDOW || K == SK_LEVELS;
     static constexpr bool general = K == SK_GRANULAR || K == SK_FUSED;   // axisymmetric, any limiter
     static constexpr bool amr = general || K == SK_LEVELS;
-    static constexpr bool window = K == SK_FUSED || K == SK_WINDOW;
-    static constexpr bool first = K == SK_MG_FIRST;
+    static constexpr bool step = K == SK_STEP || K == SK_STEP_FIRST;
+    static constexpr bool window = K == SK_FUSED || K == SK_WINDOW || step;
+    static constexpr bool first = K == SK_MG_FIRST || K == SK_STEP_FIRST;
 };
 // the leanest kernel that has every option of the launch
 inline int stage_kind(const StageParams &p, int fused) {
@@ -251,6 +258,33 @@ inline int stage_kind(const StageParams &p, int fused) {
     if (p.axisym || p.eflux || p.mode == GINIT_RK4) return SK_GRANULAR;
     if (p.hlle) return p.limiter == 0 && p.phi_mode != PHI_LOAD ? SK_MG_FIRST : SK_GRANULAR;
     return venkat ? SK_MG : SK_GRANULAR;
+}
+
+// Same-level ghost cells of a tile's window, read from the neighbours' W in
+// place of this block's own ghost cells; the thread that loaded a window cell
+// replaces it.  The stage reads one W buffer and writes the other, so
+// neighbours that have already been updated in this launch are not seen; and W
+// is the previous stage's W(U), the value that the exchange kernel would copy.
+template <int LJ, int LI>
+__device__ __forceinline__ void pull_ghosts(const StageParams &p, const BlockMeta &m, int b, int pi0, int pj0, int tid,
+                                            int nt, double (&sW)[4][LJ][LI]) {
+    const int ICu = m.ni + 1, JCu = m.nj + 1;
+    if (pi0 > 0 && pj0 > 0 && pi0 + LI <= ICu + 1 && pj0 + LJ <= JCu + 1) return;   // uniform over the workgroup
+    const int64_t ncp = p.ncp;
+    for (int q = tid; q < LI * LJ; q += nt) {
+        const int il = q % LI, jl = q / LI, ip = pi0 + il, jp = pj0 + jl;
+        const int di = ip < 2 ? -1 : ip > ICu ? 1 : 0, dj = jp < 2 ? -1 : jp > JCu ? 1 : 0;
+        if ((di == 0 && dj == 0) || ip >= m.nci || jp >= m.ncj) continue;
+        // slots N, S, E, W, NE, NW, SE, SW
+        const int slot = di == 0 ? (dj > 0 ? 0 : 1) : dj == 0 ? (di > 0 ? 2 : 3) : (dj > 0 ? 4 : 6) + (di > 0 ? 0 : 1);
+        const int nb = p.nbr[8 * b + slot];
+        if (nb < 0) continue;
+        const BlockMeta S = p.meta[nb];
+        const int is = di > 0 ? ip - m.ni : di < 0 ? ip + S.ni : ip, js = dj > 0 ? jp - m.nj : dj < 0 ? jp + S.nj : jp;
+        const int64_t c = S.coff + (int64_t)js * S.pitch + is;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sW[v][jl][il] = p.Win[v * ncp + c];
+    }
 }
 
 // Least-squares gradient and Venkatakrishnan limiter of one cell
@@ -506,6 +540,43 @@ __device__ __forceinline__ void fused_update(const StageParams &p, const BlockGe
     }
 }
 
+// The update of one smoothing stage of a multigrid level (update_kernel's rule:
+// U = Uo + omega dUdt, halved with the time step up to 10 times where it is
+// unphysical).  Wc: the stage's W, which a cell that stays unphysical keeps.
+__device__ __forceinline__ void mg_update(const StageParams &p, const TileDesc &t, int64_t org, uint32_t o8, int ip,
+                                          int jp, double dtc, const double (&U0)[4], double (&dU)[4],
+                                          const PS<double> &Wc) {
+    const int64_t ncp = p.ncp;
+    const double om = p.omega;
+    CS<double> Un = {U0[0] + om * dU[0], U0[1] + om * dU[1], U0[2] + om * dU[2], U0[3] + om * dU[3]};
+    bool bad = positivity_fails<double>(Un);
+    if (__builtin_expect(bad && p.halve, 0)) {
+        double f = 1.0, dtl = dtc;
+        for (int n = 1; n <= 10; ++n) {
+            f = 0.5 * f;
+            dtl = f * dtl;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) dU[v] = f * dU[v];
+            Un = {U0[0] + om * dU[0], U0[1] + om * dU[1], U0[2] + om * dU[2], U0[3] + om * dU[3]};
+            if (!positivity_fails<double>(Un)) break;
+        }
+        at(p.dt + org, o8) = dtl;
+        bad = positivity_fails<double>(Un);
+    }
+    double *Ub = p.U + org;
+    at(Ub, o8) = Un.d; at(Ub + ncp, o8) = Un.mx; at(Ub + 2 * ncp, o8) = Un.my; at(Ub + 3 * ncp, o8) = Un.E;
+    if (p.first_stage) {
+        double *Uob = p.Uo + org;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) at(Uob + v * ncp, o8) = U0[v];
+    }
+    if (__builtin_expect(bad, 0))
+        atomicMin(p.err, ((unsigned long long)t.b << 32) | ((unsigned long long)jp << 16) | (unsigned long long)ip);
+    const PS<double> Wn = bad ? Wc : W_of_U(Un);
+    double *Wb = p.Wout + org;
+    at(Wb, o8) = Wn.d; at(Wb + ncp, o8) = Wn.vx; at(Wb + 2 * ncp, o8) = Wn.vy; at(Wb + 3 * ncp, o8) = Wn.p;
+}
+
 // Physical ghost states of a tile's window (BCs, Euler2DQuadSingleBlock.cc:
 // 2354-3010), formed in LDS from the window's own cells: both ghost layers
 // copy, mirror or replace the two cells next to the boundary, which a window
@@ -674,7 +745,8 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
         }
         phim = ps == PART_FROZEN ? PHI_LOAD : p.last_stage ? PHI_COMPUTE_STORE : PHI_COMPUTE;
     }
-    if (!FUSED && p.part_frozen) phim = p.part_frozen[p.part_of_block[t.b]] ? PHI_LOAD : PHI_COMPUTE_STORE;
+    if (!FUSED && p.part_frozen)
+        phim = p.part_frozen[p.part_of_block[t.b]] ? PHI_LOAD : O::step ? PHI_COMPUTE : PHI_COMPUTE_STORE;
     const int ICu = m.ni + 1, JCu = m.nj + 1;
     const int pi0 = t.i0, pj0 = t.j0;   // padded index of the LDS window origin
     // the update waits (in update_tile_kernel) for residual smoothing, or
@@ -727,6 +799,8 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
         }
 #pragma unroll
         for (int k = 0; k < NIT; ++k) {
+            // a ghost cell that pull_ghosts replaces is written by its own thread only
+            if (O::step && tid + k * NT >= NWIN) continue;
             const int il = slot[k] % LI, jl = slot[k] / LI;
 #pragma unroll
             for (int v = 0; v < 4; ++v) sW[v][jl][il] = wv[k][v];
@@ -749,7 +823,10 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
             }
         }
     }
-    if (O::window && p.window_bcs && m.has_bc) window_ghosts<FT, LJ, LI>(p, m, pi0, pj0, tid, NT, sW);
+    if constexpr (O::step) {
+        if (p.pull) pull_ghosts<LJ, LI>(p, m, t.b, pi0, pj0, tid, NT, sW);
+    }
+    if (O::window && (O::step ? p.pull : p.window_bcs) && m.has_bc) window_ghosts<FT, LJ, LI>(p, m, pi0, pj0, tid, NT, sW);
     __syncthreads();
 
     // ---- phase 2: least-squares reconstruction + limiter -------------------
@@ -963,6 +1040,11 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
 #pragma unroll
             for (int v = 0; v < 4; ++v) U4[v] = at(p.U + v * ncp + org, o8);
         }
+        if constexpr (O::step) {
+            const double *U0 = (p.first_stage ? p.U : p.Uo) + org;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) U4[v] = at(U0 + v * ncp, o8);
+        }
         if (readS) {
 #pragma unroll
             for (int v = 0; v < 4; ++v) S4[v] = at(p.S + v * ncp + org, o8);
@@ -999,7 +1081,7 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
                 for (int v = 0; v < 4; ++v) dU[v] = 0.0;
             }
         } else {
-            if (p.mode == GINIT_KEEP) {
+            if (!O::step && p.mode == GINIT_KEEP) {
 #pragma unroll
                 for (int v = 0; v < 4; ++v) dU[v] = at(p.S + v * ncp + org, o8);
             } else if (KIND == SK_GRANULAR && p.mode == GINIT_RK4) {
@@ -1114,11 +1196,19 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
                 for (int v = 0; v < 4; ++v) e[v] = (-(double)fW(v)) * lW;
             }
         }
-        if (!FUSED || defer) {
+        if constexpr (O::step) {
+            mg_update(p, t, org, o8, ip, jp, dtc, U4, dU,
+                      PS<double>{sW[0][tr + 2][tc + 2], sW[1][tr + 2][tc + 2], sW[2][tr + 2][tc + 2],
+                                 sW[3][tr + 2][tc + 2]});
+        } else if (!FUSED || defer) {
             // granular residual, or a correction / smoothing follows: store dUdt
             double *Sx = FUSED ? p.Sd : p.S;
 #pragma unroll
             for (int v = 0; v < 4; ++v) at(Sx + v * ncp + org, o8) = dU[v];
+            if (!FUSED && p.Psub) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) at(p.Psub + v * ncp + org, o8) -= dU[v];
+            }
         } else {
             fused_update<FT, O>(p, geo, m, t, org, o8, ip, jp, A, dtc, lW, lE, lS, lN, U4, readS, S4, dU, l1, l2, mx, dtn);
         }
