@@ -883,6 +883,16 @@ extern "C" int cffc_create(const cffc_mesh_desc *md, const cffc_scheme_desc *sd,
         bool windowed = sym && !c->amr;
         for (const BlockMeta &m : c->meta_h) windowed = windowed && m.ni >= 2 && m.nj >= 2;
         for (int32_t q = 0; q < bcoff; ++q) windowed = windowed && md->bc[q] != CFFC_BC_PERIODIC;
+        // every face of a block is a neighbour's or a boundary (else its ghost
+        // cells are whatever the caller left in the one buffer)
+        for (int b = 0; b < md->nblk; ++b) {
+            const BlockMeta &m = c->meta_h[b];
+            const int32_t *w = md->bc + m.bcoff, *e = w + m.ncj, *so = e + m.ncj, *no = so + m.nci;
+            for (int j = 2; j <= m.nj + 1; ++j)
+                windowed = windowed && (w[j] || same[8 * b + 3] >= 0) && (e[j] || same[8 * b + 2] >= 0);
+            for (int i = 2; i <= m.ni + 1; ++i)
+                windowed = windowed && (so[i] || same[8 * b + 1] >= 0) && (no[i] || same[8 * b] >= 0);
+        }
         // The window's ghosts cost the FP64 kernel 2% of its rate, the saved
         // launch 5 to 9 us a stage: per RK4 step 0.139 against 0.160 ms at
         // 262 k cells, 0.820 against 0.824 at 2.0 M, 1.634 against 1.603 at
@@ -2107,8 +2117,17 @@ extern "C" int cffc_kernel_times(cffc_ctx *c, double out[4]) {
 // forcing term folded into that kernel after the face fluxes, and the level
 // transfers of euler2d_mg.hip.  Per-cell dt on every level (Smooth's CFL call
 // does not apply the global minimum).
+// cell lists of a first-order level (FirstArgs), null where it has none
+struct FirstLevel {
+    MgCell *cells = nullptr;
+    int4 *nb = nullptr, *local = nullptr;
+    int32_t *group0 = nullptr;
+    int n = 0, ngroup = 0, max_group = 0;
+};
+
 struct cffc_mg {
     std::vector<cffc_ctx *> lv;
+    std::vector<FirstLevel> first;
     cffc_mg_desc d{};
     std::vector<double *> P, uo;     // per level (P unused on level 0)
     std::vector<double> Ahost;       // scratch: fine-level areas for the Wo restriction
@@ -2160,6 +2179,9 @@ static void mg_free(cffc_mg *mg) {
         if (q) (void)hipFree(q);
     if (mg->d_part_l2) (void)hipHostFree(mg->d_part_l2);
     if (mg->status) (void)hipHostFree(mg->status);
+    for (FirstLevel &f : mg->first)
+        for (void *q : {(void *)f.cells, (void *)f.nb, (void *)f.local, (void *)f.group0})
+            if (q) (void)hipFree(q);
     if (mg->gexec) (void)hipGraphExecDestroy(mg->gexec);
     if (mg->graph) (void)hipGraphDestroy(mg->graph);
     for (size_t l = 0; l < mg->lv.size(); ++l) {
@@ -2177,6 +2199,94 @@ extern "C" void cffc_mg_destroy(cffc_mg *mg) { mg_free(mg); }
 extern "C" cffc_ctx *cffc_mg_level(cffc_mg *mg, int level) {
     if (!mg || level < 0 || level >= (int)mg->lv.size()) return nullptr;
     return mg->lv[level];
+}
+
+// The cell list of one level, its blocks in connected groups: neighbours across
+// blocks as the exchange fills ghost cells, boundaries as the BCs overwrite them.
+static int mg_first_level(const cffc_ctx *c, const cffc_mesh_desc *md, FirstLevel &f) {
+    if (!c->windowable || md->lattice || c->ncp > 0x7fffffff) return 0;
+    const int nb = c->nblk;
+    std::vector<int> root(nb);
+    for (int b = 0; b < nb; ++b) root[b] = b;
+    auto find = [&](int b) {
+        while (root[b] != b) b = root[b] = root[root[b]];
+        return b;
+    };
+    for (int b = 0; b < nb; ++b)
+        for (int s = 0; s < 8; ++s) {
+            const int o = md->nbr[8 * (size_t)b + s];
+            if (o >= 0) root[find(b)] = find(o);
+        }
+    std::vector<std::vector<int>> groups;
+    std::vector<int> gid(nb, -1);
+    for (int b = 0; b < nb; ++b) {
+        int &g = gid[find(b)];
+        if (g < 0) {
+            g = (int)groups.size();
+            groups.emplace_back();
+        }
+        groups[g].push_back(b);
+    }
+    std::vector<MgCell> cells;
+    std::vector<int32_t> group0, first(nb);   // first: a block's first cell in the list
+    int max_group = 0;
+    for (const auto &g : groups) {
+        group0.push_back((int32_t)cells.size());
+        for (int b : g) {
+            const BlockMeta &m = c->meta_h[b];
+            first[b] = (int32_t)cells.size();
+            for (int j = 2; j <= m.nj + 1; ++j)
+                for (int i = 2; i <= m.ni + 1; ++i) {
+                    const int32_t q = (int32_t)(m.coff + (int64_t)j * m.pitch + i);
+                    cells.push_back(MgCell{q, q - m.pitch, b, (j << 16) | i});
+                }
+        }
+        max_group = std::max(max_group, (int)cells.size() - group0.back());
+    }
+    group0.push_back((int32_t)cells.size());
+    std::vector<int4> nbs(cells.size()), loc(cells.size());
+    for (size_t q = 0; q < cells.size(); ++q) {
+        const int b = cells[q].blk, i = cells[q].ji & 0xFFFF, j = cells[q].ji >> 16;
+        const BlockMeta &m = c->meta_h[b];
+        const int g0 = group0[gid[find(b)]];
+        int nv[4], lv[4];
+        // W, E, S, N: block face slot, boundary entry, neighbouring cell
+        const int di[4] = {-1, 1, 0, 0}, dj[4] = {0, 0, -1, 1}, slot[4] = {3, 2, 1, 0};
+        const int entry[4] = {j, m.ncj + j, 2 * m.ncj + i, 2 * m.ncj + m.nci + i};
+        for (int s = 0; s < 4; ++s) {
+            const int in = i + di[s], jn = j + dj[s];
+            const bool inside = in >= 2 && in <= m.ni + 1 && jn >= 2 && jn <= m.nj + 1;
+            const int e = m.bcoff + entry[s], o = md->nbr[8 * (size_t)b + slot[s]];
+            lv[s] = -1;
+            if (inside) {
+                nv[s] = (int32_t)(m.coff + (int64_t)jn * m.pitch + in);
+                lv[s] = first[b] + (jn - 2) * m.ni + (in - 2) - g0;
+            } else if (md->bc[e] != 0) {
+                nv[s] = -(e + 1);
+            } else {
+                const BlockMeta &S = c->meta_h[o];   // windowable: there is one
+                const int is = s == 0 ? S.ni + 1 : s == 1 ? 2 : in, js = s == 2 ? S.nj + 1 : s == 3 ? 2 : jn;
+                nv[s] = (int32_t)(S.coff + (int64_t)js * S.pitch + is);
+                lv[s] = first[o] + (js - 2) * S.ni + (is - 2) - g0;
+            }
+        }
+        nbs[q] = make_int4(nv[0], nv[1], nv[2], nv[3]);
+        loc[q] = make_int4(lv[0], lv[1], lv[2], lv[3]);
+    }
+    if (int e = dalloc(&f.cells, cells.size())) return e;
+    if (int e = dalloc(&f.nb, nbs.size())) return e;
+    HIPCHK(hipMemcpy(f.cells, cells.data(), cells.size() * sizeof(MgCell), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(f.nb, nbs.data(), nbs.size() * sizeof(int4), hipMemcpyHostToDevice));
+    f.n = (int)cells.size();
+    if (max_group <= 1024) {
+        if (int e = dalloc(&f.local, loc.size())) return e;
+        if (int e = dalloc(&f.group0, group0.size())) return e;
+        HIPCHK(hipMemcpy(f.local, loc.data(), loc.size() * sizeof(int4), hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy(f.group0, group0.data(), group0.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+        f.ngroup = (int)groups.size();
+        f.max_group = max_group;
+    }
+    return 0;
 }
 
 extern "C" int cffc_mg_create(const cffc_mesh_desc *levels, int nlevels, const cffc_scheme_desc *smoother,
@@ -2214,6 +2324,7 @@ extern "C" int cffc_mg_create(const cffc_mesh_desc *levels, int nlevels, const c
     }
     mg->lv.assign(nlevels, nullptr);
     mg->P.assign(nlevels, nullptr);
+    mg->first.resize(nlevels);
     mg->uo.assign(nlevels, nullptr);
     for (int l = 0; l < nlevels; ++l) {
         if (int e = cffc_create(&levels[l], smoother, &mg->lv[l])) {
@@ -2228,6 +2339,10 @@ extern "C" int cffc_mg_create(const cffc_mesh_desc *levels, int nlevels, const c
         }
         int e;
         if ((e = ensure_granular(c)) || (e = ensure_phi(c))) {
+            mg_free(mg);
+            return e;
+        }
+        if (l > 0 && d->first_order_coarse && (e = mg_first_level(c, &levels[l], mg->first[l]))) {
             mg_free(mg);
             return e;
         }
@@ -2275,7 +2390,8 @@ static int mg_exchange(cffc_ctx *c) {
 
 // one granular FP64 stage kernel: a smoothing stage (residual = 0) or
 // dUdt_Residual_Evaluation into dUdt[0] (residual = 1); P: forcing term or null
-static int mg_stage(cffc_ctx *c, int i_stage, int residual, const double *P, double *Psub = nullptr) {
+static int mg_stage(cffc_ctx *c, int i_stage, int residual, const double *P, double *Psub = nullptr,
+                    bool pull = false) {
     StageParams p = base_stage_params(c);
     p.Win = c->W[c->wcur];
     p.Wout = c->W[c->wcur];
@@ -2293,6 +2409,7 @@ static int mg_stage(cffc_ctx *c, int i_stage, int residual, const double *P, dou
     p.residual = residual;
     p.P = P;
     p.Psub = Psub;
+    p.pull = pull;
     HIPCHK(cffc_launch_stage_fp64(&p, c->ti, c->tj, 0, c->stream));
     return 0;
 }
@@ -2333,23 +2450,67 @@ static int mg_step(cffc_ctx *c, int i_stage, int pull, const double *P) {
     return 0;
 }
 
+// n smoothings of a first-order level over its cell list: one launch for all
+// of them where its groups fit a workgroup, else one per stage after the CFL
+static int mg_smooth_first(cffc_mg *mg, int top, int l, int n, const double *P) {
+    cffc_ctx *c = mg->lv[l];
+    const FirstLevel &fl = mg->first[l];
+    const cffc_ctx *f = l > top ? mg->lv[l - 1] : nullptr;
+    FirstArgs a = {};
+    a.meta = c->meta;
+    a.cells = fl.cells;
+    a.nb = fl.nb;
+    a.n = fl.n;
+    a.geom = c->geom;
+    a.ncp = c->ncp;
+    a.bc = c->bc;
+    a.wo = c->wo;
+    a.U = c->U;
+    a.Uo = c->Uo;
+    a.dt = c->dt;
+    a.P = P;
+    a.cfl = c->s.cfl_number;
+    a.nstage = c->s.n_stage;
+    for (int st = 1; st <= c->s.n_stage; ++st) a.omega[st - 1] = stage_omega(c->s, st);
+    a.halve = c->s.local_time_stepping == CFFC_SCALAR_LOCAL_TIME_STEPPING;
+    a.err = c->scal + 2;
+    if (fl.ngroup) {
+        a.Win = c->W[c->wcur];
+        a.Wout = c->W[c->wcur];
+        const FineLevel fine = {f ? f->meta : nullptr, f ? f->dt : nullptr, f ? area(f) : nullptr};
+        HIPCHK(cffc_launch_mg_first_smooth(&a, fl.ngroup, fl.max_group, fl.group0, fl.local, n, &fine, c->stream));
+        return 0;
+    }
+    for (int nu = 0; nu < n; ++nu) {
+        HIPCHK(cffc_launch_cfl(c->meta, c->tiles, c->ntiles, c->ti, c->tj, c->W[c->wcur], c->geom, c->ncp, c->dt,
+                               nullptr, f ? f->meta : nullptr, f ? f->dt : nullptr, f ? area(f) : nullptr, c->stream));
+        for (int st = 1; st <= c->s.n_stage; ++st) {
+            a.Win = c->W[c->wcur];
+            a.Wout = c->W[1 - c->wcur];
+            HIPCHK(cffc_launch_mg_first_step(&a, a.omega[st - 1], st == 1, c->stream));
+            c->wcur = 1 - c->wcur;
+        }
+    }
+    return 0;
+}
+
 // Smooth :2865-3110, n times.  Only the last one's closing exchange and
 // residual are evaluated: the next smoothing's stages replace both.
 static int mg_smooth(cffc_mg *mg, int top, int l, int n) {
     cffc_ctx *c = mg->lv[l];
     const double *P = l > top ? mg->P[l] : nullptr;
-    for (int nu = 0; nu < n; ++nu) {
+    const bool listed = mg->first[l].n && c->s.i_flux_function == CFFC_FLUX_FUNCTION_HLLE && mg_one_launch(mg, c);
+    if (listed && n > 0)
+        if (int e = mg_smooth_first(mg, top, l, n, P)) return e;
+    for (int nu = 0; nu < n && !listed; ++nu) {
         // local time steps only (the levels' stages read dt per cell): no
         // global minimum is formed
         const cffc_ctx *f = l > top ? mg->lv[l - 1] : nullptr;
         HIPCHK(cffc_launch_cfl(c->meta, c->tiles, c->ntiles, c->ti, c->tj, c->W[c->wcur], c->geom, c->ncp, c->dt,
                                nullptr, f ? f->meta : nullptr, f ? f->dt : nullptr, f ? area(f) : nullptr, c->stream));
         if (mg_one_launch(mg, c)) {
-            // Stage 1 of the first smoothing reads the ghosts that the exchange
-            // after the restriction or prolongation filled; the top level, whose
-            // state may have been set since, exchanges first (ghosts = W(U))
-            if (nu == 0 && l == top)
-                if (int e = mg_exchange(c)) return e;
+            // stage 1 of the first smoothing reads the ghosts that the exchange
+            // after the restriction or prolongation, or before the cycle, filled
             for (int st = 1; st <= c->s.n_stage; ++st)
                 if (int e = mg_step(c, st, nu > 0 || st > 1, P)) return e;
             continue;
@@ -2370,8 +2531,12 @@ static int mg_smooth(cffc_mg *mg, int top, int l, int n) {
         }
     }
     if (n == 0) return 0;
-    if (int e = mg_exchange(c)) return e;
-    if (int e = mg_stage(c, 1, 1, P)) return e;
+    // the coarse levels' ghost U takes part in the change they return; the top
+    // level's residual forms the ghosts it reads itself
+    const bool pull = l == top && mg_one_launch(mg, c);
+    if (!pull)
+        if (int e = mg_exchange(c)) return e;
+    if (int e = mg_stage(c, 1, 1, P, nullptr, pull)) return e;
     if (!c->freeze) c->phi_valid = 1;
     return 0;
 }
@@ -2394,6 +2559,7 @@ static int mg_cgc(cffc_mg *mg, int top, int l) {
     int e;
     if (l == L - 1) {
         if (l != top && (e = mg_store_uo(mg, l))) return e;
+        if (l == top && (e = mg_exchange(c))) return e;
         if ((e = mg_smooth(mg, top, l, d.smooths_on_coarsest_level))) return e;
     } else {
         cffc_ctx *cc = mg->lv[l + 1];
@@ -2533,6 +2699,7 @@ extern "C" int cffc_mg_cycle(cffc_mg *mg, int64_t *bad_cell) {
     mg_set_top(mg, 0);
     mg->base = mg->lv[0]->wcur;
     if (int e = mg_reset_errors(mg)) return e;
+    if (int e = mg_exchange(mg->lv[0])) return e;   // the state may be new
     if (int e = mg_cgc(mg, 0, 0)) return e;
     return mg_check_errors(mg, bad_cell);
 }
@@ -2710,6 +2877,7 @@ extern "C" int cffc_mg_execute(cffc_mg *mg, int max_cycles, double freeze_level,
             mg->frozen = false;
         }
         const long long ncyc = top != 0 ? mg->d.fmg_cycles : 0x7fffffffffffffffLL;
+        if (int e = mg_exchange(t)) return e;   // the cycles start from current ghosts; the state may be new
         double init_l2 = -1.0, ratio = -1.0;
         for (long long cycles = 1; cycles <= ncyc; ++cycles) {
             double nr[3];

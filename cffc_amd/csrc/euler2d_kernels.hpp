@@ -74,6 +74,35 @@ struct ErrorKeys {
     int n;
 };
 
+// A first-order multigrid level as a list of its interior cells: padded cell,
+// the cell to its south, block, (j << 16) | i; and per cell its W, E, S, N
+// neighbours (nb): a padded cell, or -(e + 1) for boundary entry e of the bc / wo
+// arrays.
+struct MgCell {
+    int32_t c, south, blk, ji;
+};
+struct FirstArgs {
+    const BlockMeta *meta;
+    const MgCell *cells;
+    const int4 *nb;
+    int32_t n;
+    const double *geom;
+    int64_t ncp;
+    const int32_t *bc;
+    const double *wo;
+    const double *Win;
+    double *Wout, *U, *Uo, *dt;
+    const double *P;            // forcing term, or null
+    double cfl, omega[5];
+    int32_t nstage, halve;
+    unsigned long long *err;
+};
+// the next finer level, for CFL_Multigrid (meta null: none)
+struct FineLevel {
+    const BlockMeta *meta;
+    const double *dt, *A;
+};
+
 }  // namespace cffc
 
 // tile shapes the stage kernel is instantiated for (TI x TJ interior cells)
@@ -140,6 +169,11 @@ hipError_t cffc_launch_mg_changes(const cffc::BlockMeta *meta, int nblk, int max
                                   int64_t ncp, hipStream_t st);
 hipError_t cffc_launch_mg_copy(const cffc::BlockMeta *meta, int nblk, int max_cells, double *dst, const double *src,
                                int64_t ncp, hipStream_t st);
+hipError_t cffc_launch_mg_first_step(const cffc::FirstArgs *a, double omega, int first_stage, hipStream_t st);
+// group0: first cell of every group of connected blocks; local: the neighbours'
+// places in their group, or -1
+hipError_t cffc_launch_mg_first_smooth(const cffc::FirstArgs *a, int ngroup, int max_group, const int32_t *group0,
+                                       const int4 *local, int nsm, const cffc::FineLevel *fl, hipStream_t st);
 hipError_t cffc_launch_mg_prolong(const cffc::BlockMeta *mc, const cffc::BlockMeta *mf, int nblk, int max_int_c,
                                   const int32_t *bc, const double *Uc, const double *gc, int64_t ncpc, double *Uf,
                                   double *Wf, const double *gf, int64_t ncpf, int neumann, int inj_dirichlet,

@@ -230,6 +230,188 @@ __global__ void mg_prolong_kernel(const BlockMeta *mc, const BlockMeta *mf, cons
     }
 }
 
+// ---------------------------------------------------------------------------
+// Smoothing of a first-order level (HLLE, zero limiter, so a face takes the
+// states of its two cells): a cell needs its four neighbours and nothing else,
+// which the host lists per cell across blocks.  No window, no LDS, no ghost cells,
+// two dependent loads to the states; the price is that both cells of a face
+// evaluate its flux.  The launches of the coarse levels are bound by that load
+// chain (a 12,288-cell case: 9.6 us a stage with windows, whatever the level).
+struct FirstCell {
+    PS<double> W;
+    double A, lW, lE, lS, lN, nWx, nWy, nEx, nEy, nSx, nSy, nNx, nNy;
+};
+__device__ __forceinline__ void load_geometry(const FirstArgs &a, const MgCell &k, FirstCell &f) {
+    const double *G = a.geom;
+    const int64_t n = a.ncp, c = k.c, w = k.c - 1, s = k.south;
+    f.A = G[GEO_A * n + c];
+    f.lW = G[GEO_LE * n + w]; f.lE = G[GEO_LE * n + c]; f.lS = G[GEO_LN * n + s]; f.lN = G[GEO_LN * n + c];
+    f.nWx = G[GEO_NEX * n + w]; f.nWy = G[GEO_NEY * n + w]; f.nEx = G[GEO_NEX * n + c]; f.nEy = G[GEO_NEY * n + c];
+    f.nSx = G[GEO_NNX * n + s]; f.nSy = G[GEO_NNY * n + s]; f.nNx = G[GEO_NNX * n + c]; f.nNy = G[GEO_NNY * n + c];
+}
+// flux through the face to neighbour state Wn, or to the boundary entry -(nb + 1)
+// of the bc / wo arrays; (nx, ny): the face's normal (E or N of its low cell), low:
+// this cell is on the high side
+__device__ __forceinline__ CS<double> first_flux(const FirstArgs &a, const PS<double> &Wc, PS<double> Wn, int nb, bool low,
+                                                 double nx, double ny) {
+    if (nb < 0) {
+        const int e = -(nb + 1), t = a.bc[e];
+        const PS<double> wo = {a.wo[4 * (int64_t)e], a.wo[4 * (int64_t)e + 1], a.wo[4 * (int64_t)e + 2],
+                               a.wo[4 * (int64_t)e + 3]};
+        const double sg = low ? -1.0 : 1.0;   // outward
+        if (t == 7001) Wn = reflect(Wc, sg * nx, sg * ny);
+        else if (t == 8001) Wn = bc_characteristic_pressure(Wc, wo, sg * nx, sg * ny);
+        else if (t == 11000) Wn = wo;
+        else Wn = Wc;
+    }
+    return low ? flux_hlle_n(Wn, Wc, nx, ny) : flux_hlle_n(Wc, Wn, nx, ny);
+}
+// (CFL dt)(+W -E +S -N)/A + (CFL dt) P, in the stage kernel's order
+template <typename State>
+__device__ __forceinline__ void first_residual(const FirstArgs &a, const FirstCell &f, const int (&nb)[4], double cdt,
+                                               const double (&P)[4], State state, double (&dU)[4]) {
+    const Recip<double> rA = recip(f.A);
+    CS<double> F = first_flux(a, f.W, state(0), nb[0], true, f.nWx, f.nWy);
+    dU[0] = 0.0 + rdivf(cdt * F.d * f.lW, rA); dU[1] = 0.0 + rdivf(cdt * F.mx * f.lW, rA);
+    dU[2] = 0.0 + rdivf(cdt * F.my * f.lW, rA); dU[3] = 0.0 + rdivf(cdt * F.E * f.lW, rA);
+    F = first_flux(a, f.W, state(1), nb[1], false, f.nEx, f.nEy);
+    dU[0] -= rdivf(cdt * F.d * f.lE, rA); dU[1] -= rdivf(cdt * F.mx * f.lE, rA);
+    dU[2] -= rdivf(cdt * F.my * f.lE, rA); dU[3] -= rdivf(cdt * F.E * f.lE, rA);
+    F = first_flux(a, f.W, state(2), nb[2], true, f.nSx, f.nSy);
+    dU[0] += rdivf(cdt * F.d * f.lS, rA); dU[1] += rdivf(cdt * F.mx * f.lS, rA);
+    dU[2] += rdivf(cdt * F.my * f.lS, rA); dU[3] += rdivf(cdt * F.E * f.lS, rA);
+    F = first_flux(a, f.W, state(3), nb[3], false, f.nNx, f.nNy);
+    dU[0] -= rdivf(cdt * F.d * f.lN, rA); dU[1] -= rdivf(cdt * F.mx * f.lN, rA);
+    dU[2] -= rdivf(cdt * F.my * f.lN, rA); dU[3] -= rdivf(cdt * F.E * f.lN, rA);
+    if (a.P) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) dU[v] += cdt * P[v];
+    }
+}
+// update_kernel's rule; returns W^(s+1), Wc where the state stays unphysical
+__device__ __forceinline__ PS<double> first_update(const FirstArgs &a, const MgCell &k, const CS<double> &U0, double om,
+                                                   const PS<double> &Wc, double &dtl, double (&dU)[4], CS<double> &Un) {
+    Un = {U0.d + om * dU[0], U0.mx + om * dU[1], U0.my + om * dU[2], U0.E + om * dU[3]};
+    bool bad = unphysical(Un);
+    if (bad && a.halve) {
+        double f = 1.0;
+        for (int n = 1; n <= 10; ++n) {
+            f = 0.5 * f;
+            dtl = f * dtl;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) dU[v] = f * dU[v];
+            Un = {U0.d + om * dU[0], U0.mx + om * dU[1], U0.my + om * dU[2], U0.E + om * dU[3]};
+            if (!unphysical(Un)) break;
+        }
+        bad = unphysical(Un);
+    }
+    if (bad) atomicMin(a.err, ((unsigned long long)(unsigned)k.blk << 32) | (unsigned long long)(unsigned)k.ji);
+    return bad ? Wc : W_of_U(Un);
+}
+__device__ __forceinline__ PS<double> ldW4(const double *W, int64_t ncp, int64_t c) {
+    return {W[c], W[ncp + c], W[2 * ncp + c], W[3 * ncp + c]};
+}
+
+// one smoothing stage of a level, one thread per cell, from Win to Wout
+__global__ __launch_bounds__(256) void mg_first_step_kernel(FirstArgs a, double om, int first_stage) {
+    const int q = blockIdx.x * 256 + threadIdx.x;
+    if (q >= a.n) return;
+    const MgCell k = a.cells[q];
+    if (a.meta[k.blk].skip) return;
+    const int4 n4 = a.nb[q];
+    const int nb[4] = {n4.x, n4.y, n4.z, n4.w};
+    const int64_t ncp = a.ncp, c = k.c;
+    FirstCell f;
+    f.W = ldW4(a.Win, ncp, c);
+    PS<double> Wn[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) Wn[s] = ldW4(a.Win, ncp, nb[s] >= 0 ? nb[s] : k.c);
+    load_geometry(a, k, f);
+    const CS<double> U0 = ldU(first_stage ? a.U : a.Uo, ncp, c);
+    double P[4] = {0.0, 0.0, 0.0, 0.0}, dtl = a.dt[c], dU[4];
+    if (a.P) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) P[v] = a.P[v * ncp + c];
+    }
+    const double dt0 = dtl;
+    first_residual(a, f, nb, a.cfl * dtl, P, [&](int s) { return Wn[s]; }, dU);
+    CS<double> Un;
+    const PS<double> w = first_update(a, k, U0, om, f.W, dtl, dU, Un);
+    if (dtl != dt0) a.dt[c] = dtl;
+    stU(a.U, ncp, c, Un);
+    if (first_stage) stU(a.Uo, ncp, c, U0);
+    a.Wout[c] = w.d; a.Wout[ncp + c] = w.vx; a.Wout[2 * ncp + c] = w.vy; a.Wout[3 * ncp + c] = w.p;
+}
+
+// All smoothings of a level whose connected groups of blocks have at most 1,024
+// cells, in one launch: a workgroup per group, a thread per cell, W in LDS,
+// everything else of the cell in registers.  nsm smoothings of a.nstage stages;
+// each starts with the cell's CFL time step and the finer level's rule
+// (cfl_kernel).  18 launches of the coarsest level of a V cycle (3 smoothings)
+// become one.
+__global__ __launch_bounds__(1024) void mg_first_smooth_kernel(FirstArgs a, const int32_t *group0, const int4 *local,
+                                                               int nsm, FineLevel fl) {
+    __shared__ double sW[4][1024];
+    const int g0 = group0[blockIdx.x], n = group0[blockIdx.x + 1] - g0, t = threadIdx.x;
+    const bool on = t < n;
+    const int q = g0 + (on ? t : 0);
+    const MgCell k = a.cells[q];
+    if (a.meta[k.blk].skip) return;   // a group lies in one case: uniform
+    const int4 n4 = a.nb[q], l4 = local[q];
+    const int nb[4] = {n4.x, n4.y, n4.z, n4.w}, lo[4] = {l4.x, l4.y, l4.z, l4.w};
+    const int64_t ncp = a.ncp, c = k.c;
+    FirstCell f;
+    f.W = ldW4(a.Win, ncp, c);
+    load_geometry(a, k, f);
+    CS<double> U = ldU(a.U, ncp, c), U0 = U;
+    double P[4] = {0.0, 0.0, 0.0, 0.0};
+    if (a.P) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) P[v] = a.P[v * ncp + c];
+    }
+    // the finer level's part of the time step (CFL_Multigrid)
+    double dtf = MILLION;
+    const bool fine = fl.meta != nullptr;
+    if (fine) {
+        const BlockMeta m = fl.meta[k.blk];
+        const int i = k.ji & 0xFFFF, j = k.ji >> 16;
+        const int64_t sw = cell(m, 2 * (i - 2) + 2, 2 * (j - 2) + 2), se = sw + 1, nw = sw + m.pitch, ne = nw + 1;
+        const double dt_NE = qsqrt(qdiv(f.A, fl.A[ne])) * fl.dt[ne], dt_SE = qsqrt(qdiv(f.A, fl.A[se])) * fl.dt[se];
+        const double dt_NW = qsqrt(qdiv(f.A, fl.A[nw])) * fl.dt[nw], dt_SW = qsqrt(qdiv(f.A, fl.A[sw])) * fl.dt[sw];
+        dtf = dmin(dt_NE, dmin(dt_SE, dmin(dt_NW, dt_SW)));
+    }
+    double dtl = 0.0;
+    for (int nu = 0; nu < nsm; ++nu) {
+        {
+            const double d_i = 2.0 * qdiv(f.A, f.lE + f.lW), d_j = 2.0 * qdiv(f.A, f.lN + f.lS);
+            const double v_i = 0.5 * (f.W.vx * (f.nEx - -f.nWx) + f.W.vy * (f.nEy - -f.nWy));
+            const double v_j = 0.5 * (f.W.vx * (f.nNx - -f.nSx) + f.W.vy * (f.nNy - -f.nSy));
+            const double so = W_a(f.W);
+            dtl = dmin(qdiv(d_i, so + fabs(v_i)), qdiv(d_j, so + fabs(v_j)));
+            if (fine) dtl = dmin(dtl, dtf);
+        }
+        U0 = U;
+        for (int st = 0; st < a.nstage; ++st) {
+            if (on) { sW[0][t] = f.W.d; sW[1][t] = f.W.vx; sW[2][t] = f.W.vy; sW[3][t] = f.W.p; }
+            __syncthreads();
+            if (on) {
+                double dU[4];
+                first_residual(a, f, nb, a.cfl * dtl, P, [&](int s) -> PS<double> {
+                    const int q = lo[s] >= 0 ? lo[s] : t;   // at a boundary: not used
+                    return {sW[0][q], sW[1][q], sW[2][q], sW[3][q]};
+                }, dU);
+                f.W = first_update(a, k, U0, a.omega[st], f.W, dtl, dU, U);
+            }
+            __syncthreads();
+        }
+    }
+    if (!on) return;
+    stU(a.U, ncp, c, U);
+    stU(a.Uo, ncp, c, U0);
+    a.dt[c] = dtl;
+    a.Wout[c] = f.W.d; a.Wout[ncp + c] = f.W.vx; a.Wout[2 * ncp + c] = f.W.vy; a.Wout[3 * ncp + c] = f.W.p;
+}
+
 }  // namespace
 }  // namespace cffc
 
@@ -261,5 +443,15 @@ extern "C" hipError_t cffc_launch_mg_prolong(const BlockMeta *mc, const BlockMet
     const int nt = max_int_c <= 64 ? 64 : max_int_c <= 128 ? 128 : 256;
     hipLaunchKernelGGL(mg_prolong_kernel, dim3((max_int_c + nt - 1) / nt, nblk), dim3(nt), 0, st, mc, mf, bc, Uc, gc,
                        ncpc, Uf, Wf, gf, ncpf, neumann, inj_dirichlet, inj_always, stability, max_red, assign);
+    return hipGetLastError();
+}
+extern "C" hipError_t cffc_launch_mg_first_step(const FirstArgs *a, double omega, int first_stage, hipStream_t st) {
+    hipLaunchKernelGGL(mg_first_step_kernel, dim3((a->n + 255) / 256), dim3(256), 0, st, *a, omega, first_stage);
+    return hipGetLastError();
+}
+extern "C" hipError_t cffc_launch_mg_first_smooth(const FirstArgs *a, int ngroup, int max_group, const int32_t *group0,
+                                       const int4 *local, int nsm, const FineLevel *fl, hipStream_t st) {
+    hipLaunchKernelGGL(mg_first_smooth_kernel, dim3(ngroup), dim3((max_group + 63) / 64 * 64), 0, st, *a, group0, local,
+                       nsm, *fl);
     return hipGetLastError();
 }

@@ -245,7 +245,8 @@ template <int K> struct StageOpt {
     static constexpr bool general = K == SK_GRANULAR || K == SK_FUSED;   // axisymmetric, any limiter
     static constexpr bool amr = general || K == SK_LEVELS;
     static constexpr bool step = K == SK_STEP || K == SK_STEP_FIRST;
-    static constexpr bool window = K == SK_FUSED || K == SK_WINDOW || step;
+    static constexpr bool pull = step || K == SK_MG;   // can form all its ghost cells
+    static constexpr bool window = K == SK_FUSED || K == SK_WINDOW || pull;
     static constexpr bool first = K == SK_MG_FIRST || K == SK_STEP_FIRST;
 };
 // the leanest kernel that has every option of the launch
@@ -800,7 +801,7 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
 #pragma unroll
         for (int k = 0; k < NIT; ++k) {
             // a ghost cell that pull_ghosts replaces is written by its own thread only
-            if (O::step && tid + k * NT >= NWIN) continue;
+            if (O::pull && tid + k * NT >= NWIN) continue;
             const int il = slot[k] % LI, jl = slot[k] / LI;
 #pragma unroll
             for (int v = 0; v < 4; ++v) sW[v][jl][il] = wv[k][v];
@@ -823,10 +824,10 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
             }
         }
     }
-    if constexpr (O::step) {
+    if constexpr (O::pull && !Fast<FT>::on) {
         if (p.pull) pull_ghosts<LJ, LI>(p, m, t.b, pi0, pj0, tid, NT, sW);
     }
-    if (O::window && (O::step ? p.pull : p.window_bcs) && m.has_bc) window_ghosts<FT, LJ, LI>(p, m, pi0, pj0, tid, NT, sW);
+    if (O::window && (O::pull ? p.pull : p.window_bcs) && m.has_bc) window_ghosts<FT, LJ, LI>(p, m, pi0, pj0, tid, NT, sW);
     __syncthreads();
 
     // ---- phase 2: least-squares reconstruction + limiter -------------------
