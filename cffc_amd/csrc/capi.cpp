@@ -2120,9 +2120,10 @@ extern "C" int cffc_kernel_times(cffc_ctx *c, double out[4]) {
 // cell lists of a first-order level (FirstArgs), null where it has none
 struct FirstLevel {
     MgCell *cells = nullptr;
-    int4 *nb = nullptr, *local = nullptr;
-    int32_t *group0 = nullptr;
-    int n = 0, ngroup = 0, max_group = 0;
+    int4 *nb = nullptr, *cell_faces = nullptr;
+    MgFace *faces = nullptr;
+    int32_t *groups = nullptr;
+    int n = 0, ngroup = 0, nt = 0;   // groups, 0: not all of them fit; threads of one
 };
 
 struct cffc_mg {
@@ -2180,7 +2181,7 @@ static void mg_free(cffc_mg *mg) {
     if (mg->d_part_l2) (void)hipHostFree(mg->d_part_l2);
     if (mg->status) (void)hipHostFree(mg->status);
     for (FirstLevel &f : mg->first)
-        for (void *q : {(void *)f.cells, (void *)f.nb, (void *)f.local, (void *)f.group0})
+        for (void *q : {(void *)f.cells, (void *)f.nb, (void *)f.cell_faces, (void *)f.faces, (void *)f.groups})
             if (q) (void)hipFree(q);
     if (mg->gexec) (void)hipGraphExecDestroy(mg->gexec);
     if (mg->graph) (void)hipGraphDestroy(mg->graph);
@@ -2244,47 +2245,81 @@ static int mg_first_level(const cffc_ctx *c, const cffc_mesh_desc *md, FirstLeve
         max_group = std::max(max_group, (int)cells.size() - group0.back());
     }
     group0.push_back((int32_t)cells.size());
-    std::vector<int4> nbs(cells.size()), loc(cells.size());
-    for (size_t q = 0; q < cells.size(); ++q) {
-        const int b = cells[q].blk, i = cells[q].ji & 0xFFFF, j = cells[q].ji >> 16;
-        const BlockMeta &m = c->meta_h[b];
-        const int g0 = group0[gid[find(b)]];
-        int nv[4], lv[4];
-        // W, E, S, N: block face slot, boundary entry, neighbouring cell
-        const int di[4] = {-1, 1, 0, 0}, dj[4] = {0, 0, -1, 1}, slot[4] = {3, 2, 1, 0};
-        const int entry[4] = {j, m.ncj + j, 2 * m.ncj + i, 2 * m.ncj + m.nci + i};
-        for (int s = 0; s < 4; ++s) {
-            const int in = i + di[s], jn = j + dj[s];
-            const bool inside = in >= 2 && in <= m.ni + 1 && jn >= 2 && jn <= m.nj + 1;
-            const int e = m.bcoff + entry[s], o = md->nbr[8 * (size_t)b + slot[s]];
-            lv[s] = -1;
-            if (inside) {
-                nv[s] = (int32_t)(m.coff + (int64_t)jn * m.pitch + in);
-                lv[s] = first[b] + (jn - 2) * m.ni + (in - 2) - g0;
-            } else if (md->bc[e] != 0) {
-                nv[s] = -(e + 1);
-            } else {
-                const BlockMeta &S = c->meta_h[o];   // windowable: there is one
-                const int is = s == 0 ? S.ni + 1 : s == 1 ? 2 : in, js = s == 2 ? S.nj + 1 : s == 3 ? 2 : jn;
-                nv[s] = (int32_t)(S.coff + (int64_t)js * S.pitch + is);
-                lv[s] = first[o] + (js - 2) * S.ni + (is - 2) - g0;
+    std::vector<int4> nbs(cells.size()), cfs(cells.size());
+    std::vector<MgFace> faces, edge;
+    std::vector<int32_t> ends;   // per group: first cell, face, boundary face
+    int max_faces = 0, max_edge = 0;
+    for (size_t g = 0; g < groups.size(); ++g) {
+        const int32_t g0 = group0[g], g1 = group0[g + 1], f0 = (int32_t)faces.size();
+        edge.clear();
+        // boundary faces after the others, so that few waves hold both
+        auto add = [&](const MgFace &f) -> int {
+            std::vector<MgFace> &v = f.e < 0 ? faces : edge;
+            v.push_back(f);
+            return f.e < 0 ? (int)faces.size() - 1 - f0 : -(int)edge.size();
+        };
+        for (int32_t q = g0; q < g1; ++q) {
+            const int b = cells[q].blk, i = cells[q].ji & 0xFFFF, j = cells[q].ji >> 16;
+            const BlockMeta &m = c->meta_h[b];
+            int nv[4], fv[4];
+            // W, E, S, N: block face slot, boundary entry, neighbouring cell,
+            // the cell whose E or N face it is
+            const int di[4] = {-1, 1, 0, 0}, dj[4] = {0, 0, -1, 1}, slot[4] = {3, 2, 1, 0};
+            const int entry[4] = {j, m.ncj + j, 2 * m.ncj + i, 2 * m.ncj + m.nci + i};
+            const int32_t geo[4] = {cells[q].c - 1, cells[q].c, cells[q].south, cells[q].c};
+            for (int s = 0; s < 4; ++s) {
+                const int in = i + di[s], jn = j + dj[s];
+                const bool inside = in >= 2 && in <= m.ni + 1 && jn >= 2 && jn <= m.nj + 1, high = s & 1;
+                const int e = m.bcoff + entry[s];
+                const int16_t me = (int16_t)(q - g0);
+                int loc;
+                if (inside) {
+                    nv[s] = (int32_t)(m.coff + (int64_t)jn * m.pitch + in);
+                    loc = first[b] + (jn - 2) * m.ni + (in - 2) - g0;
+                } else if (md->bc[e] != 0) {
+                    nv[s] = -(e + 1);
+                    loc = -1;
+                } else {
+                    const int o = md->nbr[8 * (size_t)b + slot[s]];   // windowable: there is one
+                    const BlockMeta &S = c->meta_h[o];
+                    const int is = s == 0 ? S.ni + 1 : s == 1 ? 2 : in, js = s == 2 ? S.nj + 1 : s == 3 ? 2 : jn;
+                    nv[s] = (int32_t)(S.coff + (int64_t)js * S.pitch + is);
+                    loc = first[o] + (js - 2) * S.ni + (is - 2) - g0;
+                }
+                if (inside && !high) fv[s] = s == 0 ? cfs[g0 + loc].y : cfs[g0 + loc].w;   // that cell's E or N
+                else fv[s] = add(MgFace{geo[s], high ? me : (int16_t)loc, high ? (int16_t)loc : me,
+                                        loc < 0 ? e : -1, s >= 2});
             }
+            nbs[q] = make_int4(nv[0], nv[1], nv[2], nv[3]);
+            cfs[q] = make_int4(fv[0], fv[1], fv[2], fv[3]);
         }
-        nbs[q] = make_int4(nv[0], nv[1], nv[2], nv[3]);
-        loc[q] = make_int4(lv[0], lv[1], lv[2], lv[3]);
+        const int inner = (int)faces.size() - f0;
+        ends.insert(ends.end(), {g0, f0, f0 + inner});
+        max_edge = std::max(max_edge, (int)edge.size());
+        for (int32_t q = g0; q < g1; ++q)
+            for (int *f : {&cfs[q].x, &cfs[q].y, &cfs[q].z, &cfs[q].w})
+                if (*f < 0) *f = inner - *f - 1;
+        faces.insert(faces.end(), edge.begin(), edge.end());
+        max_faces = std::max(max_faces, (int)faces.size() - f0);
+        if (max_group > MG_GROUP_CELLS) faces.clear();   // places do not fit, nor are they used
     }
+    ends.push_back((int32_t)cells.size());
+    ends.push_back((int32_t)faces.size());
     if (int e = dalloc(&f.cells, cells.size())) return e;
     if (int e = dalloc(&f.nb, nbs.size())) return e;
     HIPCHK(hipMemcpy(f.cells, cells.data(), cells.size() * sizeof(MgCell), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(f.nb, nbs.data(), nbs.size() * sizeof(int4), hipMemcpyHostToDevice));
     f.n = (int)cells.size();
-    if (max_group <= 1024) {
-        if (int e = dalloc(&f.local, loc.size())) return e;
-        if (int e = dalloc(&f.group0, group0.size())) return e;
-        HIPCHK(hipMemcpy(f.local, loc.data(), loc.size() * sizeof(int4), hipMemcpyHostToDevice));
-        HIPCHK(hipMemcpy(f.group0, group0.data(), group0.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    if (max_group <= MG_GROUP_CELLS && max_faces <= MG_GROUP_FACES && max_edge <= MG_GROUP_EDGES) {
+        if (int e = dalloc(&f.cell_faces, cfs.size())) return e;
+        if (int e = dalloc(&f.faces, faces.size())) return e;
+        if (int e = dalloc(&f.groups, ends.size())) return e;
+        HIPCHK(hipMemcpy(f.cell_faces, cfs.data(), cfs.size() * sizeof(int4), hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy(f.faces, faces.data(), faces.size() * sizeof(MgFace), hipMemcpyHostToDevice));
+        HIPCHK(hipMemcpy(f.groups, ends.data(), ends.size() * sizeof(int32_t), hipMemcpyHostToDevice));
         f.ngroup = (int)groups.size();
-        f.max_group = max_group;
+        // a thread per face up to the largest workgroup, two beyond
+        f.nt = (std::min(std::max(max_group, max_faces), 1024) + 63) / 64 * 64;
     }
     return 0;
 }
@@ -2419,11 +2454,14 @@ static int mg_stage(cffc_ctx *c, int i_stage, int residual, const double *P, dou
 // from a zero residual (multistage optimal smoothing) and nothing runs between
 // the residual and the update.
 static bool mg_one_launch(const cffc_mg *mg, const cffc_ctx *c) {
-    const bool hlle = c->s.i_flux_function == CFFC_FLUX_FUNCTION_HLLE;
     return c->windowable && mg->rs_iters == 0 && !c->s.axisymmetric &&
            c->s.i_time_integration == CFFC_TIME_STEPPING_MULTISTAGE_OPTIMAL_SMOOTHING &&
-           (hlle ? c->s.i_limiter == CFFC_LIMITER_ZERO && !c->freeze
-                 : c->s.i_limiter == CFFC_LIMITER_VENKATAKRISHNAN);
+           c->s.i_flux_function != CFFC_FLUX_FUNCTION_HLLE && c->s.i_limiter == CFFC_LIMITER_VENKATAKRISHNAN;
+}
+static bool mg_listed(const cffc_mg *mg, const cffc_ctx *c, int l) {
+    return mg->first[l].n && mg->rs_iters == 0 && !c->s.axisymmetric &&
+           c->s.i_time_integration == CFFC_TIME_STEPPING_MULTISTAGE_OPTIMAL_SMOOTHING &&
+           c->s.i_flux_function == CFFC_FLUX_FUNCTION_HLLE && c->s.i_limiter == CFFC_LIMITER_ZERO && !c->freeze;
 }
 
 // one smoothing stage from the level's W buffer to its other one; pull: the
@@ -2478,7 +2516,8 @@ static int mg_smooth_first(cffc_mg *mg, int top, int l, int n, const double *P) 
         a.Win = c->W[c->wcur];
         a.Wout = c->W[c->wcur];
         const FineLevel fine = {f ? f->meta : nullptr, f ? f->dt : nullptr, f ? area(f) : nullptr};
-        HIPCHK(cffc_launch_mg_first_smooth(&a, fl.ngroup, fl.max_group, fl.group0, fl.local, n, &fine, c->stream));
+        const GroupArgs ga = {fl.groups, fl.faces, fl.cell_faces};
+        HIPCHK(cffc_launch_mg_first_smooth(&a, &ga, fl.ngroup, fl.nt, n, &fine, c->stream));
         return 0;
     }
     for (int nu = 0; nu < n; ++nu) {
@@ -2499,7 +2538,7 @@ static int mg_smooth_first(cffc_mg *mg, int top, int l, int n, const double *P) 
 static int mg_smooth(cffc_mg *mg, int top, int l, int n) {
     cffc_ctx *c = mg->lv[l];
     const double *P = l > top ? mg->P[l] : nullptr;
-    const bool listed = mg->first[l].n && c->s.i_flux_function == CFFC_FLUX_FUNCTION_HLLE && mg_one_launch(mg, c);
+    const bool listed = mg_listed(mg, c, l);
     if (listed && n > 0)
         if (int e = mg_smooth_first(mg, top, l, n, P)) return e;
     for (int nu = 0; nu < n && !listed; ++nu) {
@@ -2590,51 +2629,6 @@ static int mg_cgc(cffc_mg *mg, int top, int l) {
     return 0;
 }
 
-// Restrict_Boundary_Ref_States :1112-1186 on the host (the fine areas read
-// back once): coarse WoN/S/E/W over the interior span
-static int mg_restrict_wo(cffc_mg *mg, int lf) {
-    cffc_ctx *f = mg->lv[lf], *c = mg->lv[lf + 1];
-    std::vector<double> Af(f->ncp);
-    HIPCHK(hipMemcpyAsync(Af.data(), area(f), f->ncp * sizeof(double), hipMemcpyDeviceToHost, f->stream));
-    const size_t nwf = 4 * (size_t)(f->meta_h.back().bcoff + 2 * f->meta_h.back().ncj + 2 * f->meta_h.back().nci);
-    const size_t nwc = 4 * (size_t)(c->meta_h.back().bcoff + 2 * c->meta_h.back().ncj + 2 * c->meta_h.back().nci);
-    std::vector<double> wf(nwf), wc(nwc);
-    HIPCHK(hipMemcpyAsync(wf.data(), f->wo, nwf * sizeof(double), hipMemcpyDeviceToHost, f->stream));
-    HIPCHK(hipMemcpyAsync(wc.data(), c->wo, nwc * sizeof(double), hipMemcpyDeviceToHost, f->stream));
-    HIPCHK(hipStreamSynchronize(f->stream));
-    for (int b = 0; b < c->nblk; ++b) {
-        const BlockMeta &F = f->meta_h[b], &C = c->meta_h[b];
-        auto A = [&](int i, int j) { return Af[F.coff + (int64_t)j * F.pitch + i]; };
-        // entry (side, k) -> AoS offset; sides W, E (ncj entries), S, N (nci)
-        auto fo = [&](int side, int k) {
-            const int base = side == 0 ? 0 : side == 1 ? F.ncj : side == 2 ? 2 * F.ncj : 2 * F.ncj + F.nci;
-            return 4 * (size_t)(F.bcoff + base + k);
-        };
-        auto co = [&](int side, int k) {
-            const int base = side == 0 ? 0 : side == 1 ? C.ncj : side == 2 ? 2 * C.ncj : 2 * C.ncj + C.nci;
-            return 4 * (size_t)(C.bcoff + base + k);
-        };
-        auto avg = [&](int side_f, int k0, double A0, double A1, int side_c, int kc) {
-            const double *w0 = &wf[fo(side_f, k0)], *w1 = &wf[fo(side_f, k0 + 1)];
-            double *o = &wc[co(side_c, kc)];
-            for (int v = 0; v < 4; ++v) o[v] = (w0[v] * A0 + w1[v] * A1) / (A0 + A1);
-        };
-        const int JCl = 2, JCu = F.nj + 1, ICl = 2, ICu = F.ni + 1;
-        for (int ic = 2; ic <= C.ni + 1; ++ic) {
-            const int i0 = 2 * (ic - 2) + 2;
-            avg(3, i0, A(i0, JCu), A(i0 + 1, JCu), 3, ic);
-            avg(2, i0, A(i0, JCl), A(i0 + 1, JCl), 2, ic);
-        }
-        for (int jc = 2; jc <= C.nj + 1; ++jc) {
-            const int j0 = 2 * (jc - 2) + 2;
-            avg(0, j0, A(ICl, j0), A(ICl, j0 + 1), 0, jc);
-            avg(1, j0, A(ICu, j0), A(ICu, j0 + 1), 1, jc);
-        }
-    }
-    HIPCHK(hipMemcpy(c->wo, wc.data(), nwc * sizeof(double), hipMemcpyHostToDevice));
-    return 0;
-}
-
 // The start of Execute :3395-3420 for a state set on level 0: coarse levels
 // restricted from the level above (the IC_RESTART path of Apply_ICs
 // :719-733) with their boundary reference states, then messages and BCs.
@@ -2665,7 +2659,7 @@ extern "C" int cffc_mg_initialize(cffc_mg *mg) {
         cffc_ctx *f = mg->lv[l - 1], *c = mg->lv[l];
         HIPCHK(cffc_launch_mg_restrict(f->meta, c->meta, c->nblk, c->max_int, f->U, nullptr, area(f), f->ncp, c->U,
                                        c->W[c->wcur], nullptr, area(c), c->ncp, c->stream));
-        if (int e = mg_restrict_wo(mg, (int)l - 1)) return e;
+        HIPCHK(cffc_launch_mg_restrict_wo(f->meta, c->meta, c->nblk, 2 * c->max_edge, area(f), f->wo, c->wo, c->stream));
         if (int e = mg_exchange(c)) return e;
     }
     HIPCHK(hipStreamSynchronize(mg->lv[0]->stream));

@@ -777,7 +777,6 @@ static hipError_t launch_stage_kind(const StageParams *p, int ti, int tj, int ki
         case SK_MG: launch_stage_kernel<double, TI, TJ, SK_MG>(p, st); break;                              \
         case SK_MG_FIRST: launch_stage_kernel<double, TI, TJ, SK_MG_FIRST>(p, st); break;                  \
         case SK_STEP: launch_stage_kernel<double, TI, TJ, SK_STEP>(p, st); break;                          \
-        case SK_STEP_FIRST: launch_stage_kernel<double, TI, TJ, SK_STEP_FIRST>(p, st); break;              \
         case SK_FUSED: launch_stage_kernel<double, TI, TJ, SK_FUSED>(p, st); break;                            \
         default: launch_stage_kernel<double, TI, TJ, SK_GRANULAR>(p, st); break;                               \
         }                                                                                                  \
@@ -923,7 +922,7 @@ hipError_t cffc_launch_stage_fp64(const StageParams *p, int ti, int tj, int fuse
 // one smoothing stage of a multigrid level (SK_STEP): ghosts, residual, forcing
 // term and update, from W (Win) to the level's other buffer (Wout)
 hipError_t cffc_launch_mg_step(const StageParams *p, int ti, int tj, hipStream_t st) {
-    return launch_stage_kind(p, ti, tj, p->hlle ? SK_STEP_FIRST : SK_STEP, st);
+    return launch_stage_kind(p, ti, tj, SK_STEP, st);
 }
 
 }  // extern "C"

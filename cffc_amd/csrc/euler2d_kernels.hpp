@@ -97,6 +97,20 @@ struct FirstArgs {
     int32_t nstage, halve;
     unsigned long long *err;
 };
+// A face of a group of connected blocks, by the cells' places in the group: from
+// l to r, -1: boundary entry e (else e < 0); normal: E or N one of padded cell g.
+// A face between blocks is listed for each of them, with its own geometry.
+struct MgFace {
+    int32_t g;
+    int16_t l, r;
+    int32_t e, north;
+};
+enum { MG_GROUP_CELLS = 1024, MG_GROUP_FACES = 2048, MG_GROUP_EDGES = 512 };   // edges: faces on boundaries
+struct GroupArgs {
+    const int32_t *groups;   // first cell, face and boundary face of every group, and the ends
+    const MgFace *faces;
+    const int4 *cell_faces;  // W, E, S, N face of every cell, by place in the group
+};
 // the next finer level, for CFL_Multigrid (meta null: none)
 struct FineLevel {
     const BlockMeta *meta;
@@ -169,11 +183,12 @@ hipError_t cffc_launch_mg_changes(const cffc::BlockMeta *meta, int nblk, int max
                                   int64_t ncp, hipStream_t st);
 hipError_t cffc_launch_mg_copy(const cffc::BlockMeta *meta, int nblk, int max_cells, double *dst, const double *src,
                                int64_t ncp, hipStream_t st);
+hipError_t cffc_launch_mg_restrict_wo(const cffc::BlockMeta *mf, const cffc::BlockMeta *mc, int nblk, int max_faces,
+                                      const double *Af, const double *wf, double *wc, hipStream_t st);
 hipError_t cffc_launch_mg_first_step(const cffc::FirstArgs *a, double omega, int first_stage, hipStream_t st);
-// group0: first cell of every group of connected blocks; local: the neighbours'
-// places in their group, or -1
-hipError_t cffc_launch_mg_first_smooth(const cffc::FirstArgs *a, int ngroup, int max_group, const int32_t *group0,
-                                       const int4 *local, int nsm, const cffc::FineLevel *fl, hipStream_t st);
+// nt threads, at least a group's cells and half its faces
+hipError_t cffc_launch_mg_first_smooth(const cffc::FirstArgs *a, const cffc::GroupArgs *ga, int ngroup, int nt, int nsm,
+                                       const cffc::FineLevel *fl, hipStream_t st);
 hipError_t cffc_launch_mg_prolong(const cffc::BlockMeta *mc, const cffc::BlockMeta *mf, int nblk, int max_int_c,
                                   const int32_t *bc, const double *Uc, const double *gc, int64_t ncpc, double *Uf,
                                   double *Wf, const double *gf, int64_t ncpf, int neumann, int inj_dirichlet,

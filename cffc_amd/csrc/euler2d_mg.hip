@@ -230,6 +230,32 @@ __global__ void mg_prolong_kernel(const BlockMeta *mc, const BlockMeta *mf, cons
     }
 }
 
+// Restrict_Boundary_Ref_States :1112-1186: the reference state of a coarse
+// boundary face is the area-weighted mean of its two fine ones.  The states stay
+// on the device: through the host this was four copies a level, one of them every
+// cell's area.
+__global__ __launch_bounds__(64) void mg_restrict_wo_kernel(const BlockMeta *mf, const BlockMeta *mc, const double *Af,
+                                                            const double *wf, double *wc) {
+    const BlockMeta F = mf[blockIdx.x], C = mc[blockIdx.x];
+    const int n = 2 * (C.ni + C.nj);
+    for (int q = blockIdx.y * 64 + threadIdx.x; q < n; q += gridDim.y * 64) {
+        // sides W, E (nj entries each), S, N (ni each)
+        const int side = q < C.nj ? 0 : q < 2 * C.nj ? 1 : q < 2 * C.nj + C.ni ? 2 : 3;
+        const int k = q - (side == 0 ? 0 : side == 1 ? C.nj : side == 2 ? 2 * C.nj : 2 * C.nj + C.ni);
+        const int k0 = 2 * k + 2;
+        const int64_t c0 = side == 0 ? cell(F, 2, k0) : side == 1 ? cell(F, F.ni + 1, k0)
+                                     : side == 2 ? cell(F, k0, 2) : cell(F, k0, F.nj + 1);
+        const int64_t c1 = c0 + (side < 2 ? F.pitch : 1);
+        const int fb = side == 0 ? 0 : side == 1 ? F.ncj : side == 2 ? 2 * F.ncj : 2 * F.ncj + F.nci;
+        const int cb = side == 0 ? 0 : side == 1 ? C.ncj : side == 2 ? 2 * C.ncj : 2 * C.ncj + C.nci;
+        const double A0 = Af[c0], A1 = Af[c1];
+        const double *w0 = wf + 4 * (int64_t)(F.bcoff + fb + k0), *w1 = w0 + 4;
+        double *o = wc + 4 * (int64_t)(C.bcoff + cb + k + 2);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) o[v] = (w0[v] * A0 + w1[v] * A1) / (A0 + A1);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Smoothing of a first-order level (HLLE, zero limiter, so a face takes the
 // states of its two cells): a cell needs its four neighbours and nothing else,
@@ -249,44 +275,27 @@ __device__ __forceinline__ void load_geometry(const FirstArgs &a, const MgCell &
     f.nWx = G[GEO_NEX * n + w]; f.nWy = G[GEO_NEY * n + w]; f.nEx = G[GEO_NEX * n + c]; f.nEy = G[GEO_NEY * n + c];
     f.nSx = G[GEO_NNX * n + s]; f.nSy = G[GEO_NNY * n + s]; f.nNx = G[GEO_NNX * n + c]; f.nNy = G[GEO_NNY * n + c];
 }
-// flux through the face to neighbour state Wn, or to the boundary entry -(nb + 1)
-// of the bc / wo arrays; (nx, ny): the face's normal (E or N of its low cell), low:
-// this cell is on the high side
-__device__ __forceinline__ CS<double> first_flux(const FirstArgs &a, const PS<double> &Wc, PS<double> Wn, int nb, bool low,
-                                                 double nx, double ny) {
-    if (nb < 0) {
-        const int e = -(nb + 1), t = a.bc[e];
-        const PS<double> wo = {a.wo[4 * (int64_t)e], a.wo[4 * (int64_t)e + 1], a.wo[4 * (int64_t)e + 2],
-                               a.wo[4 * (int64_t)e + 3]};
-        const double sg = low ? -1.0 : 1.0;   // outward
-        if (t == 7001) Wn = reflect(Wc, sg * nx, sg * ny);
-        else if (t == 8001) Wn = bc_characteristic_pressure(Wc, wo, sg * nx, sg * ny);
-        else if (t == 11000) Wn = wo;
-        else Wn = Wc;
-    }
-    return low ? flux_hlle_n(Wn, Wc, nx, ny) : flux_hlle_n(Wc, Wn, nx, ny);
+// state beyond a boundary face of cell Wc; (nx, ny): the face's normal (E or N of
+// its low cell), low: the cell is on the high side, the boundary on the low one
+__device__ __forceinline__ PS<double> first_ghost(int t, const PS<double> &wo, const PS<double> &Wc, bool low, double nx,
+                                                  double ny) {
+    const double sg = low ? -1.0 : 1.0;   // outward
+    if (t == 7001) return reflect(Wc, sg * nx, sg * ny);
+    if (t == 8001) return bc_characteristic_pressure(Wc, wo, sg * nx, sg * ny);
+    return t == 11000 ? wo : Wc;
 }
-// (CFL dt)(+W -E +S -N)/A + (CFL dt) P, in the stage kernel's order
-template <typename State>
-__device__ __forceinline__ void first_residual(const FirstArgs &a, const FirstCell &f, const int (&nb)[4], double cdt,
-                                               const double (&P)[4], State state, double (&dU)[4]) {
-    const Recip<double> rA = recip(f.A);
-    CS<double> F = first_flux(a, f.W, state(0), nb[0], true, f.nWx, f.nWy);
-    dU[0] = 0.0 + rdivf(cdt * F.d * f.lW, rA); dU[1] = 0.0 + rdivf(cdt * F.mx * f.lW, rA);
-    dU[2] = 0.0 + rdivf(cdt * F.my * f.lW, rA); dU[3] = 0.0 + rdivf(cdt * F.E * f.lW, rA);
-    F = first_flux(a, f.W, state(1), nb[1], false, f.nEx, f.nEy);
-    dU[0] -= rdivf(cdt * F.d * f.lE, rA); dU[1] -= rdivf(cdt * F.mx * f.lE, rA);
-    dU[2] -= rdivf(cdt * F.my * f.lE, rA); dU[3] -= rdivf(cdt * F.E * f.lE, rA);
-    F = first_flux(a, f.W, state(2), nb[2], true, f.nSx, f.nSy);
-    dU[0] += rdivf(cdt * F.d * f.lS, rA); dU[1] += rdivf(cdt * F.mx * f.lS, rA);
-    dU[2] += rdivf(cdt * F.my * f.lS, rA); dU[3] += rdivf(cdt * F.E * f.lS, rA);
-    F = first_flux(a, f.W, state(3), nb[3], false, f.nNx, f.nNy);
-    dU[0] -= rdivf(cdt * F.d * f.lN, rA); dU[1] -= rdivf(cdt * F.mx * f.lN, rA);
-    dU[2] -= rdivf(cdt * F.my * f.lN, rA); dU[3] -= rdivf(cdt * F.E * f.lN, rA);
-    if (a.P) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) dU[v] += cdt * P[v];
-    }
+// (CFL dt)(+W -E +S -N)/A in the stage kernel's order
+__device__ __forceinline__ void first_sum(const CS<double> &W, const CS<double> &E, const CS<double> &S, const CS<double> &N,
+                                          double lW, double lE, double lS, double lN, const Recip<double> &rA, double cdt,
+                                          double (&dU)[4]) {
+    dU[0] = 0.0 + rdivf(cdt * W.d * lW, rA); dU[1] = 0.0 + rdivf(cdt * W.mx * lW, rA);
+    dU[2] = 0.0 + rdivf(cdt * W.my * lW, rA); dU[3] = 0.0 + rdivf(cdt * W.E * lW, rA);
+    dU[0] -= rdivf(cdt * E.d * lE, rA); dU[1] -= rdivf(cdt * E.mx * lE, rA);
+    dU[2] -= rdivf(cdt * E.my * lE, rA); dU[3] -= rdivf(cdt * E.E * lE, rA);
+    dU[0] += rdivf(cdt * S.d * lS, rA); dU[1] += rdivf(cdt * S.mx * lS, rA);
+    dU[2] += rdivf(cdt * S.my * lS, rA); dU[3] += rdivf(cdt * S.E * lS, rA);
+    dU[0] -= rdivf(cdt * N.d * lN, rA); dU[1] -= rdivf(cdt * N.mx * lN, rA);
+    dU[2] -= rdivf(cdt * N.my * lN, rA); dU[3] -= rdivf(cdt * N.E * lN, rA);
 }
 // update_kernel's rule; returns W^(s+1), Wc where the state stays unphysical
 __device__ __forceinline__ PS<double> first_update(const FirstArgs &a, const MgCell &k, const CS<double> &U0, double om,
@@ -334,7 +343,21 @@ __global__ __launch_bounds__(256) void mg_first_step_kernel(FirstArgs a, double 
         for (int v = 0; v < 4; ++v) P[v] = a.P[v * ncp + c];
     }
     const double dt0 = dtl;
-    first_residual(a, f, nb, a.cfl * dtl, P, [&](int s) { return Wn[s]; }, dU);
+    auto flux = [&](int h, bool low, double nx, double ny) -> CS<double> {
+        if (nb[h] < 0) {
+            const int e = -(nb[h] + 1);
+            const double *w = a.wo + 4 * (int64_t)e;
+            Wn[h] = first_ghost(a.bc[e], PS<double>{w[0], w[1], w[2], w[3]}, f.W, low, nx, ny);
+        }
+        return low ? flux_hlle_n(Wn[h], f.W, nx, ny) : flux_hlle_n(f.W, Wn[h], nx, ny);
+    };
+    const double cdt = a.cfl * dtl;
+    first_sum(flux(0, true, f.nWx, f.nWy), flux(1, false, f.nEx, f.nEy), flux(2, true, f.nSx, f.nSy),
+              flux(3, false, f.nNx, f.nNy), f.lW, f.lE, f.lS, f.lN, recip(f.A), cdt, dU);
+    if (a.P) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) dU[v] += cdt * P[v];
+    }
     CS<double> Un;
     const PS<double> w = first_update(a, k, U0, om, f.W, dtl, dU, Un);
     if (dtl != dt0) a.dt[c] = dtl;
@@ -343,32 +366,59 @@ __global__ __launch_bounds__(256) void mg_first_step_kernel(FirstArgs a, double 
     a.Wout[c] = w.d; a.Wout[ncp + c] = w.vx; a.Wout[2 * ncp + c] = w.vy; a.Wout[3 * ncp + c] = w.p;
 }
 
-// All smoothings of a level whose connected groups of blocks have at most 1,024
-// cells, in one launch: a workgroup per group, a thread per cell, W in LDS,
-// everything else of the cell in registers.  nsm smoothings of a.nstage stages;
-// each starts with the cell's CFL time step and the finer level's rule
-// (cfl_kernel).  18 launches of the coarsest level of a V cycle (3 smoothings)
-// become one.
-__global__ __launch_bounds__(1024) void mg_first_smooth_kernel(FirstArgs a, const int32_t *group0, const int4 *local,
-                                                               int nsm, FineLevel fl) {
-    __shared__ double sW[4][1024];
-    const int g0 = group0[blockIdx.x], n = group0[blockIdx.x + 1] - g0, t = threadIdx.x;
+// All smoothings of a level whose connected groups of blocks are small (at most
+// MG_GROUP_CELLS cells, MG_GROUP_FACES faces), in one launch: a workgroup per
+// group.  nsm smoothings of a.nstage stages; each starts with the cell's CFL time
+// step and the finer level's rule (cfl_kernel).  In a stage a thread first
+// evaluates one or two faces of the group's list into LDS, then updates its cell
+// from its four faces; W, the fluxes, the faces' normals and the boundaries' states live in LDS (155 of
+// 160 KB), the cells' geometry and U in registers.  A wave alone on its SIMD is bound by the flux's own dependent
+// instructions, so faces, not cells, are spread over the threads: 15 stages of
+// 48 cells 65 -> 58 us, of 768 cells (64 cases at once) 151 -> 140 us against a
+// thread per cell that evaluates its four faces.
+__global__ __launch_bounds__(1024) void mg_first_smooth_kernel(FirstArgs a, GroupArgs ga, int nsm, FineLevel fl) {
+    __shared__ double sW[4][MG_GROUP_CELLS], sF[4][MG_GROUP_FACES], sn[2][MG_GROUP_FACES];
+    __shared__ double swo[4][MG_GROUP_EDGES];
+    __shared__ int16_t sLR[2][MG_GROUP_FACES];   // negative: the boundary's kind, -1 ... -4
+    const int32_t *gr = ga.groups + 3 * blockIdx.x;
+    const int g0 = gr[0], n = gr[3] - g0, f0 = gr[1], nf = gr[4] - f0, inner = gr[2] - f0;
+    const int t = threadIdx.x, nt = blockDim.x;
     const bool on = t < n;
     const int q = g0 + (on ? t : 0);
     const MgCell k = a.cells[q];
     if (a.meta[k.blk].skip) return;   // a group lies in one case: uniform
-    const int4 n4 = a.nb[q], l4 = local[q];
-    const int nb[4] = {n4.x, n4.y, n4.z, n4.w}, lo[4] = {l4.x, l4.y, l4.z, l4.w};
+    const double *G = a.geom;
     const int64_t ncp = a.ncp, c = k.c;
-    FirstCell f;
-    f.W = ldW4(a.Win, ncp, c);
-    load_geometry(a, k, f);
+    for (int f = t; f < nf; f += nt) {
+        const MgFace k = ga.faces[f0 + f];
+        int l = k.l, r = k.r;
+        if (k.e >= 0) {
+            const int bc = a.bc[k.e], kind = bc == 7001 ? -2 : bc == 8001 ? -3 : bc == 11000 ? -4 : -1;
+            if (l < 0) l = kind;
+            else r = kind;
+            const double *w = a.wo + 4 * (int64_t)k.e;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) swo[v][f - inner] = w[v];
+        }
+        sLR[0][f] = (int16_t)l;
+        sLR[1][f] = (int16_t)r;
+        sn[0][f] = G[(k.north ? GEO_NNX : GEO_NEX) * ncp + k.g];
+        sn[1][f] = G[(k.north ? GEO_NNY : GEO_NEY) * ncp + k.g];
+    }
+    // the thread's cell
+    const int4 cf = ga.cell_faces[q];
+    const int fW = cf.x, fE = cf.y, fS = cf.z, fN = cf.w;
+    PS<double> W = ldW4(a.Win, ncp, c);
     CS<double> U = ldU(a.U, ncp, c), U0 = U;
     double P[4] = {0.0, 0.0, 0.0, 0.0};
     if (a.P) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) P[v] = a.P[v * ncp + c];
     }
+    const int64_t wc = c - 1, sc = k.south;
+    const double lW = G[GEO_LE * ncp + wc], lE = G[GEO_LE * ncp + c], lS = G[GEO_LN * ncp + sc], lN = G[GEO_LN * ncp + c];
+    const double A = G[GEO_A * ncp + c];
+    const Recip<double> rA = recip(A);
     // the finer level's part of the time step (CFL_Multigrid)
     double dtf = MILLION;
     const bool fine = fl.meta != nullptr;
@@ -376,40 +426,63 @@ __global__ __launch_bounds__(1024) void mg_first_smooth_kernel(FirstArgs a, cons
         const BlockMeta m = fl.meta[k.blk];
         const int i = k.ji & 0xFFFF, j = k.ji >> 16;
         const int64_t sw = cell(m, 2 * (i - 2) + 2, 2 * (j - 2) + 2), se = sw + 1, nw = sw + m.pitch, ne = nw + 1;
-        const double dt_NE = qsqrt(qdiv(f.A, fl.A[ne])) * fl.dt[ne], dt_SE = qsqrt(qdiv(f.A, fl.A[se])) * fl.dt[se];
-        const double dt_NW = qsqrt(qdiv(f.A, fl.A[nw])) * fl.dt[nw], dt_SW = qsqrt(qdiv(f.A, fl.A[sw])) * fl.dt[sw];
+        const double dt_NE = qsqrt(qdiv(A, fl.A[ne])) * fl.dt[ne], dt_SE = qsqrt(qdiv(A, fl.A[se])) * fl.dt[se];
+        const double dt_NW = qsqrt(qdiv(A, fl.A[nw])) * fl.dt[nw], dt_SW = qsqrt(qdiv(A, fl.A[sw])) * fl.dt[sw];
         dtf = dmin(dt_NE, dmin(dt_SE, dmin(dt_NW, dt_SW)));
     }
     double dtl = 0.0;
+    if (on) { sW[0][t] = W.d; sW[1][t] = W.vx; sW[2][t] = W.vy; sW[3][t] = W.p; }
     for (int nu = 0; nu < nsm; ++nu) {
-        {
-            const double d_i = 2.0 * qdiv(f.A, f.lE + f.lW), d_j = 2.0 * qdiv(f.A, f.lN + f.lS);
-            const double v_i = 0.5 * (f.W.vx * (f.nEx - -f.nWx) + f.W.vy * (f.nEy - -f.nWy));
-            const double v_j = 0.5 * (f.W.vx * (f.nNx - -f.nSx) + f.W.vy * (f.nNy - -f.nSy));
-            const double so = W_a(f.W);
-            dtl = dmin(qdiv(d_i, so + fabs(v_i)), qdiv(d_j, so + fabs(v_j)));
-            if (fine) dtl = dmin(dtl, dtf);
-        }
+        // the normals are read again rather than held: 1,024 threads have 128
+        // registers each
+        const double d_i = 2.0 * qdiv(A, lE + lW), d_j = 2.0 * qdiv(A, lN + lS);
+        const double v_i = 0.5 * (W.vx * (G[GEO_NEX * ncp + c] - -G[GEO_NEX * ncp + wc]) +
+                                  W.vy * (G[GEO_NEY * ncp + c] - -G[GEO_NEY * ncp + wc]));
+        const double v_j = 0.5 * (W.vx * (G[GEO_NNX * ncp + c] - -G[GEO_NNX * ncp + sc]) +
+                                  W.vy * (G[GEO_NNY * ncp + c] - -G[GEO_NNY * ncp + sc]));
+        const double so = W_a(W);
+        dtl = dmin(qdiv(d_i, so + fabs(v_i)), qdiv(d_j, so + fabs(v_j)));
+        if (fine) dtl = dmin(dtl, dtf);
         U0 = U;
         for (int st = 0; st < a.nstage; ++st) {
-            if (on) { sW[0][t] = f.W.d; sW[1][t] = f.W.vx; sW[2][t] = f.W.vy; sW[3][t] = f.W.p; }
             __syncthreads();
-            if (on) {
-                double dU[4];
-                first_residual(a, f, nb, a.cfl * dtl, P, [&](int s) -> PS<double> {
-                    const int q = lo[s] >= 0 ? lo[s] : t;   // at a boundary: not used
-                    return {sW[0][q], sW[1][q], sW[2][q], sW[3][q]};
-                }, dU);
-                f.W = first_update(a, k, U0, a.omega[st], f.W, dtl, dU, U);
+#pragma unroll 1
+            for (int f = t; f < nf; f += nt) {
+                const int l = sLR[0][f], r = sLR[1][f], il = l >= 0 ? l : r, ir = r >= 0 ? r : l;
+                PS<double> Wl = {sW[0][il], sW[1][il], sW[2][il], sW[3][il]};
+                PS<double> Wr = {sW[0][ir], sW[1][ir], sW[2][ir], sW[3][ir]};
+                const double nx = sn[0][f], ny = sn[1][f];
+                if ((l | r) < 0) {
+                    const int q = f - inner, kind = l < 0 ? l : r;
+                    const PS<double> wo = {swo[0][q], swo[1][q], swo[2][q], swo[3][q]};
+                    const PS<double> g = first_ghost(kind == -2 ? 7001 : kind == -3 ? 8001 : kind == -4 ? 11000 : 0, wo, Wl,
+                                                     l < 0, nx, ny);
+                    if (l < 0) Wl = g;
+                    else Wr = g;
+                }
+                const CS<double> F = flux_hlle_n(Wl, Wr, nx, ny);
+                sF[0][f] = F.d; sF[1][f] = F.mx; sF[2][f] = F.my; sF[3][f] = F.E;
             }
             __syncthreads();
+            if (on) {
+                auto F = [&](int x) -> CS<double> { return {sF[0][x], sF[1][x], sF[2][x], sF[3][x]}; };
+                const double cdt = a.cfl * dtl;
+                double dU[4];
+                first_sum(F(fW), F(fE), F(fS), F(fN), lW, lE, lS, lN, rA, cdt, dU);
+                if (a.P) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) dU[v] += cdt * P[v];
+                }
+                W = first_update(a, k, U0, a.omega[st], W, dtl, dU, U);
+                sW[0][t] = W.d; sW[1][t] = W.vx; sW[2][t] = W.vy; sW[3][t] = W.p;
+            }
         }
     }
     if (!on) return;
     stU(a.U, ncp, c, U);
     stU(a.Uo, ncp, c, U0);
     a.dt[c] = dtl;
-    a.Wout[c] = f.W.d; a.Wout[ncp + c] = f.W.vx; a.Wout[2 * ncp + c] = f.W.vy; a.Wout[3 * ncp + c] = f.W.p;
+    a.Wout[c] = W.d; a.Wout[ncp + c] = W.vx; a.Wout[2 * ncp + c] = W.vy; a.Wout[3 * ncp + c] = W.p;
 }
 
 }  // namespace
@@ -445,13 +518,17 @@ extern "C" hipError_t cffc_launch_mg_prolong(const BlockMeta *mc, const BlockMet
                        ncpc, Uf, Wf, gf, ncpf, neumann, inj_dirichlet, inj_always, stability, max_red, assign);
     return hipGetLastError();
 }
+extern "C" hipError_t cffc_launch_mg_restrict_wo(const BlockMeta *mf, const BlockMeta *mc, int nblk, int max_faces,
+                                       const double *Af, const double *wf, double *wc, hipStream_t st) {
+    hipLaunchKernelGGL(mg_restrict_wo_kernel, dim3(nblk, (max_faces + 63) / 64), dim3(64), 0, st, mf, mc, Af, wf, wc);
+    return hipGetLastError();
+}
 extern "C" hipError_t cffc_launch_mg_first_step(const FirstArgs *a, double omega, int first_stage, hipStream_t st) {
     hipLaunchKernelGGL(mg_first_step_kernel, dim3((a->n + 255) / 256), dim3(256), 0, st, *a, omega, first_stage);
     return hipGetLastError();
 }
-extern "C" hipError_t cffc_launch_mg_first_smooth(const FirstArgs *a, int ngroup, int max_group, const int32_t *group0,
-                                       const int4 *local, int nsm, const FineLevel *fl, hipStream_t st) {
-    hipLaunchKernelGGL(mg_first_smooth_kernel, dim3(ngroup), dim3((max_group + 63) / 64 * 64), 0, st, *a, group0, local,
-                       nsm, *fl);
+extern "C" hipError_t cffc_launch_mg_first_smooth(const FirstArgs *a, const GroupArgs *ga, int ngroup, int nt, int nsm,
+                                       const FineLevel *fl, hipStream_t st) {
+    hipLaunchKernelGGL(mg_first_smooth_kernel, dim3(ngroup), dim3(nt), 0, st, *a, *ga, nsm, *fl);
     return hipGetLastError();
 }
