@@ -237,17 +237,16 @@ enum StageKind {
     SK_LEVELS = 4,     // SK_PLAIN with resolution changes
     SK_MG = 5,         // granular: one level, planar, Venkatakrishnan, Roe
     SK_MG_FIRST = 6,   // granular multigrid stage of a first-order level: zero limiter, so no reconstruction
-    SK_STEP = 7,       // SK_MG with its ghost cells and its update: one launch per smoothing stage
-    SK_STEP_FIRST = 8  // the same on a first-order level
+    SK_STEP = 7        // SK_MG with its ghost cells and its update: one launch per smoothing stage
 };
 template <int K> struct StageOpt {
     static constexpr bool fused = K == SK_FUSED || K == SK_PLAIN || K == SK_WINDOW || K == SK_LEVELS;
     static constexpr bool general = K == SK_GRANULAR || K == SK_FUSED;   // axisymmetric, any limiter
     static constexpr bool amr = general || K == SK_LEVELS;
-    static constexpr bool step = K == SK_STEP || K == SK_STEP_FIRST;
+    static constexpr bool step = K == SK_STEP;
     static constexpr bool pull = step || K == SK_MG;   // can form all its ghost cells
     static constexpr bool window = K == SK_FUSED || K == SK_WINDOW || pull;
-    static constexpr bool first = K == SK_MG_FIRST || K == SK_STEP_FIRST;
+    static constexpr bool first = K == SK_MG_FIRST;
 };
 // the leanest kernel that has every option of the launch
 inline int stage_kind(const StageParams &p, int fused) {
@@ -411,6 +410,60 @@ __device__ __forceinline__ void reconstruct(const StageParams &p, const BlockGeo
         }
         if (n == 0) ph.d = phi; else if (n == 1) ph.vx = phi; else if (n == 2) ph.vy = phi; else ph.p = phi;
     }
+}
+
+// One variable's share of reconstruct (FP64): the same sums, quotients and limiter
+// in the same order, with the matrix formed again by each of the four threads of
+// a cell.  Wn: the variable's window.
+template <typename O, bool FULL, int LJ, int LI>
+__device__ __forceinline__ void reconstruct_var(const StageParams &p, const BlockGeo<double> &geo, const double *phi_n,
+                                                int phim, uint32_t o8, int il, int jl, unsigned mask,
+                                                const double (&Wn)[LJ][LI], const double (&sX)[LJ][LI],
+                                                const double (&sY)[LJ][LI], double &gx, double &gy, double &ph) {
+    const double u0 = Wn[jl][il], xc0 = sX[jl][il], yc0 = sY[jl][il];
+    gx = gy = ph = 0.0;
+    if (!FULL && mask == 0u) return;
+    double Dx = 0.0, Dy = 0.0, DxDx = 0.0, DxDy = 0.0, DyDy = 0.0, umin = u0, umax = u0;
+    int n_pts = 0;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+        const int kk = s < 4 ? s : s + 1;
+        const int a = il + (kk % 3) - 1, b = jl + (kk / 3) - 1;
+        const double dX = sX[b][a] - xc0, dY = sY[b][a] - yc0, v = Wn[b][a], DU = v - u0;
+        if (FULL || (mask & (1u << s))) {
+            Dx += DU * dX; Dy += DU * dY;
+            DxDx += dX * dX; DxDy += dX * dY; DyDy += dY * dY;
+            umin = vmin64(umin, v); umax = vmax64(umax, v);
+            ++n_pts;
+        }
+    }
+    if (FULL) {
+        Dx *= 0.125; Dy *= 0.125;
+        DxDx *= 0.125; DxDy *= 0.125; DyDy *= 0.125;
+    } else {
+        const Recip<double> rn = recip((double)n_pts);
+        Dx = rdiv(Dx, rn); Dy = rdiv(Dy, rn);
+        DxDx = rdiv(DxDx, rn); DxDy = rdiv(DxDy, rn); DyDy = rdiv(DyDy, rn);
+    }
+    const Recip<double> rd = recip(DxDx * DyDy - DxDy * DxDy);
+    gx = rdivf(Dx * DyDy - Dy * DxDy, rd);
+    gy = rdivf(Dy * DxDx - Dx * DxDy, rd);
+    if (phim == PHI_LOAD) {
+        ph = at(phi_n, o8);
+        return;
+    }
+    if constexpr (O::general) {
+        if (p.limiter == -1) { ph = 1.0; return; }
+        if (p.limiter == 0) return;
+    }
+    const double dxE = geo.rd(GEO_XFE, GF_XFE, o8) - xc0, dyE = geo.rd(GEO_YFE, GF_YFE, o8) - yc0;
+    const double dxW = geo.rdw(GEO_XFE, GF_XFE, o8) - xc0, dyW = geo.rdw(GEO_YFE, GF_YFE, o8) - yc0;
+    const double dxN = geo.rd(GEO_XFN, GF_XFN, o8) - xc0, dyN = geo.rd(GEO_YFN, GF_YFN, o8) - yc0;
+    const double dxS = geo.rds(GEO_XFN, GF_XFN, o8) - xc0, dyS = geo.rds(GEO_YFN, GF_YFN, o8) - yc0;
+    ph = venkat_fold(1.0, u0 + gx * dxE + gy * dyE, u0, umin, umax);
+    ph = venkat_fold(ph, u0 + gx * dxW + gy * dyW, u0, umin, umax);
+    ph = venkat_fold(ph, u0 + gx * dxN + gy * dyN, u0, umin, umax);
+    ph = venkat_fold(ph, u0 + gx * dxS + gy * dyS, u0, umin, umax);
 }
 
 // The update's rejection test U.d <= 0 || U.E <= 0 || U.e() <= 0
@@ -672,6 +725,19 @@ template <int TI, int TJ> struct TileThreads {
     static constexpr int value = ring_pass ? ((tile + 63) / 64) * 64 : ((tile + ring + 63) / 64) * 64;
 };
 
+// Small FP64 grids run split tiles: four threads per reconstructed cell, one for
+// each variable, then a thread per face.  Grids this small leave a SIMD one or two
+// waves, whose time is the length of a thread's chain of instructions, not their
+// number (a third more of them here).
+template <typename FT, int TI, int TJ, int KIND> struct Splittable {
+    static constexpr bool value = !Fast<FT>::on && TI * TJ >= 64 && TI * TJ <= 128 &&
+                                  (KIND == SK_PLAIN || KIND == SK_WINDOW || KIND == SK_LEVELS || KIND == SK_MG ||
+                                   KIND == SK_STEP);
+};
+template <int TI, int TJ, bool SPLIT> struct StageThreads {
+    static constexpr int value = SPLIT ? (4 * (TI * TJ + 2 * (TI + TJ)) + 63) / 64 * 64 : TileThreads<TI, TJ>::value;
+};
+
 // Resident wavefronts per SIMD asked of the compiler: the mixed ring-pass
 // tiles fit six in 80 VGPRs without spilling (0.5% faster at 32 x 8 than the
 // five that 82 VGPRs allow); the FP64 kernels are left to the compiler.
@@ -679,12 +745,12 @@ template <typename FT, int TI, int TJ> struct StageWaves {
     static constexpr int value = Fast<FT>::on ? (TileThreads<TI, TJ>::ring_pass ? 6 : 1) : 4;
 };
 
-template <typename FT, int TI, int TJ, int KIND>
-__global__ __launch_bounds__((TileThreads<TI, TJ>::value))
+template <typename FT, int TI, int TJ, int KIND, bool SPLIT = false>
+__global__ __launch_bounds__((StageThreads<TI, TJ, SPLIT>::value))
 __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_kernel(StageParams p) {
     typedef StageOpt<KIND> O;
     constexpr bool FUSED = O::fused;
-    constexpr int NT = TileThreads<TI, TJ>::value;
+    constexpr int NT = StageThreads<TI, TJ, SPLIT>::value;
     constexpr int NTILE = TI * TJ;
     constexpr int LI = TI + 4, LJ = TJ + 4;
     constexpr int RI = TI + 2, RJ = TJ + 2;
@@ -767,6 +833,11 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
         else if ((r -= TI) < TI) { ring_side = 3; ring_k = r; }
     }
 
+    // split tiles: the thread's variable, cell (ring coordinates), byte offset (0: none)
+    // and stencil, whose BC entries are loaded beside the window
+    int sir = -1, sjr = -1, sv = 0;
+    uint32_t so8 = 0;
+    unsigned smask = 0xFFu;
     // ---- phase 1: W and centroids of the window ---------------------------
     const double *Win = p.Win + org;
     const float *Winf = FUSED && Fast<FT>::on ? p.Winf + org : nullptr;
@@ -797,6 +868,29 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
             }
             xw[k] = geo.rd(GEO_XC, GF_XC, e * XS);
             yw[k] = geo.rd(GEO_YC, GF_YC, e * XS);
+        }
+        if constexpr (SPLIT) {
+            constexpr int NRING = 2 * (TI + TJ);
+            // task: variable-major over the tile's cells, then over the W, E, S, N
+            // ring cells
+            if (tid < 4 * NTILE) {
+                const int r = tid % NTILE;
+                sv = tid / NTILE;
+                sir = r % TI + 1; sjr = r / TI + 1;
+            } else if (tid < 4 * (NTILE + NRING)) {
+                int r = (tid - 4 * NTILE) % NRING;
+                sv = (tid - 4 * NTILE) / NRING;
+                if (r < TJ) { sir = 0; sjr = r + 1; }
+                else if ((r -= TJ) < TJ) { sir = TI + 1; sjr = r + 1; }
+                else if ((r -= TJ) < TI) { sir = r + 1; sjr = 0; }
+                else { r -= TI; sir = r + 1; sjr = TJ + 1; }
+            }
+            const int ip = pi0 + sir + 1, jp = pj0 + sjr + 1;
+            if (sir >= 0 && ip <= m.nci - 2 && jp <= m.ncj - 2) {
+                so8 = (uint32_t)((jp - pj0) * m.pitch + ip) * 8u;
+                if (m.has_bc && (ip <= 1 || ip >= ICu + 1 || jp <= 1 || jp >= JCu + 1))
+                    smask = stencil_mask(ip, jp, ICu, JCu, bcW[jp], bcE[jp], bcS[ip], bcN[ip]);
+            }
         }
 #pragma unroll
         for (int k = 0; k < NIT; ++k) {
@@ -837,6 +931,26 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
     // use the full 8-point stencil; only the ring cells of boundary blocks
     // read the BC arrays (reduced stencils).
     // A first-order level only records its zero limiters.
+    if constexpr (SPLIT) {
+        // a wave that holds a reduced stencil takes the masked code for all its
+        // cells (with the full mask it gives the same bits), not both codes in turn
+        const bool reduced = __any(smask != 0xFFu);
+        if (so8) {
+            const int il = sir + 1, jl = sjr + 1, ip = pi0 + il, jp = pj0 + jl;
+            double *phin = p.phi + sv * ncp + org;
+            double gx, gy, ph;
+            if (reduced) reconstruct_var<O, false>(p, geo, phin, phim, so8, il, jl, smask, sW[sv], sX, sY, gx, gy, ph);
+            else reconstruct_var<O, true>(p, geo, phin, phim, so8, il, jl, 0xFFu, sW[sv], sX, sY, gx, gy, ph);
+            if (phim == PHI_COMPUTE_STORE) {
+                const bool own_i = (ip >= pi0 + 2 && ip < pi0 + 2 + TI) || ip == 1 || ip == m.nci - 2;
+                const bool own_j = (jp >= pj0 + 2 && jp < pj0 + 2 + TJ) || jp == 1 || jp == m.ncj - 2;
+                if (own_i && own_j) at(phin, so8) = ph;
+            }
+            sPx[sv][sjr][sir] = ph * gx;
+            sPy[sv][sjr][sir] = ph * gy;
+        }
+    }
+    if constexpr (!SPLIT)
     for (int role = tid; role < (RP ? NTILE + 2 * (TI + TJ) : tid + 1) && !(O::first && phim != PHI_COMPUTE_STORE);
          role += NT) {
         // role: a tile cell, then the W, E, S, N ring cells
@@ -914,13 +1028,25 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
     const int ring_fk = ring_w ? tid : tid - TJ;
     uint32_t cF1 = 0, cF2 = 0, cFR = 0;
     bool v1 = false, v2 = false, vR = false;
-    if (is_tile) {
-        v1 = face_cell(true, tc + 1, tr, cF1);
-        v2 = face_cell(false, tr + 1, tc, cF2);
+    // i-face f1 of row g1 and j-face f2 of column g2
+    int f1 = is_tile ? tc + 1 : 0, g1r = is_tile ? tr : ring_k, f2 = is_tile ? tr + 1 : 0, g2c = is_tile ? tc : ring_k;
+    if constexpr (SPLIT) {
+        // E faces, N faces, W ring faces, S ring faces
+        const int r = tid - NTILE, w = r - NTILE;
+        if (!is_tile) {
+            f2 = r < NTILE ? r / TI + 1 : 0;
+            g2c = r < NTILE ? r % TI : w - TJ;
+            g1r = w;
+        }
+        if (is_tile || (w >= 0 && w < TJ)) v1 = face_cell(true, f1, g1r, cF1);
+        else if (w < TJ + TI) v2 = face_cell(false, f2, g2c, cF2);
+    } else if (is_tile) {
+        v1 = face_cell(true, f1, g1r, cF1);
+        v2 = face_cell(false, f2, g2c, cF2);
     } else if (ring_side == 0) {
-        v1 = face_cell(true, 0, ring_k, cF1);
+        v1 = face_cell(true, f1, g1r, cF1);
     } else if (ring_side == 2) {
-        v2 = face_cell(false, 0, ring_k, cF2);
+        v2 = face_cell(false, f2, g2c, cF2);
     }
     if (ring_face) vR = face_cell(ring_w, 0, ring_fk, cFR);
     // issued before the barrier: the loads are in flight while the
@@ -931,6 +1057,19 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
     if (vR) {
         if (ring_w) gR = face_geo(true, cFR);
         else gR = face_geo(false, cFR);
+    }
+    // split tiles: the BC entries on both sides of the thread's face as well
+    int bcl = 0, bcr = 0;
+    if (SPLIT && m.has_bc) {
+        if (v1) {
+            const int i = pi0 + 1 + f1, j = pj0 + 2 + g1r;
+            bcl = i == 1 ? bcW[j] : 0;
+            bcr = i == ICu ? bcE[j] : 0;
+        } else if (v2) {
+            const int i = pi0 + 2 + g2c, j = pj0 + 1 + f2;
+            bcl = j == 1 ? bcS[i] : 0;
+            bcr = j == JCu ? bcN[i] : 0;
+        }
     }
     __syncthreads();
 
@@ -957,15 +1096,15 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
             W = face_state(W, px, py, (FT)(xf - sX[jl][il]), (FT)(yf - sY[jl][il]));
         };
         PS<FT> Wl, Wr;
-        int bcL = 0, bcR = 0, slotL, slotR;
+        int bcL = bcl, bcR = bcr, slotL, slotR;
         if (idir) {
-            if (m.has_bc) {
+            if (!SPLIT && m.has_bc) {
                 bcL = (ipL == 1) ? bcW[jpL] : 0;
                 bcR = (ipL == ICu) ? bcE[jpL] : 0;
             }
             slotL = jpL; slotR = m.ncj + jpL;
         } else {
-            if (m.has_bc) {
+            if (!SPLIT && m.has_bc) {
                 bcL = (jpL == 1) ? bcS[ipL] : 0;
                 bcR = (jpL == JCu) ? bcN[ipL] : 0;
             }
@@ -1016,8 +1155,16 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
         const int st = ring_w ? TJ : TI;
         dst[0] = Fr.d; dst[st] = Fr.mx; dst[2 * st] = Fr.my; dst[3 * st] = Fr.E;
     }
-    if (v1) h1 = face(true, is_tile ? tc + 1 : 0, is_tile ? tr : ring_k, g1, F1);
-    if (v2) h2 = face(false, is_tile ? tr + 1 : 0, is_tile ? tc : ring_k, g2, F2);
+    if constexpr (SPLIT) {
+        // one face per thread, one copy of its code
+        if (v1 || v2) {
+            if (!v1) g1 = g2;
+            (v1 ? h1 : h2) = face(v1, v1 ? f1 : f2, v1 ? g1r : g2c, g1, F1);
+        }
+    } else {
+        if (v1) h1 = face(true, f1, g1r, g1, F1);
+        if (v2) h2 = face(false, f2, g2c, g2, F2);
+    }
 
     // phase-4 operands of the thread's cell: area, face lengths, time step,
     // U^n and the FP64 accumulator where the stage reads it.  Only this
@@ -1055,12 +1202,13 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
     if (valid) load4();
     __syncthreads();  // all gradient reads done: the flux arrays may now overwrite them
     if (h1) {
-        const int f = is_tile ? tc + 1 : 0, g = is_tile ? tr : ring_k;
+        const int f = f1, g = g1r;
         sFi[0][g][f] = F1.d; sFi[1][g][f] = F1.mx; sFi[2][g][f] = F1.my; sFi[3][g][f] = F1.E;
     }
     if (h2) {
-        const int f = is_tile ? tr + 1 : 0, g = is_tile ? tc : ring_k;
-        sFj[0][f][g] = F2.d; sFj[1][f][g] = F2.mx; sFj[2][f][g] = F2.my; sFj[3][f][g] = F2.E;
+        const int f = f2, g = g2c;
+        const CS<FT> &F = SPLIT ? F1 : F2;
+        sFj[0][f][g] = F.d; sFj[1][f][g] = F.mx; sFj[2][f][g] = F.my; sFj[3][f][g] = F.E;
     }
     __syncthreads();
 
@@ -1242,9 +1390,24 @@ __attribute__((amdgpu_waves_per_eu(StageWaves<FT, TI, TJ>::value))) void stage_k
     }
 }
 
+// Split tiles up to a cell for every lane of the chip (256 CUs x 4 SIMDs x 64): the
+// waves of a split launch, eleven for 16 x 8 cells, are then all resident, and each
+// is shorter.  Beyond, the extra work costs more than it hides.  ms per RK4 step,
+// split against not: 8 x 8 at 1,024 cells 0.049 / 0.074, 30,720 0.057 / 0.075,
+// 65,536 0.086 / 0.087, 98,304 0.117 / 0.107; 16 x 8 at 49,152 0.068 / 0.078,
+// 65,536 0.069 / 0.080, 81,920 0.093 / 0.091, 131,072 0.127 / 0.106.
+constexpr int SPLIT_CELLS = 65536;
 template <typename FT, int TI, int TJ, int KIND>
 inline void launch_stage_kernel(const StageParams *p, hipStream_t st) {
-    hipLaunchKernelGGL((stage_kernel<FT, TI, TJ, KIND>), dim3(p->ntiles), dim3((TileThreads<TI, TJ>::value)), 0, st, *p);
+    if constexpr (Splittable<FT, TI, TJ, KIND>::value) {
+        if (p->ntiles <= SPLIT_CELLS / (TI * TJ)) {
+            hipLaunchKernelGGL((stage_kernel<FT, TI, TJ, KIND, true>), dim3(p->ntiles),
+                               dim3((StageThreads<TI, TJ, true>::value)), 0, st, *p);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((stage_kernel<FT, TI, TJ, KIND>), dim3(p->ntiles), dim3((StageThreads<TI, TJ, false>::value)), 0, st,
+                       *p);
 }
 
 // Update of a tile from a stored residual: the second half of a fused stage
