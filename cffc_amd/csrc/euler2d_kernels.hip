@@ -739,6 +739,9 @@ __global__ void reset_keys_kernel(ErrorKeys keys) {
 }
 
 // small device-side scalar writes (graph-safe, no memset nodes)
+__global__ void copy_words_kernel(const unsigned long long *src, unsigned long long *dst, int n) {
+    if ((int)threadIdx.x < n) dst[threadIdx.x] = src[threadIdx.x];
+}
 __global__ void set_u64_kernel(unsigned long long *dst, unsigned long long v0, unsigned long long v1, int n) {
     if (threadIdx.x == 0) { dst[0] = v0; if (n > 1) dst[1] = v1; }
 }
@@ -876,6 +879,11 @@ hipError_t cffc_launch_reset_keys(const ErrorKeys *keys, hipStream_t st) {
 hipError_t cffc_launch_set_u64(unsigned long long *dst, unsigned long long v0, unsigned long long v1, int n,
                                hipStream_t st) {
     hipLaunchKernelGGL(set_u64_kernel, dim3(1), dim3(64), 0, st, dst, v0, v1, n);
+    return hipGetLastError();
+}
+
+hipError_t cffc_launch_copy_words(const unsigned long long *src, unsigned long long *dst, int n, hipStream_t st) {
+    hipLaunchKernelGGL(copy_words_kernel, dim3(1), dim3(64), 0, st, src, dst, n);
     return hipGetLastError();
 }
 

@@ -154,6 +154,7 @@ hipError_t cffc_launch_norms(const cffc::BlockMeta *meta, const cffc::TileDesc *
                              const cffc::ErrorKeys *keys, hipStream_t st);
 hipError_t cffc_launch_reset_keys(const cffc::ErrorKeys *keys, hipStream_t st);
 hipError_t cffc_launch_mg_step(const cffc::StageParams *p, int ti, int tj, hipStream_t st);
+hipError_t cffc_launch_copy_words(const unsigned long long *src, unsigned long long *dst, int n, hipStream_t st);
 hipError_t cffc_launch_set_u64(unsigned long long *dst, unsigned long long v0, unsigned long long v1, int n,
                                hipStream_t st);
 hipError_t cffc_launch_finish(const cffc::FinishParams *p, double *chunk_part, int nchunk, hipStream_t st);

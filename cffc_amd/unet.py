@@ -34,6 +34,7 @@ def _lib():
         L.cffc_unet_train_step.argtypes = [vp, pi32, i32, f, pf]
         L.cffc_unet_loss_grad.argtypes = [vp, pi32, i32, pf, i32, pf, pf]
         L.cffc_unet_predict.argtypes = [vp, pf, i32, pf]
+        L.cffc_unet_predict_all.argtypes = [vp, pf, i32, pf]
         L.cffc_unet_mfma_layout_probe.argtypes = [pf]
         L._unet_bound = True
     return L
@@ -121,9 +122,8 @@ class UNet:
     def predict(self, X):
         X = np.ascontiguousarray(X, dtype=np.float32)
         out = np.empty(X.shape[:3] + (NOUT,), dtype=np.float32)
-        for s in range(0, X.shape[0], self.max_batch):
-            xb, ob = X[s:s + self.max_batch], out[s:s + self.max_batch]
-            _check(_lib().cffc_unet_predict(self.h, _pf(xb), xb.shape[0], _pf(ob)), "predict")
+        if X.shape[0]:
+            _check(_lib().cffc_unet_predict_all(self.h, _pf(X), X.shape[0], _pf(out)), "predict")
         return out
 
     def train(self, nsteps, batch, lr=2e-3, seed=0, log_every=0):

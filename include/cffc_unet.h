@@ -58,6 +58,9 @@ int  cffc_unet_loss_grad(cffc_unet *net, const int32_t *idx, int batch, float *l
 
 /* Predict: inputs [batch][H][W][IN] host FP32 -> outputs [batch][H][W][OUT]. */
 int  cffc_unet_predict(cffc_unet *net, const float *inputs, int batch, float *outputs);
+/* The same for any number of samples, max_batch at a time, their copies beside
+   the computation. */
+int  cffc_unet_predict_all(cffc_unet *net, const float *inputs, int count, float *outputs);
 
 /* Check of the MFMA operand layout the kernels assume: D = A*B for a known
    16x32 and 32x16 pair computed on the device; out receives 64 lanes x 4
