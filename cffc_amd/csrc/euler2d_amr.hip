@@ -1,6 +1,6 @@
 // euler2d_amr.hip -- resolution changes of quadtree block meshes on gfx950.
 //
-// Three small list-driven kernels, one thread per operation.  The
+// Three small list-driven kernels, one thread per operation (prolongation: four).  The
 // restriction and prolongation run at the start of every stage, before the
 // BCs (and repeatedly while the ghosts of a new state are primed); the flux
 // correction runs between the residual and the update of the deferred tiles
@@ -77,85 +77,74 @@ __global__ __launch_bounds__(64) void restrict_kernel(const RestrictOp *ops, int
     amr_stW(W, ncp, o.dst, W_of_U(Ur));
 }
 
+// Four threads per coarse cell: each reconstructs one variable, then, after a
+// transpose over the quad, forms one of the four fine ghost states.  A thread that
+// did all four ran four limiters and four conversions in a chain (8.4 us a launch on
+// an explosion mesh of three levels and 16 x 16 roots, 5.0 us now); the lists are far
+// too short to fill the chip.
 template <typename ST>
 __global__ __launch_bounds__(64) void prolong_kernel(const ProlongOp *ops, int nops, const BlockMeta *meta,
                                                       const double *geom, const double *phi, int frozen,
                                                       const int32_t *part_state, int64_t ncp, ST *W,
                                                       const int32_t *stop_flag) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    const int q = (blockIdx.x * blockDim.x + threadIdx.x) / 4, v = threadIdx.x & 3;
     if (q >= nops || (stop_flag && *stop_flag)) return;
     // limiters frozen by the caller, or by a one-part steady run
     if (part_state && part_state[0] != PART_RUNNING) frozen = 1;
-    const ProlongOp o = ops[q];
+    const ProlongOp &o = ops[q];
     const int64_t c = o.src;
     const int64_t pitch = meta[o.blk].pitch;
     const double *G = geom;
-    const double xc0 = G[GEO_XC * ncp + c], yc0 = G[GEO_YC * ncp + c];
-    const PS<double> W0 = amr_ldW(W, ncp, c);
+    const ST *Wv = W + v * ncp;
+    const double xc0 = G[GEO_XC * ncp + c], yc0 = G[GEO_YC * ncp + c], w0 = (double)Wv[c];
     // the 8-point stencil in the reference's order
     const int64_t nb[8] = {c - pitch - 1, c - pitch, c - pitch + 1, c - 1, c + 1, c + pitch - 1, c + pitch,
                            c + pitch + 1};
-    double Dx[4] = {0, 0, 0, 0}, Dy[4] = {0, 0, 0, 0};
-    double DxDx = 0.0, DxDy = 0.0, DyDy = 0.0;
-    double wmin[4] = {W0.d, W0.vx, W0.vy, W0.p}, wmax[4] = {W0.d, W0.vx, W0.vy, W0.p};
-    const double w0[4] = {W0.d, W0.vx, W0.vy, W0.p};
+    double Dx = 0.0, Dy = 0.0, DxDx = 0.0, DxDy = 0.0, DyDy = 0.0, wmin = w0, wmax = w0;
 #pragma unroll
     for (int n2 = 0; n2 < 8; ++n2) {
         const int64_t cn = nb[n2];
         const double dXx = G[GEO_XC * ncp + cn] - xc0, dXy = G[GEO_YC * ncp + cn] - yc0;
-        const PS<double> Wn = amr_ldW(W, ncp, cn);
-        const double wn[4] = {Wn.d, Wn.vx, Wn.vy, Wn.p};
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const double DU = wn[v] - w0[v];
-            Dx[v] += DU * dXx;
-            Dy[v] += DU * dXy;
-            wmin[v] = wmin[v] < wn[v] ? wmin[v] : wn[v];   // min(u0Min, v), Math.h:73-92
-            wmax[v] = wmax[v] > wn[v] ? wmax[v] : wn[v];
-        }
+        const double wn = (double)Wv[cn], DU = wn - w0;
+        Dx += DU * dXx;
+        Dy += DU * dXy;
+        wmin = wmin < wn ? wmin : wn;   // min(u0Min, v), Math.h:73-92
+        wmax = wmax > wn ? wmax : wn;
         DxDx += dXx * dXx;
         DxDy += dXx * dXy;
         DyDy += dXy * dXy;
     }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { Dx[v] /= 8.0; Dy[v] /= 8.0; }
+    Dx /= 8.0; Dy /= 8.0;
     DxDx /= 8.0; DxDy /= 8.0; DyDy /= 8.0;
     const Recip<double> rdet = recip(DxDx * DyDy - DxDy * DxDy);
-    double gx[4], gy[4], ph[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        gx[v] = rdiv(Dx[v] * DyDy - Dy[v] * DxDy, rdet);
-        gy[v] = rdiv(Dy[v] * DxDx - Dx[v] * DxDy, rdet);
-    }
+    const double gx = rdiv(Dx * DyDy - Dy * DxDy, rdet), gy = rdiv(Dy * DxDx - Dx * DxDy, rdet);
+    double ph = 1.0;
     if (frozen) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) ph[v] = phi[v * ncp + c];
+        ph = phi[v * ncp + c];
     } else {
         // Limiter_Venkatakrishnan over the E, W, N, S face midpoints
         const double xE = G[GEO_XFE * ncp + c], yE = G[GEO_YFE * ncp + c];
         const double xW = G[GEO_XFE * ncp + c - 1], yW = G[GEO_YFE * ncp + c - 1];
         const double xN = G[GEO_XFN * ncp + c], yN = G[GEO_YFN * ncp + c];
         const double xS = G[GEO_XFN * ncp + c - pitch], yS = G[GEO_YFN * ncp + c - pitch];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const double u0 = w0[v];
-            double p = 1.0;
-            p = venkat_fold<double>(p, u0 + gx[v] * (xE - xc0) + gy[v] * (yE - yc0), u0, wmin[v], wmax[v]);
-            p = venkat_fold<double>(p, u0 + gx[v] * (xW - xc0) + gy[v] * (yW - yc0), u0, wmin[v], wmax[v]);
-            p = venkat_fold<double>(p, u0 + gx[v] * (xN - xc0) + gy[v] * (yN - yc0), u0, wmin[v], wmax[v]);
-            p = venkat_fold<double>(p, u0 + gx[v] * (xS - xc0) + gy[v] * (yS - yc0), u0, wmin[v], wmax[v]);
-            ph[v] = p;
-        }
+        ph = venkat_fold<double>(ph, w0 + gx * (xE - xc0) + gy * (yE - yc0), w0, wmin, wmax);
+        ph = venkat_fold<double>(ph, w0 + gx * (xW - xc0) + gy * (yW - yc0), w0, wmin, wmax);
+        ph = venkat_fold<double>(ph, w0 + gx * (xN - xc0) + gy * (yN - yc0), w0, wmin, wmax);
+        ph = venkat_fold<double>(ph, w0 + gx * (xS - xc0) + gy * (yS - yc0), w0, wmin, wmax);
     }
+    double r[4], t[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const double dXx = o.xq[k] - xc0, dXy = o.yq[k] - yc0;
-        double r[4];
+    for (int k = 0; k < 4; ++k) r[k] = w0 + (ph * gx) * (o.xq[k] - xc0) + (ph * gy) * (o.yq[k] - yc0);
+    // step s: the value for thread v ^ s leaves, variable v ^ s of ghost v arrives
 #pragma unroll
-        for (int v = 0; v < 4; ++v) r[v] = w0[v] + (ph[v] * gx[v]) * dXx + (ph[v] * gy[v]) * dXy;
-        const PS<double> Wq = {r[0], r[1], r[2], r[3]};
-        amr_stW(W, ncp, o.dst[k], W_of_U(U_of_W(Wq)));
+    for (int s = 0; s < 4; ++s) {
+        const int k = v ^ s;
+        const double x = __shfl_xor(k == 0 ? r[0] : k == 1 ? r[1] : k == 2 ? r[2] : r[3], s);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) t[u] = k == u ? x : t[u];
     }
+    const PS<double> Wq = {t[0], t[1], t[2], t[3]};
+    amr_stW(W, ncp, o.dst[v], W_of_U(U_of_W(Wq)));
 }
 
 __global__ __launch_bounds__(256) void flux_fix_kernel(const FluxFixOp *ops, int nops, double *S,
@@ -208,7 +197,7 @@ extern "C" hipError_t cffc_launch_prolong(const ProlongOp *ops, int nops, const 
                                           const double *phi, int frozen, const int32_t *part_state, int64_t ncp,
                                           double *W, float *Wf, const int32_t *stop_flag, hipStream_t st) {
     if (nops <= 0) return hipSuccess;
-    const int nb = (nops + 63) / 64;
+    const int nb = (nops + 15) / 16;
     if (Wf)
         hipLaunchKernelGGL((prolong_kernel<float>), dim3(nb), dim3(64), 0, st, ops, nops, meta, geom, phi, frozen,
                            part_state, ncp, Wf, stop_flag);
