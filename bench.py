@@ -439,7 +439,7 @@ def main():
     ap.add_argument("--cpu-threads", type=int, default=min(16, os.cpu_count() or 1))
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--precision", default="both", choices=["both", "mixed", "fp64"])
-    ap.add_argument("--no-autotune", action="store_true", help="keep the default 16x8 tile")
+    ap.add_argument("--no-autotune", action="store_true", help="keep a 16x8 tile")
     ap.add_argument("--tile", default=None, metavar="TIxTJ", help="use this tile shape (no autotuning)")
     ap.add_argument("--error-steps", type=int, default=500,
                     help="steps of the mixed-vs-FP64 error runs (0: skip)")
@@ -487,7 +487,7 @@ def main():
     res = {}
     precs = ["mixed", "fp64"] if args.precision == "both" else [args.precision]
     for prec in precs:
-        tile, tune = (16, 8), {}   # the library's default tile
+        tile, tune = (16, 8), {}   # without autotuning or --tile
         if args.tile:
             tile = tuple(int(x) for x in args.tile.lower().split("x"))
         elif not args.no_autotune:
