@@ -2408,8 +2408,8 @@ static int mg_first_level(const cffc_ctx *c, const cffc_mesh_desc *md, FirstLeve
         HIPCHK(hipMemcpy(f.faces, faces.data(), faces.size() * sizeof(MgFace), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(f.groups, ends.data(), ends.size() * sizeof(int32_t), hipMemcpyHostToDevice));
         f.ngroup = (int)groups.size();
-        // a thread per face up to the largest workgroup, two beyond
-        f.nt = (std::min(std::max(max_group, max_faces), 1024) + 63) / 64 * 64;
+        // a thread per face up to the largest workgroup
+        f.nt = (std::min(std::max(max_group, max_faces), 512) + 63) / 64 * 64;
     }
     return 0;
 }

@@ -105,7 +105,7 @@ struct MgFace {
     int16_t l, r;
     int32_t e, north;
 };
-enum { MG_GROUP_CELLS = 1024, MG_GROUP_FACES = 2048, MG_GROUP_EDGES = 512 };   // edges: faces on boundaries
+enum { MG_GROUP_CELLS = 512, MG_GROUP_FACES = 1536, MG_GROUP_EDGES = 256 };   // edges: faces on boundaries
 struct GroupArgs {
     const int32_t *groups;   // first cell, face and boundary face of every group, and the ends
     const MgFace *faces;

@@ -367,16 +367,19 @@ __global__ __launch_bounds__(256) void mg_first_step_kernel(FirstArgs a, double 
 }
 
 // All smoothings of a level whose connected groups of blocks are small (at most
-// MG_GROUP_CELLS cells, MG_GROUP_FACES faces), in one launch: a workgroup per
-// group.  nsm smoothings of a.nstage stages; each starts with the cell's CFL time
-// step and the finer level's rule (cfl_kernel).  In a stage a thread first
-// evaluates one or two faces of the group's list into LDS, then updates its cell
-// from its four faces; W, the fluxes, the faces' normals and the boundaries' states live in LDS (155 of
-// 160 KB), the cells' geometry and U in registers.  A wave alone on its SIMD is bound by the flux's own dependent
-// instructions, so faces, not cells, are spread over the threads: 15 stages of
-// 48 cells 65 -> 58 us, of 768 cells (64 cases at once) 151 -> 140 us against a
-// thread per cell that evaluates its four faces.
-__global__ __launch_bounds__(1024) void mg_first_smooth_kernel(FirstArgs a, GroupArgs ga, int nsm, FineLevel fl) {
+// MG_GROUP_CELLS cells, MG_GROUP_FACES faces, MG_GROUP_EDGES of them on boundaries),
+// in one launch: a workgroup per group.  nsm smoothings of a.nstage stages; each
+// starts with the cell's CFL time step and the finer level's rule (cfl_kernel).
+// In a stage a thread first evaluates one to three faces of the group's list into
+// LDS, then updates its cell from its four faces; W, the fluxes, the faces' normals
+// and the boundaries' states live in LDS (102 of 160 KB), the cells' geometry and U
+// in registers.  A wave alone on its SIMD is bound by the flux's own dependent
+// instructions, so faces, not cells, are spread over the threads.  15 stages of 192
+// cells take 52 us, 3.4 us each, against 6.7 us for a launch per stage; of 768 cells
+// (16 waves at 128 registers, some spilled) 10 us each, no less than by launches:
+// hence the limit of 512 cells and threads (40 cycles of one case 16.4 -> 15.3 ms; 64
+// cases of up to 768 cells on that level 28.0 and 28.3 ms, runs differing by 0.5%).
+__global__ __launch_bounds__(512) void mg_first_smooth_kernel(FirstArgs a, GroupArgs ga, int nsm, FineLevel fl) {
     __shared__ double sW[4][MG_GROUP_CELLS], sF[4][MG_GROUP_FACES], sn[2][MG_GROUP_FACES];
     __shared__ double swo[4][MG_GROUP_EDGES];
     __shared__ int16_t sLR[2][MG_GROUP_FACES];   // negative: the boundary's kind, -1 ... -4
@@ -433,8 +436,7 @@ __global__ __launch_bounds__(1024) void mg_first_smooth_kernel(FirstArgs a, Grou
     double dtl = 0.0;
     if (on) { sW[0][t] = W.d; sW[1][t] = W.vx; sW[2][t] = W.vy; sW[3][t] = W.p; }
     for (int nu = 0; nu < nsm; ++nu) {
-        // the normals are read again rather than held: 1,024 threads have 128
-        // registers each
+        // the normals are read again rather than held in registers
         const double d_i = 2.0 * qdiv(A, lE + lW), d_j = 2.0 * qdiv(A, lN + lS);
         const double v_i = 0.5 * (W.vx * (G[GEO_NEX * ncp + c] - -G[GEO_NEX * ncp + wc]) +
                                   W.vy * (G[GEO_NEY * ncp + c] - -G[GEO_NEY * ncp + wc]));

@@ -1,7 +1,7 @@
 """The multigrid cycle's one-launch smoothing stages: tile windows that form
 their own ghost cells (blocks no tile divides, many workgroups on the state
 they update), first-order levels by cell list (connected blocks of more and of
-fewer than 1,024 cells, disjoint meshes, blocks of 2 x 2 cells), every boundary
+fewer cells than one workgroup takes, disjoint meshes, blocks of 2 x 2 cells), every boundary
 type on every side, repeated smoothings, and start-up on a coarse level that
 keeps the full scheme.  Bitwise against the oracle."""
 import numpy as np
@@ -20,8 +20,9 @@ SIDES = [(F, E, R, R), (C, F, E, R), (R, C, F, E), (E, R, C, F)]
 # blocks, cells of one, levels: coarsest cells of a connected mesh in brackets
 MESHES = [((1, 1, 8, 8), 3),      # [4] one block of 2 x 2
           ((3, 2, 40, 24), 3),    # [360] 10 x 6
-          ((2, 2, 64, 64), 3),    # [1024] 16 x 16
-          ((3, 3, 44, 24), 2),    # [2376] 22 x 12: listed, stage by stage
+          ((2, 1, 64, 64), 3),    # [512] 16 x 16: the largest in one workgroup
+          ((2, 2, 64, 64), 3),    # [1024] listed, stage by stage
+          ((3, 3, 44, 24), 2),    # [2376] 22 x 12
           ((2, 1, 72, 136), 3)]   # [1224] 18 x 34
 
 
