@@ -2579,7 +2579,7 @@ static int mg_step(cffc_ctx *c, int i_stage, int pull, const double *P) {
 }
 
 // n smoothings of a first-order level over its cell list: one launch for all
-// of them where its groups fit a workgroup, else one per stage after the CFL
+// of them where its groups fit a workgroup, else one per stage
 static int mg_smooth_first(cffc_mg *mg, int top, int l, int n, const double *P) {
     cffc_ctx *c = mg->lv[l];
     const FirstLevel &fl = mg->first[l];
@@ -2602,21 +2602,19 @@ static int mg_smooth_first(cffc_mg *mg, int top, int l, int n, const double *P) 
     for (int st = 1; st <= c->s.n_stage; ++st) a.omega[st - 1] = stage_omega(c->s, st);
     a.halve = c->s.local_time_stepping == CFFC_SCALAR_LOCAL_TIME_STEPPING;
     a.err = c->scal + 2;
+    const FineLevel fine = {f ? f->meta : nullptr, f ? f->dt : nullptr, f ? area(f) : nullptr};
     if (fl.ngroup) {
         a.Win = c->W[c->wcur];
         a.Wout = c->W[c->wcur];
-        const FineLevel fine = {f ? f->meta : nullptr, f ? f->dt : nullptr, f ? area(f) : nullptr};
         const GroupArgs ga = {fl.groups, fl.faces, fl.cell_faces};
         HIPCHK(cffc_launch_mg_first_smooth(&a, &ga, fl.ngroup, fl.nt, n, &fine, c->stream));
         return 0;
     }
     for (int nu = 0; nu < n; ++nu) {
-        HIPCHK(cffc_launch_cfl(c->meta, c->tiles, c->ntiles, c->ti, c->tj, c->W[c->wcur], c->geom, c->ncp, c->dt,
-                               nullptr, f ? f->meta : nullptr, f ? f->dt : nullptr, f ? area(f) : nullptr, c->stream));
         for (int st = 1; st <= c->s.n_stage; ++st) {
             a.Win = c->W[c->wcur];
             a.Wout = c->W[1 - c->wcur];
-            HIPCHK(cffc_launch_mg_first_step(&a, a.omega[st - 1], st == 1, c->stream));
+            HIPCHK(cffc_launch_mg_first_step(&a, a.omega[st - 1], st == 1, &fine, c->stream));
             c->wcur = 1 - c->wcur;
         }
     }

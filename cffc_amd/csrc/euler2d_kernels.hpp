@@ -186,7 +186,8 @@ hipError_t cffc_launch_mg_copy(const cffc::BlockMeta *meta, int nblk, int max_ce
                                int64_t ncp, hipStream_t st);
 hipError_t cffc_launch_mg_restrict_wo(const cffc::BlockMeta *mf, const cffc::BlockMeta *mc, int nblk, int max_faces,
                                       const double *Af, const double *wf, double *wc, hipStream_t st);
-hipError_t cffc_launch_mg_first_step(const cffc::FirstArgs *a, double omega, int first_stage, hipStream_t st);
+hipError_t cffc_launch_mg_first_step(const cffc::FirstArgs *a, double omega, int first_stage, const cffc::FineLevel *fl,
+                                     hipStream_t st);
 // nt threads, at least a group's cells and half its faces
 hipError_t cffc_launch_mg_first_smooth(const cffc::FirstArgs *a, const cffc::GroupArgs *ga, int ngroup, int nt, int nsm,
                                        const cffc::FineLevel *fl, hipStream_t st);

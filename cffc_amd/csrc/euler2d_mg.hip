@@ -321,8 +321,28 @@ __device__ __forceinline__ PS<double> ldW4(const double *W, int64_t ncp, int64_t
     return {W[c], W[ncp + c], W[2 * ncp + c], W[3 * ncp + c]};
 }
 
-// one smoothing stage of a level, one thread per cell, from Win to Wout
-__global__ __launch_bounds__(256) void mg_first_step_kernel(FirstArgs a, double om, int first_stage) {
+// CFL_Multigrid: the finer level's bound on a cell's time step
+__device__ __forceinline__ double first_dt_fine(const FineLevel &fl, const MgCell &k, double A) {
+    const BlockMeta m = fl.meta[k.blk];
+    const int i = k.ji & 0xFFFF, j = k.ji >> 16;
+    const int64_t sw = cell(m, 2 * (i - 2) + 2, 2 * (j - 2) + 2), se = sw + 1, nw = sw + m.pitch, ne = nw + 1;
+    const double dt_NE = qsqrt(qdiv(A, fl.A[ne])) * fl.dt[ne], dt_SE = qsqrt(qdiv(A, fl.A[se])) * fl.dt[se];
+    const double dt_NW = qsqrt(qdiv(A, fl.A[nw])) * fl.dt[nw], dt_SW = qsqrt(qdiv(A, fl.A[sw])) * fl.dt[sw];
+    return dmin(dt_NE, dmin(dt_SE, dmin(dt_NW, dt_SW)));
+}
+// cfl_kernel's time step; s?i, s?j: sums of the opposite faces' normals
+__device__ __forceinline__ double first_dt(const PS<double> &W, double A, double lW, double lE, double lS, double lN,
+                                           double sxi, double syi, double sxj, double syj) {
+    const double d_i = 2.0 * qdiv(A, lE + lW), d_j = 2.0 * qdiv(A, lN + lS);
+    const double v_i = 0.5 * (W.vx * sxi + W.vy * syi), v_j = 0.5 * (W.vx * sxj + W.vy * syj);
+    const double so = W_a(W);
+    return dmin(qdiv(d_i, so + fabs(v_i)), qdiv(d_j, so + fabs(v_j)));
+}
+
+// One smoothing stage of a level, one thread per cell, from Win to Wout.  The first
+// one of a smoothing forms the time step from the geometry it has loaded anyway; as
+// a launch of its own that took 4 us (one case) to 18 us (64 cases).
+__global__ __launch_bounds__(256) void mg_first_step_kernel(FirstArgs a, double om, int first_stage, FineLevel fl) {
     const int q = blockIdx.x * 256 + threadIdx.x;
     if (q >= a.n) return;
     const MgCell k = a.cells[q];
@@ -337,7 +357,13 @@ __global__ __launch_bounds__(256) void mg_first_step_kernel(FirstArgs a, double 
     for (int s = 0; s < 4; ++s) Wn[s] = ldW4(a.Win, ncp, nb[s] >= 0 ? nb[s] : k.c);
     load_geometry(a, k, f);
     const CS<double> U0 = ldU(first_stage ? a.U : a.Uo, ncp, c);
-    double P[4] = {0.0, 0.0, 0.0, 0.0}, dtl = a.dt[c], dU[4];
+    double P[4] = {0.0, 0.0, 0.0, 0.0}, dtl, dU[4];
+    if (first_stage) {
+        dtl = first_dt(f.W, f.A, f.lW, f.lE, f.lS, f.lN, f.nEx - -f.nWx, f.nEy - -f.nWy, f.nNx - -f.nSx, f.nNy - -f.nSy);
+        if (fl.meta) dtl = dmin(dtl, first_dt_fine(fl, k, f.A));
+    } else {
+        dtl = a.dt[c];
+    }
     if (a.P) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) P[v] = a.P[v * ncp + c];
@@ -360,7 +386,7 @@ __global__ __launch_bounds__(256) void mg_first_step_kernel(FirstArgs a, double 
     }
     CS<double> Un;
     const PS<double> w = first_update(a, k, U0, om, f.W, dtl, dU, Un);
-    if (dtl != dt0) a.dt[c] = dtl;
+    if (first_stage || dtl != dt0) a.dt[c] = dtl;
     stU(a.U, ncp, c, Un);
     if (first_stage) stU(a.Uo, ncp, c, U0);
     a.Wout[c] = w.d; a.Wout[ncp + c] = w.vx; a.Wout[2 * ncp + c] = w.vy; a.Wout[3 * ncp + c] = w.p;
@@ -422,28 +448,15 @@ __global__ __launch_bounds__(512) void mg_first_smooth_kernel(FirstArgs a, Group
     const double lW = G[GEO_LE * ncp + wc], lE = G[GEO_LE * ncp + c], lS = G[GEO_LN * ncp + sc], lN = G[GEO_LN * ncp + c];
     const double A = G[GEO_A * ncp + c];
     const Recip<double> rA = recip(A);
-    // the finer level's part of the time step (CFL_Multigrid)
-    double dtf = MILLION;
     const bool fine = fl.meta != nullptr;
-    if (fine) {
-        const BlockMeta m = fl.meta[k.blk];
-        const int i = k.ji & 0xFFFF, j = k.ji >> 16;
-        const int64_t sw = cell(m, 2 * (i - 2) + 2, 2 * (j - 2) + 2), se = sw + 1, nw = sw + m.pitch, ne = nw + 1;
-        const double dt_NE = qsqrt(qdiv(A, fl.A[ne])) * fl.dt[ne], dt_SE = qsqrt(qdiv(A, fl.A[se])) * fl.dt[se];
-        const double dt_NW = qsqrt(qdiv(A, fl.A[nw])) * fl.dt[nw], dt_SW = qsqrt(qdiv(A, fl.A[sw])) * fl.dt[sw];
-        dtf = dmin(dt_NE, dmin(dt_SE, dmin(dt_NW, dt_SW)));
-    }
+    const double dtf = fine ? first_dt_fine(fl, k, A) : MILLION;
     double dtl = 0.0;
     if (on) { sW[0][t] = W.d; sW[1][t] = W.vx; sW[2][t] = W.vy; sW[3][t] = W.p; }
     for (int nu = 0; nu < nsm; ++nu) {
         // the normals are read again rather than held in registers
-        const double d_i = 2.0 * qdiv(A, lE + lW), d_j = 2.0 * qdiv(A, lN + lS);
-        const double v_i = 0.5 * (W.vx * (G[GEO_NEX * ncp + c] - -G[GEO_NEX * ncp + wc]) +
-                                  W.vy * (G[GEO_NEY * ncp + c] - -G[GEO_NEY * ncp + wc]));
-        const double v_j = 0.5 * (W.vx * (G[GEO_NNX * ncp + c] - -G[GEO_NNX * ncp + sc]) +
-                                  W.vy * (G[GEO_NNY * ncp + c] - -G[GEO_NNY * ncp + sc]));
-        const double so = W_a(W);
-        dtl = dmin(qdiv(d_i, so + fabs(v_i)), qdiv(d_j, so + fabs(v_j)));
+        dtl = first_dt(W, A, lW, lE, lS, lN, G[GEO_NEX * ncp + c] - -G[GEO_NEX * ncp + wc],
+                       G[GEO_NEY * ncp + c] - -G[GEO_NEY * ncp + wc], G[GEO_NNX * ncp + c] - -G[GEO_NNX * ncp + sc],
+                       G[GEO_NNY * ncp + c] - -G[GEO_NNY * ncp + sc]);
         if (fine) dtl = dmin(dtl, dtf);
         U0 = U;
         for (int st = 0; st < a.nstage; ++st) {
@@ -525,8 +538,9 @@ extern "C" hipError_t cffc_launch_mg_restrict_wo(const BlockMeta *mf, const Bloc
     hipLaunchKernelGGL(mg_restrict_wo_kernel, dim3(nblk, (max_faces + 63) / 64), dim3(64), 0, st, mf, mc, Af, wf, wc);
     return hipGetLastError();
 }
-extern "C" hipError_t cffc_launch_mg_first_step(const FirstArgs *a, double omega, int first_stage, hipStream_t st) {
-    hipLaunchKernelGGL(mg_first_step_kernel, dim3((a->n + 255) / 256), dim3(256), 0, st, *a, omega, first_stage);
+extern "C" hipError_t cffc_launch_mg_first_step(const FirstArgs *a, double omega, int first_stage, const FineLevel *fl,
+                                       hipStream_t st) {
+    hipLaunchKernelGGL(mg_first_step_kernel, dim3((a->n + 255) / 256), dim3(256), 0, st, *a, omega, first_stage, *fl);
     return hipGetLastError();
 }
 extern "C" hipError_t cffc_launch_mg_first_smooth(const FirstArgs *a, const GroupArgs *ga, int ngroup, int nt, int nsm,
