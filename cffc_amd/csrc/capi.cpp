@@ -2542,12 +2542,16 @@ static int mg_stage(cffc_ctx *c, int i_stage, int residual, const double *P, dou
 // Whether a level's smoothing stages can each be one launch (SK_STEP): the
 // kernel fills its own ghost cells (no periodic boundary), every stage starts
 // from a zero residual (multistage optimal smoothing) and nothing runs between
-// the residual and the update.
+// the residual and the update.  With an exchange, a residual and an update launch
+// a stage, 40 cycles of one case took 42.1 ms and 12 cycles of 64 serving cases
+// 54.9 ms; 22.3 and 39.8 ms so, with the transfers' launches merged.
 static bool mg_one_launch(const cffc_mg *mg, const cffc_ctx *c) {
     return c->windowable && mg->rs_iters == 0 && !c->s.axisymmetric &&
            c->s.i_time_integration == CFFC_TIME_STEPPING_MULTISTAGE_OPTIMAL_SMOOTHING &&
            c->s.i_flux_function != CFFC_FLUX_FUNCTION_HLLE && c->s.i_limiter == CFFC_LIMITER_VENKATAKRISHNAN;
 }
+// ... and whether a first-order level runs over its cell list (from 22.3 to 15.3 and
+// from 39.8 to 36.5 ms)
 static bool mg_listed(const cffc_mg *mg, const cffc_ctx *c, int l) {
     return mg->first[l].n && mg->rs_iters == 0 && !c->s.axisymmetric &&
            c->s.i_time_integration == CFFC_TIME_STEPPING_MULTISTAGE_OPTIMAL_SMOOTHING &&
