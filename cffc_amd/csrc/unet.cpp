@@ -92,10 +92,14 @@ struct cffc_unet {
     std::vector<void *> allocs;
 };
 
+// Cleared when it returns: hipMemset of device memory only enqueues on the null
+// stream, which the network's streams (hipStreamNonBlocking) do not wait for, so
+// a clear could otherwise run after their first writes.
 static int ualloc(cffc_unet *n, void **p, size_t bytes) {
     if (hipMalloc(p, bytes) != hipSuccess) return ufail(CFFC_E_NOMEM, "hipMalloc(%zu) failed", bytes);
     n->allocs.push_back(*p);
-    if (hipMemset(*p, 0, bytes) != hipSuccess) return ufail(CFFC_E_HIP, "hipMemset failed");
+    if (hipMemset(*p, 0, bytes) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess)
+        return ufail(CFFC_E_HIP, "hipMemset failed");
     return 0;
 }
 
@@ -472,7 +476,6 @@ static int ensure_pipeline(cffc_unet *n) {
         if (!*q) UCHK(hipStreamCreateWithFlags(q, hipStreamNonBlocking));
     for (hipEvent_t &q : n->computed)
         if (!q) UCHK(hipEventCreateWithFlags(&q, hipEventDisableTiming));
-    UCHK(hipStreamSynchronize(nullptr));   // ualloc's clears
     return 0;
 }
 

@@ -1,0 +1,31 @@
+"""The U-Net's host runtime (cffc_amd/csrc/unet.cpp) compiled against a
+stand-in for the HIP runtime that runs null-stream work as late and the
+network's own streams as early as their ordering allows
+(tests/native/unet_runtime_check.cpp)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+SRC = os.path.join(ROOT, "tests", "native", "unet_runtime_check.cpp")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+
+@pytest.fixture(scope="module")
+def checker(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("g++ not available")
+    exe = str(tmp_path_factory.mktemp("unet") / "unet_runtime_check")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(ROCM, "include"),
+                    "-o", exe, SRC, "-lpthread"], check=True)
+    return exe
+
+
+# create: no buffer is cleared after the network has been handed out;
+# order: a dataset's samples and targets are not cleared after they were stored
+@pytest.mark.parametrize("what", ["create", "order"])
+def test_runtime(checker, what):
+    r = subprocess.run([checker, what], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
