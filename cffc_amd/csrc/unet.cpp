@@ -323,12 +323,15 @@ extern "C" int cffc_unet_set_weights(cffc_unet *n, int l, const float *w, const 
 extern "C" int cffc_unet_set_dataset(cffc_unet *n, int ns, const float *inputs, const float *targets) {
     if (!n || ns <= 0 || !inputs || !targets) return ufail(CFFC_E_ARG, "bad dataset");
     const size_t per_in = (size_t)n->H * n->W * CFFC_UNET_IN, per_tg = (size_t)n->H * n->W * CFFC_UNET_OUT;
-    if (n->ds_in) {
-        (void)hipFree(n->ds_in);
-        (void)hipFree(n->ds_tg);
-        n->allocs.erase(std::remove(n->allocs.begin(), n->allocs.end(), (void *)n->ds_in), n->allocs.end());
-        n->allocs.erase(std::remove(n->allocs.begin(), n->allocs.end(), (void *)n->ds_tg), n->allocs.end());
+    // a call that fails from here on leaves the network without a dataset
+    n->ds_n = 0;
+    for (void *q : {(void *)n->ds_in, (void *)n->ds_tg}) {
+        if (!q) continue;
+        (void)hipFree(q);
+        n->allocs.erase(std::remove(n->allocs.begin(), n->allocs.end(), q), n->allocs.end());
     }
+    n->ds_in = nullptr;
+    n->ds_tg = nullptr;
     int e;
     if ((e = ualloc(n, (void **)&n->ds_in, per_in * ns * 2)) || (e = ualloc(n, (void **)&n->ds_tg, per_tg * ns * 4))) return e;
     // rounded to BF16 on the device, max_batch samples at a time

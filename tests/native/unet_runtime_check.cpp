@@ -10,7 +10,7 @@
 
 static std::map<char *, size_t> live;                 // device allocations
 static std::vector<std::function<void()>> null_work;  // not run yet
-static size_t malloc_limit = ~(size_t)0;
+static int mallocs_left = -1;                         // allocations that succeed; -1: all
 
 static void drain() {
     for (auto &w : null_work) w();
@@ -29,7 +29,8 @@ hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 const char *hipGetErrorString(hipError_t) { return "error"; }
 hipError_t hipMalloc(void **p, size_t n) {
-    if (n > malloc_limit) return hipErrorOutOfMemory;
+    if (mallocs_left == 0) return hipErrorOutOfMemory;
+    if (mallocs_left > 0) --mallocs_left;
     *p = malloc(n);
     memset(*p, 0xA5, n);
     live[(char *)*p] = n;
@@ -146,10 +147,24 @@ int main(int argc, char **argv) {
             CHECK(n->ds_in[i] == (bf16_t)(u >> 16));
         }
         CHECK(memcmp(n->ds_tg, y.data(), y.size() * 4) == 0);
+    } else if (what == "dataset") {
+        const int32_t idx[2] = {0, NS - 1};
+        float loss;
+        for (int ok : {0, 1}) {   // neither buffer of the new dataset can be allocated, or only the first
+            CHECK(cffc_unet_set_dataset(n, NS, x.data(), y.data()) == 0);
+            CHECK(cffc_unet_train_step(n, idx, 2, 1e-3f, &loss) == 0);
+            mallocs_left = ok;
+            CHECK(cffc_unet_set_dataset(n, NS, x.data(), y.data()) == CFFC_E_NOMEM);
+            mallocs_left = -1;
+            CHECK(cffc_unet_train_step(n, idx, 2, 1e-3f, &loss) == CFFC_E_ARG);   // no dataset
+        }
+        CHECK(cffc_unet_set_dataset(n, NS, x.data(), y.data()) == 0);
+        CHECK(cffc_unet_train_step(n, idx, 2, 1e-3f, &loss) == 0);
     } else {
         return 2;
     }
     cffc_unet_destroy(n);
+    CHECK(live.empty());
     printf("ok\n");
     return 0;
 }

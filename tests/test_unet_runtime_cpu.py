@@ -24,8 +24,10 @@ def checker(tmp_path_factory):
 
 
 # create: no buffer is cleared after the network has been handed out;
-# order: a dataset's samples and targets are not cleared after they were stored
-@pytest.mark.parametrize("what", ["create", "order"])
+# order: a dataset's samples and targets are not cleared after they were stored;
+# dataset: after a dataset that could not be stored there is none, and its
+# predecessor's buffers are neither read nor freed again
+@pytest.mark.parametrize("what", ["create", "order", "dataset"])
 def test_runtime(checker, what):
     r = subprocess.run([checker, what], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
