@@ -112,6 +112,9 @@ struct cffc_ctx {
     bool windowable = false, window_bcs = false;   // could, and does where it is faster
     int nbc = 0;
     int32_t *bc_blocks = nullptr;
+    // changes of what a recorded launch of this context holds (tile arrays, the
+    // limiters' mode); a multigrid solver records its cycle again after one
+    long long recorded_gen = 0;
     // resolution changes (quadtree meshes): level-change legs of the exchange
     // and the conservative flux correction, as operation lists
     bool amr = false;
@@ -182,6 +185,7 @@ static int build_tiles(cffc_ctx *c, int ti, int tj) {
         for (int j0 = 0; j0 < m.nj; j0 += tj)
             for (int i0 = 0; i0 < m.ni; i0 += ti) t.push_back(TileDesc{b, i0, j0, part});
     }
+    c->recorded_gen++;
     if (c->tiles) (void)hipFree(c->tiles);
     if (c->norm_part) (void)hipFree(c->norm_part);
     if (c->part_tile0) (void)hipFree(c->part_tile0);
@@ -1494,6 +1498,7 @@ extern "C" int cffc_freeze_limiters(cffc_ctx *c, int freeze) {
     if (!c) return fail(CFFC_E_ARG, "null context");
     if (freeze && !c->phi_valid) return fail(CFFC_E_ARG, "no evaluated limiters to freeze (run a stage first)");
     c->freeze = freeze ? 1 : 0;
+    c->recorded_gen++;
     return 0;
 }
 
@@ -2228,12 +2233,15 @@ struct cffc_mg {
     // the smoother's scheme (top level) and the one below the top level
     cffc_scheme_desc fine_s{}, coarse_s{};
     // Execute replays one captured cycle (kernels only); recaptured when the
-    // limiters freeze (the stage kernels' phi mode changes) or the top level
-    // changes
+    // limiters freeze (the stage kernels' phi mode changes), the top level
+    // changes, or a setter has changed what the nodes hold: the parts' arrays
+    // and the residual smoothing (setting_gen), a level's tiles and limiters
+    // (its recorded_gen)
     bool use_graph = true;
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     int graph_frozen = -1, graph_top = -1, graph_base = -1;
+    long long setting_gen = 0, graph_gen = -1;
     // norms of the top level and the levels' error keys of the last check, and
     // the parts' norms, in pinned host memory (written by the kernels)
     double *status = nullptr;
@@ -2500,6 +2508,7 @@ extern "C" int cffc_mg_set_residual_smoothing(cffc_mg *mg, double epsilon, int i
     if (!mg || iterations < 0 || !(epsilon >= 0.0)) return fail(CFFC_E_ARG, "bad argument");
     mg->rs_eps = epsilon;
     mg->rs_iters = iterations;
+    mg->setting_gen++;
     return 0;
 }
 
@@ -2797,8 +2806,8 @@ extern "C" int cffc_mg_set_graph(cffc_mg *mg, int on) {
 }
 
 // enqueue one cycle from a top level: a replay of the captured cycle,
-// captured first (and again after the limiters freeze or the top level
-// changes), or the launches themselves
+// captured first (and again where what it recorded is no longer current), or
+// the launches themselves
 static int mg_enqueue_cycle(cffc_mg *mg, int top) {
     cffc_ctx *f = mg->lv[0];
     mg->base = mg->lv[top]->wcur;
@@ -2806,7 +2815,11 @@ static int mg_enqueue_cycle(cffc_mg *mg, int top) {
         if (int e = mg_reset_errors(mg)) return e;
         return mg_cgc(mg, top, top);
     }
-    if (!mg->gexec || mg->graph_frozen != (int)mg->frozen || mg->graph_top != top || mg->graph_base != mg->base) {
+    // counters that only grow: the sum is the same only if each of them is
+    long long gen = mg->setting_gen;
+    for (const cffc_ctx *c : mg->lv) gen += c->recorded_gen;
+    if (!mg->gexec || mg->graph_frozen != (int)mg->frozen || mg->graph_top != top || mg->graph_base != mg->base ||
+        mg->graph_gen != gen) {
         if (mg->gexec) (void)hipGraphExecDestroy(mg->gexec);
         if (mg->graph) (void)hipGraphDestroy(mg->graph);
         mg->gexec = nullptr;
@@ -2821,6 +2834,7 @@ static int mg_enqueue_cycle(cffc_mg *mg, int top) {
         mg->graph_frozen = (int)mg->frozen;
         mg->graph_top = top;
         mg->graph_base = mg->base;
+        mg->graph_gen = gen;
     }
     HIPCHK(hipGraphLaunch(mg->gexec, f->stream));
     return 0;
@@ -2860,6 +2874,7 @@ extern "C" int cffc_mg_set_parts(cffc_mg *mg, int npart, const int32_t *first_bl
                                  const double *freeze) {
     if (!mg) return fail(CFFC_E_ARG, "null argument");
     cffc_ctx *f = mg->lv[0];
+    mg->setting_gen++;
     for (cffc_ctx *c : mg->lv) {
         c->mg_part_of_block = nullptr;
         c->mg_part_frozen = nullptr;
