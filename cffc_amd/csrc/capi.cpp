@@ -1023,33 +1023,44 @@ extern "C" int cffc_create(const cffc_mesh_desc *md, const cffc_scheme_desc *sd,
             return e;
         }
     }
-    // Default tile.  A launch with fewer 16 x 8 tiles than compute units is
-    // latency-bound and takes 8 x 8 tiles; up to 1,280 of them (five
-    // resident workgroups on each of 256 units, 164 k cells) 16 x 8 spreads the
-    // work best; beyond, blocks at least 32 cells wide take the larger ring-pass
-    // tiles, which recompute fewer ring cells: 32 x 16 (FP64; mixed up to 1.5 M
-    // cells), 32 x 8 (mixed).  Narrower blocks stay with 16 x 8, in FP64 except
-    // for the stretch in which it has just begun a second round and 16 x 16 (four
-    // resident of half as many tiles) still fits one: 197 k cells of 16^2 blocks,
-    // five stages, 16x16 0.179 ms, 16x8 0.204.  Per RK4 step in blocks of 64^2, FP64: 16 k cells
-    // 8x8 0.071, 16x8 0.071, 32x16 0.094 ms; 66 k 16x8 0.078, 8x8 0.084, 32x16
-    // 0.095; 147 k 0.119 / 32x16 0.129; 262 k 32x16 0.140 / 16x8 0.163; 2.2 M
-    // 0.885 / 0.961.  Blocks of 16^2: 16 k cells 8x8 0.071, 16x8 0.075; 66 k
-    // 0.087 / 0.085.  Mixed, 64^2: 66 k 16x8 0.064, 32x8 0.068; 262 k 32x16
-    // 0.094, 32x8 0.100, 16x8 0.104; 2.2 M 32x8 0.506, 32x16 0.510.
-    // 8 x 8 for blocks narrower than 16 cells; in FP64, 4 x 4 (one wavefront
-    // per block) for blocks narrower than 8 cells.
+    // Default tile, by the number of tiles of a launch (256 compute units).  ms per
+    // RK4 step, graph replays, blocks of the size given.
+    // * FP64 8 x 8 while every tile has a unit to itself, mixed below 256 tiles of
+    //   16 x 8: such launches are bound by a thread's chain.  FP64, 24^2: 189 tiles of
+    //   8 x 8 0.049 (16 x 8 0.053), 297 0.057 (0.054); 30^2: 256 0.049 (0.054).  Mixed,
+    //   16^2: 1 k cells 0.064 (0.066), 25 k 0.064 (0.065); 33^2: 4 k 0.066 (0.070),
+    //   17 k 0.066 (0.064); 64^2: 16 k 0.061 (0.062).
+    // * 16 x 8 up to 1,280 tiles, five resident workgroups on each unit.  FP64,
+    //   64^2: 66 k cells 16 x 8 0.078, 32 x 16 0.095; 33^2: 90 k 0.113, 0.135.  Mixed,
+    //   64^2: 66 k 16 x 8 0.064, 32 x 8 0.068; 72^2: 140 k 0.081, 0.087.
+    // * FP64 blocks 16 to 31 cells wide beyond that: 16 x 16 while all its tiles
+    //   are resident, three on each unit (41,088 bytes of LDS), else 16 x 8.  16^2: 660
+    //   tiles of 16 x 16 0.134 (16 x 8 0.147), 768 0.139 (0.155), 850 0.182 (0.160),
+    //   1,024 0.200 (0.179); 24 x 32: 768 0.124 (0.136), 784 0.165 (0.140); 17^2: 864
+    //   0.179 (0.128).
+    // * Blocks at least 32 cells wide beyond that: the ring-pass tiles, which
+    //   recompute fewer ring cells.  FP64 32 x 16 (64^2: 262 k cells 0.140, 16 x 8
+    //   0.163; 2.2 M 0.885, 0.961).  Mixed 32 x 16 up to 1.5 M cells (64^2: 262 k 0.094,
+    //   32 x 8 0.100), then 32 x 8 (2.2 M 0.506, 32 x 16 0.510).
+    // * 8 x 8 for blocks narrower than 16 cells; in FP64, 4 x 4 (one wavefront per
+    //   block) for blocks narrower than 8 cells.
     const bool fp64 = c->s.flux_precision == CFFC_FLUX_FP64;
-    int ti = 16, tj = 8;
     int mini = 1 << 30;
-    int64_t n168 = 0;
-    for (auto &m : c->meta_h) {
-        mini = std::min(mini, m.ni);
-        n168 += (int64_t)((m.ni + 15) / 16) * ((m.nj + 7) / 8);
+    for (auto &m : c->meta_h) mini = std::min(mini, m.ni);
+    auto count = [&](int a, int b) {
+        int64_t n = 0;
+        for (auto &m : c->meta_h) n += (int64_t)((m.ni + a - 1) / a) * ((m.nj + b - 1) / b);
+        return n;
+    };
+    const int64_t units = 256, n16x8 = count(16, 8);
+    int ti = 16, tj = 8;
+    if (mini >= 32 && n16x8 > 5 * units) {
+        ti = 32;
+        tj = fp64 || c->ncell < 1500000 ? 16 : 8;
+    } else if (fp64 && n16x8 > 5 * units && count(16, 16) <= 3 * units) {
+        tj = 16;
     }
-    if (mini >= 32 && n168 > 1280) { ti = 32; tj = fp64 || c->ncell < 1500000 ? 16 : 8; }
-    else if (fp64 && n168 > 1280 && n168 <= 1700) tj = 16;
-    if (mini < 16 || n168 < 256) ti = tj = 8;
+    if (mini < 16 || (fp64 ? count(8, 8) <= units : n16x8 < units)) ti = tj = 8;
     if (mini < 8 && fp64) ti = tj = 4;
     if ((e = build_tiles(c, ti, tj))) {
         free_ctx(c);
