@@ -1040,8 +1040,14 @@ extern "C" int cffc_create(const cffc_mesh_desc *md, const cffc_scheme_desc *sd,
     //   0.179 (0.128).
     // * Blocks at least 32 cells wide beyond that: the ring-pass tiles, which
     //   recompute fewer ring cells.  FP64 32 x 16 (64^2: 262 k cells 0.140, 16 x 8
-    //   0.163; 2.2 M 0.885, 0.961).  Mixed 32 x 16 up to 1.5 M cells (64^2: 262 k 0.094,
-    //   32 x 8 0.100), then 32 x 8 (2.2 M 0.506, 32 x 16 0.510).
+    //   0.163; 2.2 M 0.885, 0.961).  Mixed 32 x 8 (2.2 M 0.506, 32 x 16 0.510), or
+    //   32 x 16 where it divides the blocks as well as 32 x 8 does, up to 1.5 M cells
+    //   (64^2: 213 k 0.093 against 0.098, 783 k 0.198 / 0.205; 96^2: 1.3 M 0.279 /
+    //   0.285), or where all its tiles are resident, three on each unit, and the
+    //   fullest unit's work is less, a tile costing a little under two of 32 x 8
+    //   (72^2: 765 tiles 0.104 / 0.118, 795 0.134 / 0.119; 100^2: 756 0.102 / 0.115,
+    //   784 0.130 / 0.115; 64 x 36: 558 0.100 / 0.094, 696 0.104 / 0.110; 33^2: 1,998
+    //   0.239 / 0.214).
     // * 8 x 8 for blocks narrower than 16 cells; in FP64, 4 x 4 (one wavefront per
     //   block) for blocks narrower than 8 cells.
     const bool fp64 = c->s.flux_precision == CFFC_FLUX_FP64;
@@ -1055,8 +1061,12 @@ extern "C" int cffc_create(const cffc_mesh_desc *md, const cffc_scheme_desc *sd,
     const int64_t units = 256, n16x8 = count(16, 8);
     int ti = 16, tj = 8;
     if (mini >= 32 && n16x8 > 5 * units) {
+        const int64_t tall = count(32, 16), flat = count(32, 8);
+        auto fullest = [&](int64_t n) { return (n + units - 1) / units; };
+        const bool mixed_tall = tall <= 3 * units ? 2 * fullest(tall) - 1 <= fullest(flat)
+                                                  : 2 * tall == flat && c->ncell < 1500000;
         ti = 32;
-        tj = fp64 || c->ncell < 1500000 ? 16 : 8;
+        tj = fp64 || mixed_tall ? 16 : 8;
     } else if (fp64 && n16x8 > 5 * units && count(16, 16) <= 3 * units) {
         tj = 16;
     }

@@ -24,6 +24,13 @@ pytestmark = pytest.mark.gpu
     (True, (51, 5), 16, 8, (8, 8)),       # 255 of 16 x 8
     (True, (16, 16), 16, 8, (16, 8)),
     (True, (16, 4), 64, 64, (32, 16)),    # 512 of 32 x 16
+    (True, (96, 1), 64, 64, (32, 16)),    # 768
+    (True, (20, 5), 64, 64, (32, 16)),    # 800, half as many as of 32 x 8
+    (True, (51, 1), 72, 72, (32, 16)),    # 765
+    (True, (53, 1), 72, 72, (32, 8)),     # 795, more than half
+    (True, (31, 3), 64, 36, (32, 8)),     # 558: three a unit, of 32 x 8 four
+    (True, (29, 4), 64, 36, (32, 16)),    # 696: three a unit, of 32 x 8 five
+    (True, (37, 9), 33, 33, (32, 8)),
 ])
 def test_default_tile(mixed, blocks, ni, nj, tile):
     m = M.cartesian(blocks[0], blocks[1], ni, nj)
