@@ -2896,6 +2896,7 @@ extern "C" int cffc_mg_set_parts(cffc_mg *mg, int npart, const int32_t *first_bl
     if (!mg) return fail(CFFC_E_ARG, "null argument");
     cffc_ctx *f = mg->lv[0];
     mg->setting_gen++;
+    mg->npart = 0;   // also after a call that fails from here on
     for (cffc_ctx *c : mg->lv) {
         c->mg_part_of_block = nullptr;
         c->mg_part_frozen = nullptr;
@@ -2906,10 +2907,7 @@ extern "C" int cffc_mg_set_parts(cffc_mg *mg, int npart, const int32_t *first_bl
         }
         if (any) HIPCHK(hipMemcpy(c->meta, c->meta_h.data(), c->nblk * sizeof(BlockMeta), hipMemcpyHostToDevice));
     }
-    if (npart == 0) {
-        mg->npart = 0;
-        return 0;
-    }
+    if (npart == 0) return 0;
     if (npart < 0 || npart > f->nblk || !first_block || !tol) return fail(CFFC_E_ARG, "bad argument");
     if (first_block[0] != 0 || first_block[npart] != f->nblk) return fail(CFFC_E_ARG, "parts must cover all blocks");
     std::vector<int32_t> pob(f->nblk);
@@ -2944,7 +2942,6 @@ extern "C" int cffc_mg_set_parts(cffc_mg *mg, int npart, const int32_t *first_bl
         c->mg_part_of_block = mg->d_part_of_block;
         c->mg_part_frozen = mg->d_part_frozen;
     }
-    mg->npart = npart;
     mg->part_block0.assign(first_block, first_block + npart + 1);
     mg->part_tol.assign(tol, tol + npart);
     mg->part_freeze.assign(npart, 0.0);
@@ -2952,6 +2949,7 @@ extern "C" int cffc_mg_set_parts(cffc_mg *mg, int npart, const int32_t *first_bl
     mg->part_l2.assign(npart, -1.0);
     mg->part_done.assign(npart, -1);
     mg->cycles = 0;
+    mg->npart = npart;
     return 0;
 }
 
