@@ -358,8 +358,6 @@ static void host_quarter_centroid(const cffc_mesh_desc *md, const BlockMeta &m, 
 }
 #pragma clang fp contract(on)
 
-static int floor_half(int k) { return k >= 0 ? k / 2 : -((1 - k) / 2); }
-
 // Levels, second face neighbours and the same-level table of the push /
 // pull exchange; for a mesh with resolution changes, the restriction,
 // prolongation and flux-correction lists, the per-block AMR flags and the
@@ -2247,7 +2245,6 @@ struct cffc_mg {
     std::vector<FirstLevel> first;
     cffc_mg_desc d{};
     std::vector<double *> P, uo;     // per level (P unused on level 0)
-    std::vector<double> Ahost;       // scratch: fine-level areas for the Wo restriction
     double rs_eps = 0.0;
     int rs_iters = 0;
     bool frozen = false;
@@ -2718,9 +2715,8 @@ static int mg_cgc(cffc_mg *mg, int top, int l) {
     cffc_ctx *c = mg->lv[l];
     const int base = l == top ? mg->base : 0;
     int e;
-    if (l == L - 1) {
-        if (l != top && (e = mg_store_uo(mg, l))) return e;
-        if (l == top && (e = mg_exchange(c))) return e;
+    if (l == L - 1) {   // never the top level: there are two levels or more
+        if ((e = mg_store_uo(mg, l))) return e;
         if ((e = mg_smooth(mg, top, l, d.smooths_on_coarsest_level))) return e;
     } else {
         cffc_ctx *cc = mg->lv[l + 1];

@@ -35,10 +35,6 @@
 
 namespace cffc {
 
-template <typename ST> __device__ __forceinline__ PS<double> amr_ldW(const ST *W, int64_t ncp, int64_t c) {
-    PS<double> r = {(double)W[c], (double)W[ncp + c], (double)W[2 * ncp + c], (double)W[3 * ncp + c]};
-    return r;
-}
 template <typename ST> __device__ __forceinline__ void amr_stW(ST *W, int64_t ncp, int64_t c, const PS<double> &r) {
     W[c] = (ST)r.d; W[ncp + c] = (ST)r.vx; W[2 * ncp + c] = (ST)r.vy; W[3 * ncp + c] = (ST)r.p;
 }

@@ -181,11 +181,6 @@ __device__ __forceinline__ PS<FT> face_state(const PS<FT> &W, const PS<FT> &px, 
 // to the block origin, which halves the geometry traffic.
 template <typename FT> struct CoordT { typedef double type; };
 template <> struct CoordT<float> { typedef float type; };
-template <typename FT>
-__device__ __forceinline__ typename CoordT<FT>::type rdgeo(const StageParams &p, int gd, int gf, int64_t i) {
-    if constexpr (Fast<FT>::on) return p.geomf[gf * p.ncp + i];
-    else return p.geom[gd * p.ncp + i];
-}
 
 // Element access by a 32-bit byte offset from a base that is the same for the
 // whole workgroup (plane + row j0 of the block, the tile's first window row):

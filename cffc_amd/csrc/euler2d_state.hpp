@@ -264,12 +264,6 @@ template <typename T> CFFC_HD T harten_delta(T la, T ll, T lr) {
         return add2k(-tabs(la), K::HALF, qdivf(sqr(la), delta) + delta);
     }
 }
-template <typename T> CFFC_HD T harten_pos(T la, T ll, T lr) {
-    return Consts<T>::HALF * (la + tabs(la) + harten_delta(la, ll, lr));
-}
-template <typename T> CFFC_HD T harten_neg(T la, T ll, T lr) {
-    return Consts<T>::HALF * (la - tabs(la) - harten_delta(la, ll, lr));
-}
 
 // RoeAverage, Euler2DState.cc:654-683
 template <typename T> CFFC_HD PS<T> roe_average(const PS<T> &Wl, const PS<T> &Wr) {
