@@ -86,18 +86,22 @@ template <> struct Fast<float> { static constexpr bool on = true; };
 // a - b q and the corrected quotient q + (a - b q) r.  The remainder is below
 // two units of q's last place, so r's own last-place error enters at 2^-104 of
 // q: the result is a / b correctly rounded, as the compiler's sequence (two
-// Newton steps, one instruction more) gives it.  v_div_fixup_f64 gives zeros,
-// infinities and NaNs their IEEE results (rdiv); rdivf leaves it out, for
-// finite operands and a nonzero finite divisor, where it only restores the sign
-// of a -0 dividend's quotient.  The operand scaling of the compiler's
-// division (v_div_scale_f64 and the scale applied by v_div_fmas_f64) is left
-// out of both: it acts when a/b or 1/b would be subnormal, |a/b| >= 2^767 or a
-// nonzero |a| < 2^-969, so for every other operand pair the result is a / b bit
-// for bit.  The refinement depends on b alone, which is what makes the
-// reciprocal shareable; recip_near starts it from a value already close to
-// 1/b (a reciprocal of a related divisor), without the quarter-rate v_rcp_f64.
-// float: plain division (callers choose their own approximations on the mixed
-// path).
+// Newton steps, one instruction more) gives it.  Neither sequence decides the
+// quotients of a power of two by a divisor whose mantissa is all ones: they lie
+// 2^-107 above the middle of two doubles, and either of those may come out.
+// v_div_fixup_f64 gives zeros, infinities and NaNs their IEEE results (rdiv);
+// rdivf leaves it out, for finite operands and a nonzero finite divisor, where
+// it only restores the sign of a -0 dividend's quotient.  An infinite divisor
+// gives NaN there instead of 0: it takes a state or an intermediate square that
+// has overflowed, whose cell or face ends non-finite either way.  The operand
+// scaling of the compiler's division (v_div_scale_f64 and the scale applied by
+// v_div_fmas_f64) is left out of both: it acts when a/b or 1/b would be
+// subnormal, |a/b| >= 2^767 or a nonzero |a| < 2^-969, so for every other
+// operand pair the result is a / b bit for bit.  The refinement depends on b
+// alone, which is what makes the reciprocal shareable; recip_near starts it
+// from a value already close to 1/b (a reciprocal of a related divisor),
+// without the quarter-rate v_rcp_f64.  float: plain division (callers choose
+// their own approximations on the mixed path).
 template <typename T> struct Recip { T b, r; };
 template <typename T> CFFC_HD Recip<T> recip(T b) {
 #if defined(__HIP_DEVICE_COMPILE__)
