@@ -2225,12 +2225,16 @@ extern "C" int cffc_kernel_times(cffc_ctx *c, double out[4]) {
 // ---- FAS multigrid (FASMultigrid2D/FASMultigrid2D.h) -------------------------
 // One context per level on one stream, level 0 the finest; level l+1 halves
 // level l block by block.  The cycle is the reference's Coarse_Grid_Correction
-// from a top level (0, or a coarser one during the full-multigrid start-up),
-// every smoothing stage through the granular FP64 stage kernel (HLLE and the
-// zero limiter below the top level when first_order_coarse is set), the
-// forcing term folded into that kernel after the face fluxes, and the level
-// transfers of euler2d_mg.hip.  Per-cell dt on every level (Smooth's CFL call
-// does not apply the global minimum).
+// from a top level (0, or a coarser one during the full-multigrid start-up).
+// A smoothing stage is one launch where the level allows it: SK_STEP
+// (mg_one_launch), or on first-order levels (HLLE and the zero limiter below
+// the top level when first_order_coarse is set) mg_first_step_kernel over the
+// level's cell list, or one launch for all smoothings of a level whose groups
+// of blocks are small (mg_listed).  Elsewhere it is an exchange, the granular
+// FP64 stage kernel and an update.  The forcing term is added after the face
+// fluxes; the level transfers are in euler2d_mg.hip.  Per-cell dt on every
+// level (Smooth's CFL call does not apply the global minimum).
+//
 // cell lists of a first-order level (FirstArgs), null where it has none
 struct FirstLevel {
     MgCell *cells = nullptr;

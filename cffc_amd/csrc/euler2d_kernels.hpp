@@ -188,7 +188,7 @@ hipError_t cffc_launch_mg_restrict_wo(const cffc::BlockMeta *mf, const cffc::Blo
                                       const double *Af, const double *wf, double *wc, hipStream_t st);
 hipError_t cffc_launch_mg_first_step(const cffc::FirstArgs *a, double omega, int first_stage, const cffc::FineLevel *fl,
                                      hipStream_t st);
-// nt threads, at least a group's cells and half its faces
+// nt threads, at least a group's cells; its faces are looped over
 hipError_t cffc_launch_mg_first_smooth(const cffc::FirstArgs *a, const cffc::GroupArgs *ga, int ngroup, int nt, int nsm,
                                        const cffc::FineLevel *fl, hipStream_t st);
 hipError_t cffc_launch_mg_prolong(const cffc::BlockMeta *mc, const cffc::BlockMeta *mf, int nblk, int max_int_c,

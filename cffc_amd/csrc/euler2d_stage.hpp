@@ -735,7 +735,9 @@ template <int TI, int TJ, bool SPLIT> struct StageThreads {
 
 // Resident wavefronts per SIMD asked of the compiler: the mixed ring-pass
 // tiles fit six in 80 VGPRs without spilling (0.5% faster at 32 x 8 than the
-// five that 82 VGPRs allow); the FP64 kernels are left to the compiler.
+// five that 82 VGPRs allow).  The FP64 kernels are held to four, 128 VGPRs: they
+// take 71 to 112 and none spills; left alone the compiler takes up to 114, which
+// is four waves too.
 template <typename FT, int TI, int TJ> struct StageWaves {
     static constexpr int value = Fast<FT>::on ? (TileThreads<TI, TJ>::ring_pass ? 6 : 1) : 4;
 };

@@ -1,8 +1,10 @@
 // unet_kernels.hip -- BF16 MFMA kernels of the warm-start U-Net (gfx950).
 //
 // The network has no counterpart in the reference: it predicts an initial
-// state for the steady bump solves.  Activations are NHWC; weights and
-// activations are BF16, accumulation and gradients FP32.
+// state for the steady bump solves.  Activations are NHWC.  BF16: the operands
+// of every product, that is weights, activations and the masked gradients of
+// convolution outputs.  FP32: accumulation, weight and bias gradients, the
+// gradient that a skip connection brings, master weights and moments.
 //
 // 3x3 "same" convolutions are implicit GEMMs on v_mfma_f32_16x16x32_bf16:
 //   forward      Y[p,co]  = act( sum_k X[p+off(k), ci(k)] * Wt[co][k] + b[co] )
