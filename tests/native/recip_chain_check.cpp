@@ -2,10 +2,10 @@
 // side) on the host: v_rcp_f64 and v_rsq_f64 are stood in for by the correctly
 // rounded value moved by up to 2^29 units of the last place, the accuracy their
 // documentation states, at random and at its ends.  Every result has to equal the
-// host's IEEE operation, from whatever value the hardware starts.  One kind of
-// quotient is left out: a power of two over a divisor whose mantissa is all ones lies
-// 2^-107 above the middle of two doubles, which no sequence of this form sees (the
-// compiler's two Newton steps neither); it comes out as one of the two.
+// host's IEEE operation, from whatever value the hardware starts.  For recip one kind of
+// quotient depends on that value and is left to a test on the device: a power of two
+// over a divisor whose mantissa is all ones lies 2^-107 above the middle of two
+// doubles.
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
@@ -37,16 +37,40 @@ static double fixup(double q, double b, double a) {
 #define __builtin_amdgcn_rsqf(x) (1.0f / std::sqrt(x))
 #define __builtin_amdgcn_sqrtf(x) std::sqrt(x)
 #define __builtin_amdgcn_div_fixup fixup
+#define __builtin_amdgcn_ballot_w64(x) ((x) ? 1 : 0)
+static int __double2loint(double x) {
+    uint64_t u;
+    memcpy(&u, &x, 8);
+    return (int)(uint32_t)u;
+}
+static int __double2hiint(double x) {
+    uint64_t u;
+    memcpy(&u, &x, 8);
+    return (int)(uint32_t)(u >> 32);
+}
+static double __hiloint2double(int hi, int lo) {
+    const uint64_t u = ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
+    double x;
+    memcpy(&x, &u, 8);
+    return x;
+}
 #define __builtin_amdgcn_class(x, m) ((x) == 0 || ((x) > 0 && std::isinf(x)))
 #include "../../cffc_amd/csrc/euler2d_state.hpp"
 using namespace cffc;
 
+// random, or near the ends where quotients lie next to the middle of two doubles, or
+// with a low word of ones
 static double mantissa() {
-    const uint64_t r = rng();
-    if ((r & 15) == 0) return 1.0;
-    if ((r & 15) == 1) return std::nextafter(2.0, 0.0);
-    if ((r & 15) == 2) return std::nextafter(1.0, 2.0);
-    return 1.0 + (double)(r >> 12) * 0x1p-52;
+    const uint64_t r = rng(), k = (r >> 8) % 64;
+    uint64_t f = r >> 12;
+    switch (r & 15) {
+    case 0: f = 0; break;
+    case 1: f = ~(uint64_t)0 >> 12; break;
+    case 2: f = k; break;
+    case 3: f = (~(uint64_t)0 >> 12) - k; break;
+    case 4: f |= 0xFFFFFFFFu; break;
+    }
+    return 1.0 + (double)f * 0x1p-52;
 }
 static double value(int e) { return std::ldexp(mantissa(), (int)(rng() % (2 * e + 1)) - e); }
 
@@ -60,10 +84,8 @@ static uint64_t fraction(double x) {
     memcpy(&u, &x, 8);
     return u & (((uint64_t)1 << 52) - 1);
 }
-static void quotient(const char *what, double got, double a, double b) {
-    if (fraction(a) == 0 && fraction(b) == ((uint64_t)1 << 52) - 1) return;
-    same(what, got, a / b, a, b);
-}
+static bool from_estimate(double a, double b) { return fraction(a) == 0 && fraction(b) == ((uint64_t)1 << 52) - 1; }
+static void quotient(const char *what, double got, double a, double b) { same(what, got, a / b, a, b); }
 
 int main(int argc, char **argv) {
     const long n = argc > 1 ? atol(argv[1]) : 1000000;
@@ -72,15 +94,21 @@ int main(int argc, char **argv) {
         const double s = rng() & 1 ? -1.0 : 1.0;
         {   // any pair
             const double a = s * value(300), b = value(300) * (rng() & 1 ? -1.0 : 1.0);
-            quotient("rdivf(a, recip(b))", rdivf(a, recip(b)), a, b);
-            quotient("rdiv(a, recip(b))", rdiv(a, recip(b)), a, b);
-            quotient("qdivf(a, b)", qdivf(a, b), a, b);
+            if (!from_estimate(a, b)) {
+                quotient("rdivf(a, recip(b))", rdivf(a, recip(b)), a, b);
+                quotient("rdiv(a, recip(b))", rdiv(a, recip(b)), a, b);
+                quotient("qdivf(a, b)", qdivf(a, b), a, b);
+            }
         }
         {   // gamma p / ((gamma - 1) d) from 1/d
             const double d = value(60), x = value(60), b = gm1<double>() * d;
             quotient("recip_near(gm1 d)", rdivf(x, recip_near(b, recip(d).r * g1i)), x, b);
             const Recip<double> rgam = {gam<double>(), 1.0 / 1.40};
             quotient("division by gamma", rdivf(x, rgam), x, 1.40);
+        }
+        {   // any divisor from a value a few units to 2^-41 away
+            const double b = s * value(60), x = value(60), d = std::ldexp(1.0, -41 - (int)(rng() % 14));
+            quotient("recip_near(b)", rdivf(x, recip_near(b, 1.0 / b * (1.0 + (rng() & 1 ? d : -d)))), x, b);
         }
         {   // a2 -> c, and 1/c, 1/c^2, 1/a2 one from the other
             const double a2 = value(60), x = s * value(60);
