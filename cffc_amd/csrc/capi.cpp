@@ -1212,11 +1212,22 @@ static int read_words(cffc_ctx *c, const void *src, int n, void *out) {
 // staging copies with one thread (17.7 GB/s): a few threads each move chunks
 // through pinned buffers of their own (a run of 100 steps at 4.2 M cells whose
 // 134 MB come back: 178 -> 170 ms, mixed 110 -> 102 ms).  Below 16 MB the copy is
-// too short for the buffers and threads to pay.
+// too short for the buffers and threads to pay.  Memory that the runtime knows
+// (pinned, managed or a device's) takes the plain copy, which reaches the link's
+// rate there (134 MB pinned: 2.5 ms, through the chunks 4.2) and needs no host
+// access.
+static bool pageable(const void *host) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, host) != hipSuccess) {
+        (void)hipGetLastError();   // not the runtime's
+        return true;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+}
 static int copy_to_host(cffc_ctx *c, void *host, const void *dev, size_t bytes) {
     constexpr size_t MIN = 16 << 20;
     constexpr int NBUF = PIN_THREADS * PIN_BUFS;
-    bool piped = bytes >= MIN;
+    bool piped = bytes >= MIN && pageable(host);
     if (piped && !c->pin) {
         piped = hipHostMalloc((void **)&c->pin, (size_t)NBUF * PIN_CHUNK, hipHostMallocDefault) == hipSuccess;
         if (!piped) c->pin = nullptr;
