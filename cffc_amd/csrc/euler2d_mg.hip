@@ -263,7 +263,9 @@ __global__ __launch_bounds__(64) void mg_restrict_wo_kernel(const BlockMeta *mf,
 // two dependent loads to the states; the price is that both cells of a face
 // evaluate its flux.  The launches of the coarse levels are bound by that load
 // chain (a 12,288-cell case: 9.6 us a stage with windows, whatever the level, 6.7 us
-// so).
+// so).  Without the gradient that the limiter would multiply by zero (0 * NaN is
+// NaN) a state that is no longer finite spreads through faces alone, a cell a
+// stage, not through the stencils of both cells of a face.
 struct FirstCell {
     PS<double> W;
     double A, lW, lE, lS, lN, nWx, nWy, nEx, nEy, nSx, nSy, nNx, nNy;
