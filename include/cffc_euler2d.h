@@ -463,15 +463,16 @@ int  cffc_mg_execute(cffc_mg *mg, int max_cycles, double freeze_level, double *n
    level, so it keeps the state it converged in: every part ends in the
    state it reaches alone.  cffc_mg_initialize starts the parts afresh
    (none converged, frozen or skipped; the tolerances are kept).  npart = 0
-   clears the parts. */
+   clears the parts, and so does a call that is refused. */
 int  cffc_mg_set_parts(cffc_mg *mg, int npart, const int32_t *first_block, const double *tol, const double *freeze);
 /* per part: the last checked L2 norm (l2, may be NULL) and the regular
    cycles done since cffc_mg_set_parts when its norm first met its
    tolerance (done_cycles, -1: not yet; may be NULL); returns npart */
 int  cffc_mg_part_status(cffc_mg *mg, double *l2, int32_t *done_cycles);
 /* cffc_mg_execute replays one captured cycle as a HIP graph (on by
-   default; recaptured once when the limiters freeze); off: the launches
-   are issued one by one, with the same arithmetic.  No reference
+   default; recaptured when the limiters freeze or a setting of the solver
+   or of a level has changed); off: the launches are issued one by one, with
+   the same arithmetic.  No reference
    counterpart: launch overhead. */
 int  cffc_mg_set_graph(cffc_mg *mg, int on);
 /* the forcing term P of a coarse level, interior cells in block order */
