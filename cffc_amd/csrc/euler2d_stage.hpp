@@ -259,7 +259,8 @@ inline int stage_kind(const StageParams &p, int fused) {
 // place of this block's own ghost cells; the thread that loaded a window cell
 // replaces it.  The stage reads one W buffer and writes the other, so
 // neighbours that have already been updated in this launch are not seen; and W
-// is the previous stage's W(U), the value that the exchange kernel would copy.
+// is the previous stage's W(U), the value that the exchange kernel would copy (a
+// cell whose update stayed unphysical keeps its W; the run ends with its key).
 template <int LJ, int LI>
 __device__ __forceinline__ void pull_ghosts(const StageParams &p, const BlockMeta &m, int b, int pi0, int pj0, int tid,
                                             int nt, double (&sW)[4][LJ][LI]) {
